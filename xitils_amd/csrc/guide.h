@@ -64,6 +64,8 @@ __global__ void k_guide_grad(GuideNet net, GuideBounds gb, const GuideSample* sa
                              float weight_clip, float* partial);
 __global__ void k_guide_adam(float* P, float* m, float* v, const float* partial, uint32_t nparts, float lr, float b1,
                              float b2, float eps, float b1t, float b2t, float grad_scale, GuideNet net);
+__global__ void k_guide_pack(const float* queries, const float* dirs, const float* weights, uint32_t n, GuideSample* out);
+__global__ void k_guide_sum_rows(const float* partial, uint32_t rows, float* grad);
 __global__ void k_guide_finalize(const TrainRec* recs, uint32_t n, const float4* radiance, uint32_t target, GuideSample* out,
                                  uint32_t* count, float* weight_sum);
 
@@ -76,6 +78,8 @@ constexpr int GG_BLOCK = XT_GUIDE_GRAD_BLOCK;   // threads per block of k_guide_
                                                 // 256 (32 per wave, 1 wave per SIMD) 27.0 us
 constexpr int GG_BLOCK_SAMPLES = 128;   // a 32768-sample minibatch is one block per CU, each writing one partial row
 constexpr int GF_BLOCK = 1024;  // threads per block of k_guide_finalize
+constexpr int GP_BLOCK = 256;   // threads per block of k_guide_pack
+constexpr int GR_BLOCK = 64;    // threads per block of k_guide_sum_rows (276 waves, one per CU and some)
 constexpr int GA_BLOCK = 1024;  // threads per block of k_guide_adam (32 row groups x 32 parameters)
 
 }  // namespace xt

@@ -783,6 +783,36 @@ __device__ __forceinline__ int row_of_output(int o) {       // o < G_OUT
     return 16 * (s >> 2) + 4 * g + (s & 3);
 }
 
+// Host samples as uploaded (queries n x 9, dirs n x 3, weights n) -> the
+// 64-byte records the gradient kernel reads.  Packing them on the host cost
+// 1.1 ms for 32,768 samples; here it is a few microseconds after a copy of 52
+// bytes a sample.
+__global__ __launch_bounds__(GP_BLOCK) void k_guide_pack(const float* __restrict__ queries, const float* __restrict__ dirs,
+                                                         const float* __restrict__ weights, uint32_t n,
+                                                         GuideSample* __restrict__ out) {
+    const uint32_t i = blockIdx.x * GP_BLOCK + threadIdx.x;
+    if (i >= n) return;
+    const float *q = queries + 9 * (size_t)i, *d = dirs + 3 * (size_t)i;
+    float4* o = (float4*)(out + i);
+    o[0] = make_float4(q[0], q[1], q[2], q[3]);
+    o[1] = make_float4(q[4], q[5], q[6], q[7]);
+    o[2] = make_float4(q[8], d[0], d[1], d[2]);
+    o[3] = make_float4(weights[i], 0.0f, 0.0f, 0.0f);
+}
+
+// grad = the sum of the partial rows, in row order.  A thread per parameter
+// keeps 32 row loads in flight; 256 rows (18 MB) stay on the device, where
+// copying them to the host and summing there took 2 ms.
+__global__ __launch_bounds__(GR_BLOCK) void k_guide_sum_rows(const float* __restrict__ partial, uint32_t rows,
+                                                             float* __restrict__ grad) {
+    const uint32_t i = blockIdx.x * GR_BLOCK + threadIdx.x;
+    if (i >= (uint32_t)G_NPARAMS) return;
+    float acc = 0.0f;
+#pragma unroll 32
+    for (uint32_t b = 0; b < rows; ++b) acc += partial[(size_t)b * G_NPARAMS + i];
+    grad[i] = acc;
+}
+
 // Adam (Kingma & Ba) on the fp32 master parameters: the gradient is the sum
 // of nparts partial rows (GA_GROUPS interleaved row groups per parameter,
 // then the groups in order: deterministic) times grad_scale; b1t, b2t =

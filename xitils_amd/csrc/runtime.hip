@@ -74,7 +74,7 @@ struct GuideState {
     float* P = nullptr;              // fp32 master parameters
     float* m = nullptr;              // Adam moments
     float* v = nullptr;
-    float* partial = nullptr;        // per-block gradient rows of k_guide_grad
+    float* partial = nullptr;        // per-block gradient rows of k_guide_grad, and a last row for their sum
     uint32_t partial_rows = 0;
     void* net_mem = nullptr;         // GuideChain + GuideBack + the two published GuideChains
     GuideNet net{};                  // the copy training reads and Adam writes
@@ -1118,7 +1118,8 @@ static xt_status guide_ensure_training(xt_scene* s) {
     return XT_OK;
 }
 
-// Host samples -> device GuideSample array (grows a scratch buffer).
+// Host samples -> device GuideSample array (grows a scratch buffer), on
+// s->stream: the caller synchronises it before the host arrays may change.
 static xt_status guide_upload_samples(xt_scene* s, const float* queries, const float* dirs, const float* weights,
                                       uint32_t n, GuideSample** out) {
     GuideState& g = s->guide;
@@ -1133,14 +1134,23 @@ static xt_status guide_upload_samples(xt_scene* s, const float* queries, const f
         XT_HIP(dalloc(&g.samples[0], g.rec_cap));
         XT_HIP(dalloc(&g.samples[1], g.rec_cap));
     }
-    std::vector<GuideSample> hs(n);
-    for (uint32_t i = 0; i < n; ++i) {
-        for (int k = 0; k < 9; ++k) hs[i].q[k] = queries[9 * (size_t)i + k];
-        for (int k = 0; k < 3; ++k) hs[i].dir[k] = dirs[3 * (size_t)i + k];
-        hs[i].weight = weights[i];
+    // the arrays as they are into the second sample buffer (idle: the callers
+    // waited for the training bursts), packed on the device
+    float* raw = (float*)g.samples[1];
+    hipError_t e = hipMemcpyAsync(raw, queries, (size_t)n * 9 * 4, hipMemcpyHostToDevice, s->stream);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(raw + 9 * (size_t)n, dirs, (size_t)n * 3 * 4, hipMemcpyHostToDevice, s->stream);
+    if (e == hipSuccess)
+        e = hipMemcpyAsync(raw + 12 * (size_t)n, weights, (size_t)n * 4, hipMemcpyHostToDevice, s->stream);
+    if (e == hipSuccess) {
+        hipLaunchKernelGGL(k_guide_pack, dim3((n + GP_BLOCK - 1) / GP_BLOCK), dim3(GP_BLOCK), 0, s->stream, raw,
+                           raw + 9 * (size_t)n, raw + 12 * (size_t)n, n, g.samples[0]);
+        e = hipGetLastError();
     }
-    XT_HIP(hipMemcpyAsync(g.samples[0], hs.data(), n * sizeof(GuideSample), hipMemcpyHostToDevice, s->stream));
-    XT_HIP(hipStreamSynchronize(s->stream));
+    if (e != hipSuccess) {
+        hipStreamSynchronize(s->stream);   // no copy still reads the caller's arrays
+        return fail(XT_ERR_DEVICE, std::string("guide sample upload failed: ") + hipGetErrorString(e));
+    }
     *out = g.samples[0];
     return XT_OK;
 }
@@ -2324,7 +2334,7 @@ xt_status xt_guide_init(xt_scene* s, const xt_guide_config* cfg) {
     chk(dalloc(&g.P, G_NPARAMS));
     chk(dalloc(&g.m, G_NPARAMS));
     chk(dalloc(&g.v, G_NPARAMS));
-    chk(dalloc(&g.partial, (size_t)g.partial_rows * G_NPARAMS));
+    chk(dalloc(&g.partial, ((size_t)g.partial_rows + 1) * G_NPARAMS));
     chk(dalloc(&g.d_count, 1));
     chk(dalloc(&g.d_wsum, 1));
     chk(hipHostMalloc((void**)&g.host_io, 2 * sizeof(float), hipHostMallocDefault));
@@ -2430,15 +2440,19 @@ xt_status xt_guide_gradient(xt_scene* s, const float* queries, const float* dirs
     GuideState& g = s->guide;
     uint32_t grid = 0;
     st = guide_gradient_rows(s, s->stream, ds, n, weight_scale, weight_clip, &grid);
-    if (st != XT_OK) return st;
-    std::vector<float> rows((size_t)grid * G_NPARAMS);
-    XT_HIP(hipMemcpyAsync(rows.data(), g.partial, rows.size() * 4, hipMemcpyDeviceToHost, s->stream));
-    XT_HIP(hipStreamSynchronize(s->stream));
-    for (int i = 0; i < G_NPARAMS; ++i) {
-        float acc = 0.0f;
-        for (uint32_t b = 0; b < grid; ++b) acc += rows[(size_t)b * G_NPARAMS + i];
-        grad[i] = acc;
+    float* const sum = g.partial + (size_t)g.partial_rows * G_NPARAMS;
+    hipError_t e = hipSuccess;
+    if (st == XT_OK) {
+        hipLaunchKernelGGL(k_guide_sum_rows, dim3((G_NPARAMS + GR_BLOCK - 1) / GR_BLOCK), dim3(GR_BLOCK), 0, s->stream,
+                           g.partial, grid, sum);
+        e = hipGetLastError();
     }
+    if (st == XT_OK && e == hipSuccess)
+        e = hipMemcpyAsync(grad, sum, G_NPARAMS * sizeof(float), hipMemcpyDeviceToHost, s->stream);
+    const hipError_t se = hipStreamSynchronize(s->stream);
+    if (st != XT_OK) return st;
+    if (e == hipSuccess) e = se;
+    if (e != hipSuccess) return fail(XT_ERR_DEVICE, std::string("xt_guide_gradient: ") + hipGetErrorString(e));
     return XT_OK;
 }
 
@@ -2457,11 +2471,11 @@ xt_status xt_guide_train_step(xt_scene* s, const float* queries, const float* di
     s->guide.cfg.minibatch = std::max(saved, n);   // one step over all n samples
     st = guide_train(s, s->stream, ds, n, (float)(n / wsum), 1, nullptr);
     s->guide.cfg.minibatch = saved;
-    if (st != XT_OK) return st;
-    st = guide_publish_all(s);
-    if (st != XT_OK) return st;
-    XT_HIP(hipStreamSynchronize(s->stream));
-    return XT_OK;
+    if (st == XT_OK) st = guide_publish_all(s);
+    const hipError_t se = hipStreamSynchronize(s->stream);   // also lets go of the caller's arrays
+    if (st == XT_OK && se != hipSuccess)
+        st = fail(XT_ERR_DEVICE, std::string("xt_guide_train_step: ") + hipGetErrorString(se));
+    return st;
 }
 
 }  // extern "C"
