@@ -154,7 +154,7 @@ enum {
     XT_FLAG_ENV_NEE = 2u,        /* sample sun + sky as a light, MIS with BSDF escapes */
     XT_FLAG_GUIDE = 4u,          /* standard integrator: sample with the scene's guiding network */
     XT_FLAG_GUIDE_TRAIN = 8u,    /* with XT_FLAG_GUIDE: record training samples, take Adam steps per batch */
-    XT_FLAG_SORT_MATERIALS = 16u /* shade each block's queue entries grouped by material type (same film) */
+    XT_FLAG_SORT_MATERIALS = 16u /* shade each block's queue entries grouped by material type (same film; small renders keep no queues) */
 };
 
 typedef struct xt_render_params {
@@ -173,7 +173,9 @@ typedef struct xt_render_params {
 } xt_render_params;
 
 /* Counters of the last xt_render, xt_trace_closest or xt_trace_any on a
- * scene.  After a ray query only its fields are set: extension_rays (closest)
+ * scene.  A launch that follows paths to their ends (small renders, the last
+ * rounds of large ones; not while fetches are counted) counts as one extend
+ * launch and its time as ms_extend.  After a ray query only its fields are set: extension_rays (closest)
  * or shadow_rays (any) = n, ms_extend or ms_shadow = ms_total = the traversal
  * kernel's time, and with counting on its node and triangle fetches. */
 typedef struct xt_render_stats {

@@ -192,6 +192,47 @@ __global__ void k_shade_multi(MultiBatch mb, PathQueue qin, const uint32_t* coun
                               float4* radiance, float4* pending);
 __global__ void k_accumulate_multi(MultiBatch mb, const float4* radiance);
 
+// Arguments of k_walk.  MULTI uses mb, the others wp and scene; QUEUE (paths
+// taken up in mid-flight) uses q, count and pending, the others number the
+// paths of the batch or window themselves.
+struct WalkArgs {
+    WaveParams wp;
+    const DevScene* scene;
+    MultiBatch mb;
+    PathQueue q;
+    const uint32_t* count;
+    const float4* pending;
+    float4* radiance;
+    uint32_t lanes;                 // rays a wave keeps in flight (1..64)
+    uint32_t* ovf;                  // traversal spill columns
+    uint32_t* dyn;                  // chunk cursor and block counter, zero between launches
+    unsigned long long* rays;       // null, or running totals of extension and shadow rays
+    unsigned long long* rays_out;   // where the launch leaves them (mapped host memory)
+};
+// waves per SIMD of k_walk (at 3 instead of 4, with no spill instead of 28
+// registers', it measured the same; the normal-mapping form needs 256 VGPRs)
+constexpr int WALK_WAVES = 4, WALK_WAVES_NMAP = 2;
+// Paths from which a batch is queued instead of walked.  A walked path costs
+// the longest of its wave's rays at every vertex, a queued one its share of
+// three launches per round: below some half a million paths the launches, their
+// gaps and the slowest ray of each cost more.  Walked against queued, us, 100 k
+// triangle room (depth 16): 1111 / 3354 at 14 k paths, 2605 / 4055 at 230 k,
+// 4694 / 4898 at 460 k, 7452 / 6205 at 921 k; Cornell box (depth 8): 353 / 890,
+// 689 / 1003, 1168 / 1231, 1802 / 1612; 0.5 M triangle field 453 / 997,
+// 862 / 1618, 1200 / 1771, 1782 / 2137; normal-mapped plane 333 / 922,
+// 785 / 1339, 1152 / 1651, 2081 / 2313.
+constexpr uint32_t WALK_MAX = 11u << 16;
+// Paths of a queue that are walked to their ends instead of queued on: the
+// last rounds of a large batch (Cornell box 1 M paths: 1671 us without, 1641
+// at 256 Ki, 1820 at 1 Mi).
+constexpr uint32_t WALK_TAIL = 1u << 18;
+// Waves that few paths are spread over, by leaving lanes empty: a wave's step
+// takes as long as the slowest of its rays, so 6 k paths ran in 735 us at 64
+// paths a wave and in 545 / 427 / 413 / 406 us over 512 / 1024 / 2048 / 4096 waves.
+constexpr uint32_t WALK_SPREAD = 2048;
+template <bool QUEUE, bool NMAP, bool MULTI>
+__global__ void k_walk(WalkArgs a);
+
 __global__ void k_generate(WaveParams wp, PathQueue q, float4* radiance);
 template <bool GUIDE, bool NMAP, bool SORT>
 __global__ void k_shade(WaveParams wp, const DevScene* scene, PathQueue qin, const uint32_t* count_in, const float4* hits,
@@ -205,7 +246,7 @@ __global__ void k_accumulate(WaveParams wp, const float4* radiance, void* film, 
 __global__ void k_zero_u32(uint32_t* p, uint32_t n);
 constexpr int VALU_PROBE_CHAINS = 16;   // FMA chains per lane of k_valu_probe
 __global__ void k_valu_probe(uint32_t iters, float* out);
-__global__ void k_cursor_init(BatchCursor* c, BatchPlan plan);
+__global__ void k_cursor_init(BatchCursor* c, BatchPlan plan, uint32_t* dyn);
 __global__ void k_advance_cursor(BatchCursor* c, BatchPlan plan);
 __global__ void k_count_from_cursor(uint32_t* count, const BatchCursor* c);
 

@@ -200,28 +200,34 @@ XT_INST_TRACE(true, true, false, true)
 
 // ---------------------------------------------------------------- wavefront PT
 
-// Camera ray of a path (PinholeCamera::generateRay, Camera.h:45-55) at the
-// jittered film position of RenderTargetTile::GenerateFilmPosition
+// Camera ray of a pixel's sample (PinholeCamera::generateRay, Camera.h:45-55)
+// at the jittered film position of RenderTargetTile::GenerateFilmPosition
 // (RenderTarget.h:68-80).
+__device__ __forceinline__ void camera_ray(const WaveParams& wp, uint32_t pixel, uint32_t sample, f3* o, f3* d) {
+    const uint32_t x = pixel % wp.width, y = pixel / wp.width;
+    Rng rng{make_uint2(wp.seed, wp.stream), pixel, sample};
+    uint4 b0 = rng.block(0, 0);
+    float ux = Rng::to_unit(b0.x), uy = Rng::to_unit(b0.y);
+    float fx = (float)x, fy = (float)y;
+    fx /= (float)wp.width;
+    fy /= (float)wp.height;
+    fy = 1.0f - fy;
+    fx += (ux - 0.5f) / (float)wp.width;
+    fy += (uy - 0.5f) / (float)wp.height;
+    f3 dc = normalize(mk(wp.tan_x * (fx - 0.5f) * 2, wp.tan_y * (fy - 0.5f) * 2, 1));
+    *o = xf_point(wp.cam, mk(0, 0, 0));
+    *d = xf_vector(wp.cam, dc);
+}
+
+// Camera rays of a batch's paths.
 __global__ __launch_bounds__(256) void k_generate(WaveParams wp, PathQueue q, float4* __restrict__ radiance) {
     const BatchCursor bc = batch_of(wp);
     const uint32_t P = bc.num_paths;
     for (uint32_t id = blockIdx.x * blockDim.x + threadIdx.x; id < P; id += gridDim.x * blockDim.x) {
         uint32_t s_local = id / bc.num_pixels;
         uint32_t pixel = bc.first_pixel + (id - s_local * bc.num_pixels);
-        uint32_t x = pixel % wp.width, y = pixel / wp.width;
-        Rng rng{make_uint2(wp.seed, wp.stream), pixel, bc.sample0 + s_local};
-        uint4 b0 = rng.block(0, 0);
-        float ux = Rng::to_unit(b0.x), uy = Rng::to_unit(b0.y);
-        float fx = (float)x, fy = (float)y;
-        fx /= (float)wp.width;
-        fy /= (float)wp.height;
-        fy = 1.0f - fy;
-        fx += (ux - 0.5f) / (float)wp.width;
-        fy += (uy - 0.5f) / (float)wp.height;
-        f3 dc = normalize(mk(wp.tan_x * (fx - 0.5f) * 2, wp.tan_y * (fy - 0.5f) * 2, 1));
-        f3 o = xf_point(wp.cam, mk(0, 0, 0));
-        f3 d = xf_vector(wp.cam, dc);
+        f3 o, d;
+        camera_ray(wp, pixel, bc.sample0 + s_local, &o, &d);
         // e (the sampling record) and the radiance slot of a camera ray are
         // implied by its vertex index 1: the shade step reads neither
         q.o[id] = make_float4(o.x, o.y, o.z, 0.0f);
@@ -327,11 +333,22 @@ __device__ __forceinline__ ShadeConst shade_const(const WaveParams& wp, const De
     return c;
 }
 
-template <bool GUIDE, bool NMAP, class PathMap>
-__device__ __forceinline__ void shade_entry(const WaveParams& wp, const DevScene& sc, const ShadeConst& sc0,
-                                            const PathQueue& qin, const float4* __restrict__ hits,
-                                            float4* __restrict__ radiance, float4* __restrict__ pending,
-                                            const GuideRender& gr, uint32_t i, const PathMap& pmap, ShadeOut& out) {
+// A path's arrival at a vertex: the ray that reached it (direction, BSDF
+// sample) and the path's state.
+struct VertexIn {
+    f3 d, weight, meval;
+    float pdf_prev, pe_prev;
+    uint32_t v, qflags, id;
+    float4 h;          // hit record of the ray
+    f3 rad, pend;      // radiance so far; light sample of the previous vertex (QF_PENDING)
+};
+
+// One loop step of the path at `in`; i: its guide lobes' entry.  put_rad(rad)
+// takes the path's radiance up to here.
+template <bool GUIDE, bool NMAP, class PathMap, class PutRad>
+__device__ __forceinline__ void shade_vertex(const WaveParams& wp, const DevScene& sc, const ShadeConst& sc0,
+                                             const VertexIn& in, const GuideRender& gr, uint32_t i, const PathMap& pmap,
+                                             PutRad put_rad, ShadeOut& out) {
     const bool standard = sc0.standard;
     const bool can_sample = sc0.can_sample;
     const EnvNee envn = sc0.envn;
@@ -353,24 +370,12 @@ __device__ __forceinline__ void shade_entry(const WaveParams& wp, const DevScene
     f3& sh_d = out.sh_d;
     f3& sh_c = out.sh_c;
     float& sh_tmax = out.sh_tmax;
-    uint32_t& id = out.id;
-        const float4 o4 = qin.o[i], d4 = qin.d[i], w4 = qin.w[i], h = hits[i];
-        id = __float_as_uint(d4.w);
-        const uint32_t vf = __float_as_uint(w4.w);
-        const uint32_t v = vf & 0xFFFFFFu, qflags = vf >> 24;
-        // a camera ray (vertex 1) has no sampling record and no radiance yet:
-        // the generate step writes neither
-        const float4 e4 = v > 1 ? qin.e[i] : make_float4(1.0f, 1.0f, 1.0f, 0.0f);
-        const float pdf_prev = o4.w, pe_prev = e4.w;
-        const f3 d = xyz(d4), meval = xyz(e4);
-        f3 weight = xyz(w4);
-        f3 rad = v > 1 ? xyz(radiance[id]) : splat(0.0f);
-        const f3 pend = (qflags & QF_PENDING) ? xyz(pending[id]) : splat(0.0f);
-        if (GUIDE && gr.recs) {
-            // the vertex that sampled this ray: radiance up to and including its light sample
-            const uint32_t rin = qin.rec[i];
-            if (rin != INVALID) gr.recs[rin].f = f4(rad + pend, 0.0f);
-        }
+    const uint32_t id = out.id = in.id;
+        const uint32_t v = in.v, qflags = in.qflags;
+        const float4 h = in.h;
+        const float pdf_prev = in.pdf_prev, pe_prev = in.pe_prev;
+        const f3 d = in.d, meval = in.meval, pend = in.pend;
+        f3 weight = in.weight, rad = in.rad;
         const uint32_t slot = __float_as_uint(h.y);
         const bool hit = slot != INVALID;
         xt_material mat;
@@ -423,7 +428,7 @@ __device__ __forceinline__ void shade_entry(const WaveParams& wp, const DevScene
             }
         }
         if (qflags & QF_PENDING) rad += pend;  // light sample of the previous vertex
-        radiance[id] = f4(rad, 0.0f);
+        put_rad(rad);
 
         bool live = hit && !emissive;
         Rng rng{key, 0u, 0u};
@@ -607,6 +612,38 @@ __device__ __forceinline__ void shade_entry(const WaveParams& wp, const DevScene
                 ext_v = v + 1;
             }
         }
+}
+
+// shade_vertex of queue entry i.
+template <bool GUIDE, bool NMAP, class PathMap>
+__device__ __forceinline__ void shade_entry(const WaveParams& wp, const DevScene& sc, const ShadeConst& sc0,
+                                            const PathQueue& qin, const float4* __restrict__ hits,
+                                            float4* __restrict__ radiance, float4* __restrict__ pending,
+                                            const GuideRender& gr, uint32_t i, const PathMap& pmap, ShadeOut& out) {
+    const float4 o4 = qin.o[i], d4 = qin.d[i], w4 = qin.w[i];
+    VertexIn in;
+    in.h = hits[i];
+    in.id = __float_as_uint(d4.w);
+    const uint32_t vf = __float_as_uint(w4.w);
+    in.v = vf & 0xFFFFFFu;
+    in.qflags = vf >> 24;
+    // a camera ray (vertex 1) has no sampling record and no radiance yet:
+    // the generate step writes neither
+    const float4 e4 = in.v > 1 ? qin.e[i] : make_float4(1.0f, 1.0f, 1.0f, 0.0f);
+    in.pdf_prev = o4.w;
+    in.pe_prev = e4.w;
+    in.d = xyz(d4);
+    in.meval = xyz(e4);
+    in.weight = xyz(w4);
+    in.rad = in.v > 1 ? xyz(radiance[in.id]) : splat(0.0f);
+    in.pend = (in.qflags & QF_PENDING) ? xyz(pending[in.id]) : splat(0.0f);
+    if (GUIDE && gr.recs) {
+        // the vertex that sampled this ray: radiance up to and including its light sample
+        const uint32_t rin = qin.rec[i];
+        if (rin != INVALID) gr.recs[rin].f = f4(in.rad + in.pend, 0.0f);
+    }
+    const uint32_t id = in.id;
+    shade_vertex<GUIDE, NMAP>(wp, sc, sc0, in, gr, i, pmap, [&](f3 rad) { radiance[id] = f4(rad, 0.0f); }, out);
 }
 
 // Compacted appends of a block's shaded entries (every thread of the block
@@ -813,9 +850,12 @@ __device__ __forceinline__ BatchCursor cursor_at(const BatchPlan& pl, uint32_t p
     return c;
 }
 
-// First batch of a render whose first sample is plan.spp_offset.
-__global__ void k_cursor_init(BatchCursor* c, BatchPlan plan) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) *c = cursor_at(plan, 0, 0, plan.spp_offset);
+// First batch of a render whose first sample is plan.spp_offset; clears a
+// chunk cursor that nothing else has (dyn, or null).
+__global__ void k_cursor_init(BatchCursor* c, BatchPlan plan, uint32_t* dyn) {
+    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+    *c = cursor_at(plan, 0, 0, plan.spp_offset);
+    if (dyn) dyn[0] = dyn[1] = 0u;
 }
 
 // Next batch: the next pixel chunk, or the first chunk of the next S samples.
@@ -915,19 +955,8 @@ __global__ __launch_bounds__(256) void k_generate_multi(MultiBatch mb, PathQueue
         const uint32_t s_local = (uint32_t)(local / it.npix);
         const uint32_t pixel = (uint32_t)(local - (uint64_t)s_local * it.npix);
         const WaveParams& wp = it.wp;
-        const uint32_t x = pixel % wp.width, y = pixel / wp.width;
-        Rng rng{make_uint2(wp.seed, wp.stream), pixel, it.spp_offset + s_local};
-        uint4 b0 = rng.block(0, 0);
-        float ux = Rng::to_unit(b0.x), uy = Rng::to_unit(b0.y);
-        float fx = (float)x, fy = (float)y;
-        fx /= (float)wp.width;
-        fy /= (float)wp.height;
-        fy = 1.0f - fy;
-        fx += (ux - 0.5f) / (float)wp.width;
-        fy += (uy - 0.5f) / (float)wp.height;
-        f3 dc = normalize(mk(wp.tan_x * (fx - 0.5f) * 2, wp.tan_y * (fy - 0.5f) * 2, 1));
-        f3 o = xf_point(wp.cam, mk(0, 0, 0));
-        f3 d = xf_vector(wp.cam, dc);
+        f3 o, d;
+        camera_ray(wp, pixel, it.spp_offset + s_local, &o, &d);
         q.o[id] = make_float4(o.x, o.y, o.z, 0.0f);   // e and radiance: implied by vertex 1, as above
         q.d[id] = make_float4(d.x, d.y, d.z, __uint_as_float(id));
         q.w[id] = make_float4(1.0f, 1.0f, 1.0f, __uint_as_float(1u));
@@ -1091,5 +1120,224 @@ __global__ __launch_bounds__(256) void k_accumulate_multi(MultiBatch mb, const f
         }
     }
 }
+
+// ---------------------------------------------------------------- whole paths in one launch
+
+// Paths followed from their camera ray (or from where the queue left them) to
+// their end in one launch: a lane keeps its path's state in registers and
+// loops over shadow ray, extension ray and shade step; lanes whose path has
+// ended take the next path of the wave's chunk.  The same functions in the
+// same order per path as the queued kernels, so the same radiance.
+//
+// Between vertices the wave traces every lane's two rays to their ends (a
+// lane goes on to its extension ray as soon as WALK_SWITCH lanes, or all that
+// are left, have their shadow ray done), then shades together.
+#ifndef XT_WALK_SWITCH
+#define XT_WALK_SWITCH 8
+#endif
+template <bool QUEUE, bool NMAP, bool MULTI>
+__global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) void k_walk(WalkArgs a) {
+    __shared__ uint32_t lds[TRACE_LDS_DEPTH * TRACE_BLOCK];
+    __shared__ float4 top[TOP_F4];
+    __shared__ uint32_t counted[2];
+    const WaveParams& wp0 = a.wp;
+    const MultiBatch& mb = a.mb;
+    if (threadIdx.x < 2) counted[threadIdx.x] = 0u;
+    if constexpr (!MULTI) stage_top_nodes(top, *a.scene);
+    __syncthreads();
+    const uint32_t n = QUEUE ? *a.count : MULTI ? mb.cursor->n : batch_of(wp0).num_paths;
+    const size_t nthreads = (size_t)gridDim.x * blockDim.x;
+    const size_t gtid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t* my_lds = lds + threadIdx.x;
+    uint32_t* my_ovf = a.ovf ? a.ovf + gtid : nullptr;
+    const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)(gtid / 64);
+    const uint32_t lanes = a.lanes, lane = __lane_id();
+    const uint64_t below = (1ull << lane) - 1ull;
+    RayChunks ch = chunks_first<true>(wave, nwaves, n, lanes);
+    const GuideRender gr{};
+    const CursorMap cmap{wp0};
+    ShadeConst c0;
+    if constexpr (!MULTI) c0 = shade_const(wp0, *a.scene);
+    // the lane's path: its next extension ray, the sample that made it, the
+    // radiance so far and the light sample its shadow ray decides on
+    bool alive = false, has_ext = false, has_pend = false;
+    uint32_t id = 0, v = 0, item = 0, n_ext = 0, n_sh = 0;
+    f3 eo = splat(0.0f), ed = eo, weight = eo, meval = eo, rad = eo, c = eo;
+    float pdf = 0.0f, pe = 0.0f;
+    enum { IDLE, SHADOW, EXTEND, SWITCH };   // SWITCH: shadow ray done, extension ray next
+    int mode = IDLE;
+    RayPre r;
+    Trav t;
+    TravView view{nullptr, nullptr, 0u};
+    while (true) {
+        const uint64_t busy = __ballot(alive);
+        const uint32_t nidle = lanes - (uint32_t)__popcll(busy);
+        const bool refill = busy == 0 || nidle * 4 >= lanes;
+        if (refill && ch.next >= ch.end && !ch.exhausted) chunks_refill(ch, a.dyn);
+        if (refill && ch.next < ch.end) {
+            const uint32_t my = ch.next + (uint32_t)__popcll(~busy & below);
+            if (!alive && lane < lanes && my < ch.end) {
+                if constexpr (QUEUE) {
+                    const float4 o4 = a.q.o[my], d4 = a.q.d[my], w4 = a.q.w[my];
+                    id = __float_as_uint(d4.w);
+                    const uint32_t vf = __float_as_uint(w4.w);
+                    v = vf & 0xFFFFFFu;
+                    has_pend = ((vf >> 24) & QF_PENDING) != 0;
+                    const float4 e4 = v > 1 ? a.q.e[my] : make_float4(1.0f, 1.0f, 1.0f, 0.0f);
+                    pdf = o4.w;
+                    pe = e4.w;
+                    meval = xyz(e4);
+                    weight = xyz(w4);
+                    rad = v > 1 ? xyz(a.radiance[id]) : splat(0.0f);
+                    c = has_pend ? xyz(a.pending[id]) : splat(0.0f);
+                    eo = xyz(o4);
+                    ed = xyz(d4);
+                    if constexpr (MULTI) item = mb.item_of[id];
+                } else {
+                    id = my;
+                    if constexpr (MULTI) {
+                        const MultiCursor mc = *mb.cursor;
+                        item = window_item(mb, mc, id);
+                        const MultiItem& it = mb.items[item];
+                        const uint2 ps = ItemMap{it, mc.g0}(id);
+                        camera_ray(it.wp, ps.x, ps.y, &eo, &ed);
+                    } else {
+                        const uint2 ps = cmap(id);
+                        camera_ray(wp0, ps.x, ps.y, &eo, &ed);
+                    }
+                    v = 1;
+                    pdf = pe = 0.0f;
+                    weight = meval = splat(1.0f);
+                    rad = splat(0.0f);
+                    has_pend = false;
+                }
+                if constexpr (MULTI) {
+                    view.nodes = mb.items[item].nodes;
+                    view.tris = mb.items[item].tris;
+                }
+                alive = true;
+                mode = SWITCH;
+            }
+            ch.next = min(ch.next + nidle, ch.end);
+        }
+        if (__ballot(alive) == 0) break;
+        // the rays of this vertex
+        while (true) {
+            const uint64_t tracing = __ballot(mode == SHADOW || mode == EXTEND);
+            const uint64_t waiting = __ballot(mode == SWITCH);
+            if ((tracing | waiting) == 0) break;
+            if (tracing == 0 || __popcll(waiting) >= XT_WALK_SWITCH) {
+                if (mode == SWITCH) {
+                    r = ray_setup(eo, ed);
+                    trav_init(t, INFINITY);   // extension rays: tMax = Infinity (PathTracer.h:167)
+                    mode = EXTEND;
+                    ++n_ext;
+                }
+            }
+            const bool active = mode == SHADOW || mode == EXTEND;
+            bool occ = false, done;
+            if constexpr (MULTI)
+                done = trav_step_mixed<TRACE_LDS_DEPTH>(active, mode == SHADOW, view, r, t, top, my_lds, TRACE_BLOCK, my_ovf,
+                                                        nthreads, &occ);
+            else
+                done = trav_step_mixed<TRACE_LDS_DEPTH>(active, mode == SHADOW, *a.scene, r, t, top, my_lds, TRACE_BLOCK,
+                                                        my_ovf, nthreads, &occ);
+            if (active && done) {
+                if (mode == EXTEND) {
+                    mode = IDLE;
+                } else {
+                    if (occ) c = splat(0.0f);
+                    mode = has_ext ? SWITCH : IDLE;
+                    if (!has_ext) {
+                        if (!occ) rad += c;
+                        a.radiance[id] = f4(rad, 0.0f);
+                        alive = false;
+                    }
+                }
+            }
+        }
+        if (alive) {
+            VertexIn in;
+            in.d = ed;
+            in.weight = weight;
+            in.meval = meval;
+            in.pdf_prev = pdf;
+            in.pe_prev = pe;
+            in.v = v;
+            in.qflags = has_pend ? QF_PENDING : 0u;
+            in.id = id;
+            in.h = t.best_slot != INVALID
+                       ? make_float4(t.best_t, __uint_as_float(t.best_slot), t.b0, t.b1)
+                       : make_float4(INFINITY, __uint_as_float(INVALID), 0.0f, 0.0f);
+            in.rad = rad;
+            in.pend = c;
+            ShadeOut o;
+            auto put = [&](f3 x) { rad = x; };
+            if constexpr (MULTI) {
+                const MultiItem& it = mb.items[item];
+                const DevScene& sc = mb.scenes[it.scene];
+                shade_vertex<false, NMAP>(it.wp, sc, shade_const(it.wp, sc), in, gr, 0, ItemMap{it, mb.cursor->g0}, put, o);
+            } else {
+                shade_vertex<false, NMAP>(wp0, *a.scene, c0, in, gr, 0, cmap, put, o);
+            }
+            has_ext = o.push_ext;
+            has_pend = o.push_ext && o.push_sh;
+            eo = o.ext_o;
+            ed = o.ext_d;
+            weight = o.ext_w;
+            meval = o.ext_e;
+            pdf = o.ext_pdf;
+            pe = o.ext_pe;
+            v = o.ext_v;
+            c = o.sh_c;
+            if (o.push_sh) {
+                r = ray_setup(o.sh_o, o.sh_d);
+                trav_init(t, o.sh_tmax);
+                mode = SHADOW;
+                ++n_sh;
+            } else if (o.push_ext) {
+                mode = SWITCH;
+            } else {
+                a.radiance[id] = f4(rad, 0.0f);
+                alive = false;
+            }
+        }
+    }
+    if (a.rays) {
+        for (int off = 32; off > 0; off >>= 1) {
+            n_ext += __shfl_xor(n_ext, off);
+            n_sh += __shfl_xor(n_sh, off);
+        }
+        if (lane == 0) {
+            atomicAdd(&counted[0], n_ext);
+            atomicAdd(&counted[1], n_sh);
+        }
+    }
+    // as chunks_release; the last block to leave also hands out the ray totals
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (a.rays) {
+            atomicAdd(&a.rays[0], (unsigned long long)counted[0]);
+            atomicAdd(&a.rays[1], (unsigned long long)counted[1]);
+        }
+        __threadfence();
+        if (atomicAdd(&a.dyn[1], 1u) == gridDim.x - 1) {
+            atomicExch(&a.dyn[0], 0u);
+            atomicExch(&a.dyn[1], 0u);
+            if (a.rays) {
+                a.rays_out[0] = atomicAdd(&a.rays[0], 0ull);
+                a.rays_out[1] = atomicAdd(&a.rays[1], 0ull);
+            }
+        }
+    }
+}
+template __global__ void k_walk<false, false, false>(WalkArgs);
+template __global__ void k_walk<true, false, false>(WalkArgs);
+template __global__ void k_walk<false, true, false>(WalkArgs);
+template __global__ void k_walk<true, true, false>(WalkArgs);
+template __global__ void k_walk<false, false, true>(WalkArgs);
+template __global__ void k_walk<true, false, true>(WalkArgs);
+template __global__ void k_walk<false, true, true>(WalkArgs);
+template __global__ void k_walk<true, true, true>(WalkArgs);
 
 }  // namespace xt

@@ -51,12 +51,17 @@ struct RenderBuffers {
     hipEvent_t round_ev[RB_RING] = {};
     unsigned long long* visits = nullptr;  // node, tri fetches: extension [0..1], shadow [2..3]
     uint32_t* dyn = nullptr;               // chunk cursors of the traversal kernels: extension [0..1], shadow [2..3]
+    unsigned long long* rays = nullptr;    // extension and shadow rays traced by k_walk, ever
+    unsigned long long* host_rays = nullptr;      // its last totals (pinned, behind host_counts)
+    unsigned long long* host_rays_dev = nullptr;
+    unsigned long long rays_seen[2] = {0, 0};     // totals already in some render's stats
     void release() {
         for (int k = 0; k < 2; ++k) {
             hipFree(q[k].o); hipFree(q[k].d); hipFree(q[k].w); hipFree(q[k].e);
         }
         hipFree(sq.o); hipFree(sq.d); hipFree(sq.c);
         hipFree(hits); hipFree(radiance); hipFree(pending); hipFree(counts); hipFree(visits); hipFree(dyn);
+        hipFree(rays);
         hipFree(rec[0]); hipFree(rec[1]); hipFree(lobes);
         if (host_counts) hipHostFree(host_counts);
         for (hipEvent_t& e : round_ev)
@@ -731,6 +736,17 @@ static uint32_t trace_blocks(const xt_scene* s, size_t n) {
     return (uint32_t)std::max<size_t>(1, std::min<size_t>(b, s->trace_grid));
 }
 
+// Paths a wave of k_walk follows at a time, of n in all.
+static uint32_t walk_lanes(uint64_t n) {
+    return (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>(1, (n + WALK_SPREAD - 1) / WALK_SPREAD));
+}
+// Its blocks: as many as have paths, no more than are resident at once.
+static uint32_t walk_blocks(const xt_scene* s, uint64_t n, uint32_t lanes, bool nmap, uint32_t most) {
+    const uint32_t per_block = lanes * (TRACE_BLOCK / 64);
+    const uint32_t resident = (uint32_t)s->dev->num_cu * (nmap ? WALK_WAVES_NMAP : WALK_WAVES);
+    return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((n + per_block - 1) / per_block, std::min(resident, most)));
+}
+
 static xt_status query(xt_scene* s, const xt_ray* rays, uint32_t n, void* out, int on_device, bool any) {
     if (!s || (n && (!rays || !out))) return fail(XT_ERR_INVALID_ARGUMENT, "NULL argument");
     if (n == 0) return XT_OK;
@@ -853,9 +869,15 @@ static xt_status alloc_buffers(RenderBuffers& rb, uint32_t capacity) {
     XT_HIP(dalloc(&rb.visits, 4));
     XT_HIP(dalloc(&rb.dyn, 4));
     XT_HIP(hipMemset(rb.dyn, 0, 4 * sizeof(uint32_t)));
-    XT_HIP(hipHostMalloc((void**)&rb.host_counts, RB_RING * 4 * sizeof(uint32_t),
+    XT_HIP(dalloc(&rb.rays, 2));
+    XT_HIP(hipMemset(rb.rays, 0, 2 * sizeof(unsigned long long)));
+    constexpr size_t ring_words = RB_RING * 4;
+    XT_HIP(hipHostMalloc((void**)&rb.host_counts, ring_words * sizeof(uint32_t) + 2 * sizeof(unsigned long long),
                          hipHostMallocMapped | hipHostMallocCoherent));
     XT_HIP(hipHostGetDevicePointer((void**)&rb.host_counts_dev, rb.host_counts, 0));
+    rb.host_rays = (unsigned long long*)(rb.host_counts + ring_words);
+    rb.host_rays_dev = (unsigned long long*)(rb.host_counts_dev + ring_words);
+    rb.host_rays[0] = rb.host_rays[1] = 0;
     for (hipEvent_t& e : rb.round_ev) XT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     rb.capacity = capacity;
     return XT_OK;
@@ -1246,12 +1268,44 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                 net_r = GuideNet{g.pub[rd], g.net.back};
             }
             hipEvent_t a = tm.mark();
-            hipLaunchKernelGGL(k_generate, dim3(blocks256(wp.num_paths)), dim3(256), 0, s->stream, wp, rb.q[0], rb.radiance);
-            XT_LAUNCHED(result);
-            hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, s->stream, rb.counts + 0, wp.num_paths);
-            XT_LAUNCHED(result);
-            tm.add(3, a, tm.mark());
             s->stats.camera_rays += wp.num_paths;
+            // the rest of the batch in one launch: at most n paths, of the
+            // queue `q` or (q < 0) from their camera rays
+            auto walk = [&](int q, uint64_t n) {
+                WalkArgs wa{};
+                wa.wp = wp;
+                wa.scene = s->d_ds;
+                if (q >= 0) {
+                    wa.q = rb.q[q];
+                    wa.count = rb.counts + q;
+                }
+                wa.pending = rb.pending;
+                wa.radiance = rb.radiance;
+                wa.lanes = walk_lanes(n);
+                wa.ovf = s->d_ovf;
+                wa.dyn = rb.dyn;
+                wa.rays = rb.rays;
+                wa.rays_out = rb.host_rays_dev;
+                auto kernel = s->nmap ? (q >= 0 ? k_walk<true, true, false> : k_walk<false, true, false>)
+                                      : (q >= 0 ? k_walk<true, false, false> : k_walk<false, false, false>);
+                hipEvent_t w = tm.mark();
+                hipLaunchKernelGGL(kernel, dim3(walk_blocks(s, n, wa.lanes, s->nmap, s->trace_grid_max)), dim3(TRACE_BLOCK), 0,
+                                   s->stream, wa);
+                XT_LAUNCHED(result);
+                tm.add(0, w, tm.mark());
+                s->stats.extend_launches++;
+            };
+            const bool can_walk = !guide && !s->counting;
+            const bool whole = can_walk && wp.num_paths <= WALK_MAX;
+            if (whole) {
+                walk(-1, wp.num_paths);
+            } else {
+                hipLaunchKernelGGL(k_generate, dim3(blocks256(wp.num_paths)), dim3(256), 0, s->stream, wp, rb.q[0], rb.radiance);
+                XT_LAUNCHED(result);
+                hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, s->stream, rb.counts + 0, wp.num_paths);
+                XT_LAUNCHED(result);
+                tm.add(3, a, tm.mark());
+            }
             // Bounce rounds.  Every kernel reads its queue length from device
             // memory; the host reads each round's counts from a pinned ring
             // `lag` rounds late, so the GPU does not wait for the host between
@@ -1265,7 +1319,7 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
             uint32_t queue_len[RB_RING];           // queue length of each unverified round
             int round = 0, verified = 0, cur = 0;
             uint32_t rec_base = 0;
-            bool launch = true;
+            bool launch = !whole;
             queue_len[0] = wp.num_paths;
             // a path adds one extension ray per round, so max_depth + 1 rounds hold every live queue
             const int max_rounds = p->max_depth > 0 ? p->max_depth + 2 + lag : (1 << 16);
@@ -1338,11 +1392,11 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                     cur = 1 - cur;
                 }
                 // read back every round at least `lag` behind the last launch
-                while (launch && verified <= round - 1 - lag) {
+                auto read_round = [&]() {
                     const int vs = verified % RB_RING;
                     if (hipEventSynchronize(rb.round_ev[vs]) != hipSuccess) {
                         result = fail(XT_ERR_DEVICE, std::string("render failed: ") + hipGetErrorString(hipGetLastError()));
-                        break;
+                        return false;
                     }
                     const uint32_t* hc = rb.host_counts + 4 * vs;
                     const uint32_t len = queue_len[vs];
@@ -1358,6 +1412,17 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                     bound = next;
                     if (next == 0) launch = false;
                     ++verified;
+                    return true;
+                };
+                while (launch && verified <= round - 1 - lag)
+                    if (!read_round()) break;
+                if (launch && can_walk && bound <= WALK_TAIL && result == XT_OK) {
+                    // few paths are left: the queue of the next round, whose
+                    // length is at most `bound`, in one launch
+                    walk(cur, bound);
+                    while (verified < round)
+                        if (!read_round()) break;
+                    launch = false;
                 }
             }
             if (result != XT_OK) break;
@@ -1421,6 +1486,9 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
     if (result == XT_OK) {
         float ms = 0;
         hipEventElapsedTime(&ms, t_begin, t_end);
+        s->stats.extension_rays += rb.host_rays[0] - rb.rays_seen[0];
+        s->stats.shadow_rays += rb.host_rays[1] - rb.rays_seen[1];
+        for (int k = 0; k < 2; ++k) rb.rays_seen[k] = rb.host_rays[k];
         s->stats.ms_total = ms;
         s->stats.ms_extend = tm.total(0);
         s->stats.ms_shade = tm.total(1);
@@ -1484,6 +1552,7 @@ struct BounceBufs {
     float4* pending;
     uint32_t* counts;        // [0], [1]: path queues, [2]: shadow queue
     uint32_t* ovf;           // traversal spill columns for tblocks blocks
+    uint32_t* dyn;           // k_walk's chunk cursor and block counter
     uint32_t capacity;       // paths
 };
 
@@ -1532,8 +1601,8 @@ struct BounceGuide {
 // max_depth + 1 rounds of extend / (guide) / shade / shadow, accumulate,
 // advance the cursor.  Every kernel reads its queue length from device memory.
 static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const WaveParams& wp, const BounceBufs& b,
-                                 const BatchPlan& plan, BatchCursor* cursor, uint32_t tblocks, const BounceGuide& gd,
-                                 void* d_film, int f64) {
+                                 const BatchPlan& plan, BatchCursor* cursor, uint32_t tblocks, uint32_t tmost,
+                                 const BounceGuide& gd, void* d_film, int f64) {
     const uint32_t maxpaths = plan.pix_chunk * plan.S;
     const uint32_t gblocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((maxpaths + 255) / 256, (uint64_t)s->dev->num_cu * 8));
     const uint32_t ablocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((plan.pix_chunk + 255) / 256, (uint64_t)s->dev->num_cu * 8));
@@ -1541,10 +1610,23 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
     const bool guide = gd.lobes_mk != nullptr;
     GuideState& g = s->guide;
     const uint32_t ib = std::max(1u, std::min((maxpaths + GI_BLOCK - 1) / GI_BLOCK, (uint32_t)s->dev->num_cu * 4));
-    hipLaunchKernelGGL(k_generate, dim3(gblocks), dim3(256), 0, s->stream, wp, b.q[0], b.radiance);
-    hipLaunchKernelGGL(k_count_from_cursor, dim3(1), dim3(1), 0, s->stream, b.counts + 0, cursor);
+    const bool whole = !guide && maxpaths <= WALK_MAX;   // each path in one launch
+    if (whole) {
+        WalkArgs wa{};
+        wa.wp = wp;
+        wa.scene = s->d_ds;
+        wa.radiance = b.radiance;
+        wa.lanes = walk_lanes(maxpaths);
+        wa.ovf = b.ovf;
+        wa.dyn = b.dyn;
+        hipLaunchKernelGGL((s->nmap ? k_walk<false, true, false> : k_walk<false, false, false>),
+                           dim3(walk_blocks(s, maxpaths, wa.lanes, s->nmap, tmost)), dim3(TRACE_BLOCK), 0, s->stream, wa);
+    } else {
+        hipLaunchKernelGGL(k_generate, dim3(gblocks), dim3(256), 0, s->stream, wp, b.q[0], b.radiance);
+        hipLaunchKernelGGL(k_count_from_cursor, dim3(1), dim3(1), 0, s->stream, b.counts + 0, cursor);
+    }
     int cur = 0;
-    for (int it = 0; it <= p->max_depth; ++it) {
+    for (int it = 0; it <= p->max_depth && !whole; ++it) {
         hipLaunchKernelGGL((k_trace<false, TRACE_LDS_DEPTH, false>), dim3(tblocks), dim3(TRACE_BLOCK), 0, s->stream, s->ds,
                            b.q[cur].o, b.q[cur].d, 1, b.counts + cur, 0u, b.hits, nullptr, 0, 0, b.ovf, nullptr, nullptr,
                            b.counts + (1 - cur), b.counts + 2);
@@ -1587,7 +1669,7 @@ static xt_status capture_graph(xt_scene* s, const xt_camera* cam, const xt_rende
     uint32_t nbatches = 0;
     const BatchPlan plan = cursor_plan(p, cap, &nbatches);
     const WaveParams wp = cursor_wave_params(cam, p, s->d_cursor);
-    BounceBufs b{{rb.q[0], rb.q[1]}, rb.sq, rb.hits, rb.radiance, rb.pending, rb.counts, s->d_ovf, rb.capacity};
+    BounceBufs b{{rb.q[0], rb.q[1]}, rb.sq, rb.hits, rb.radiance, rb.pending, rb.counts, s->d_ovf, rb.dyn, rb.capacity};
     BounceGuide gd;
     if (guide) {
         gd.lobes_mk = (uint2*)rb.lobes;
@@ -1596,7 +1678,7 @@ static xt_status capture_graph(xt_scene* s, const xt_camera* cam, const xt_rende
     }
     const uint32_t tblocks = trace_blocks(s, plan.pix_chunk * plan.S);
     XT_HIP(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_cursor_batch(s, p, wp, b, plan, s->d_cursor, tblocks, gd, d_film, f64);
+    enqueue_cursor_batch(s, p, wp, b, plan, s->d_cursor, tblocks, s->trace_grid_max, gd, d_film, f64);
     hipError_t launch_err = hipGetLastError();
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(s->stream, &graph);
@@ -1652,7 +1734,7 @@ static xt_status enqueue_graph_render(xt_scene* s, const RenderGraph& g, uint32_
     }
     BatchPlan plan = g.plan;
     plan.spp_offset = spp_offset;
-    hipLaunchKernelGGL(k_cursor_init, dim3(1), dim3(1), 0, s->stream, s->d_cursor, plan);
+    hipLaunchKernelGGL(k_cursor_init, dim3(1), dim3(1), 0, s->stream, s->d_cursor, plan, (uint32_t*)nullptr);
     XT_HIP(hipGetLastError());
     for (uint32_t b = 0; b < g.nbatches; ++b) XT_HIP(hipGraphLaunch(g.exec, s->stream));
     return XT_OK;
@@ -1817,7 +1899,10 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
         m.capacity = window;
     }
     xt_scene* s0 = sc_list[0];
-    const uint32_t tblocks = std::max(1u, std::min(s0->trace_grid, (window + TRACE_BLOCK - 1) / TRACE_BLOCK));
+    const bool whole = window <= WALK_MAX;   // each path in one launch
+    const uint32_t lanes = walk_lanes(window);
+    const uint32_t tblocks = whole ? walk_blocks(s0, window, lanes, nmap, s0->trace_grid_max)
+                                   : std::max(1u, std::min(s0->trace_grid, (window + TRACE_BLOCK - 1) / TRACE_BLOCK));
     const size_t ovf_need = (size_t)ovf_depth * tblocks * TRACE_BLOCK;
     if (m.ovf_entries < ovf_need) {
         hipStreamSynchronize(m.stream);
@@ -1864,10 +1949,21 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
     const bool dyn = window >= TRAV_DYN_MIN;
     XT_HIP(hipStreamBeginCapture(m.stream, hipStreamCaptureModeThreadLocal));
     hipLaunchKernelGGL(k_window_plan, dim3(1), dim3(1), 0, m.stream, mb);
-    hipLaunchKernelGGL(k_count_from_window, dim3(1), dim3(1), 0, m.stream, m.counts, m.cursor);
-    hipLaunchKernelGGL(k_generate_multi, dim3(gblocks), dim3(256), 0, m.stream, mb, m.q[0], m.radiance);
+    if (whole) {
+        WalkArgs wa{};
+        wa.mb = mb;
+        wa.radiance = m.radiance;
+        wa.lanes = lanes;
+        wa.ovf = m.ovf;
+        wa.dyn = m.dyn;
+        hipLaunchKernelGGL((nmap ? k_walk<false, true, true> : k_walk<false, false, true>),
+                           dim3(tblocks), dim3(TRACE_BLOCK), 0, m.stream, wa);
+    } else {
+        hipLaunchKernelGGL(k_count_from_window, dim3(1), dim3(1), 0, m.stream, m.counts, m.cursor);
+        hipLaunchKernelGGL(k_generate_multi, dim3(gblocks), dim3(256), 0, m.stream, mb, m.q[0], m.radiance);
+    }
     int cur = 0;
-    for (int it = 0; it <= max_depth; ++it) {
+    for (int it = 0; it <= max_depth && !whole; ++it) {
         hipLaunchKernelGGL((dyn ? k_trace<false, TRACE_LDS_DEPTH, false, true, true>
                                 : k_trace<false, TRACE_LDS_DEPTH, false, true, false>),
                            dim3(tblocks), dim3(TRACE_BLOCK), 0, m.stream, s0->ds, m.q[cur].o, m.q[cur].d, 1,
@@ -2173,6 +2269,7 @@ xt_status xt_render_static(xt_scene* s, const xt_camera* cam, const xt_render_pa
     BatchCursor* cursor = (BatchCursor*)base;
     BounceBufs b{};
     b.counts = (uint32_t*)(base + 64);
+    b.dyn = (uint32_t*)(base + 128);
     b.ovf = per_block ? (uint32_t*)(base + STATIC_HEADER) : nullptr;
     b.capacity = cap;
     float4* arr = (float4*)(base + STATIC_HEADER + spill_bytes);
@@ -2200,9 +2297,9 @@ xt_status xt_render_static(xt_scene* s, const xt_camera* cam, const xt_render_pa
     const uint32_t tblocks = std::min(trace_blocks(s, (size_t)plan.pix_chunk * plan.S), tcap);
     // the cursor is written by k_cursor_init and the counters by the kernels
     // (k_count_from_cursor, k_trace), so nothing needs clearing beforehand
-    hipLaunchKernelGGL(k_cursor_init, dim3(1), dim3(1), 0, s->stream, cursor, plan);
+    hipLaunchKernelGGL(k_cursor_init, dim3(1), dim3(1), 0, s->stream, cursor, plan, b.dyn);
     for (uint32_t k = 0; k < nbatches; ++k)
-        enqueue_cursor_batch(s, p, wp, b, plan, cursor, tblocks, BounceGuide{}, film, film_f64);
+        enqueue_cursor_batch(s, p, wp, b, plan, cursor, tblocks, tcap, BounceGuide{}, film, film_f64);
     hipError_t le = hipGetLastError();
     hipError_t se = hipStreamSynchronize(s->stream);
     if (le != hipSuccess) return fail(XT_ERR_DEVICE, std::string("xt_render_static launch failed: ") + hipGetErrorString(le));

@@ -241,7 +241,7 @@ struct RayChunks {
     bool exhausted;
 };
 template <bool DYN>
-__device__ __forceinline__ RayChunks chunks_first(uint32_t wave, uint32_t nwaves, uint32_t n) {
+__device__ __forceinline__ RayChunks chunks_first(uint32_t wave, uint32_t nwaves, uint32_t n, uint32_t min_chunk = 64) {
     RayChunks c;
     if constexpr (!DYN) {
         const uint32_t per = (n + nwaves - 1) / nwaves;
@@ -254,7 +254,7 @@ __device__ __forceinline__ RayChunks chunks_first(uint32_t wave, uint32_t nwaves
         return c;
     }
     const uint64_t quarter = ((uint64_t)n + 4ull * nwaves - 1) / (4ull * nwaves);
-    c.chunk = (uint32_t)min<uint64_t>(max<uint64_t>(quarter, 64), TRAV_CHUNK);
+    c.chunk = (uint32_t)min<uint64_t>(max<uint64_t>(quarter, min_chunk), TRAV_CHUNK);
     const uint64_t b = (uint64_t)wave * c.chunk;
     c.next = (uint32_t)min<uint64_t>(b, n);
     c.end = (uint32_t)min<uint64_t>(b + c.chunk, n);
@@ -434,9 +434,9 @@ __device__ __forceinline__ uint32_t prim_of_slot(const SV& sc, uint32_t slot) {
 }
 
 // Tests the first triangle of leaf code `leaf` (< 0); returns the code of the
-// rest of the leaf, or 0 when the leaf is done (or, for ANY, when *occ was set).
-template <bool ANY, bool COUNT, class SV>
-__device__ __forceinline__ int visit_tri(const SV& sc, const RayPre& r, Trav& t, int leaf, VisitCount& vc,
+// rest of the leaf, or 0 when the leaf is done (or, for `any`, when *occ was set).
+template <bool COUNT, class SV>
+__device__ __forceinline__ int visit_tri(const SV& sc, const RayPre& r, Trav& t, int leaf, VisitCount& vc, bool any,
                                          bool* occ) {
     uint32_t code = (uint32_t)(~leaf);
     uint32_t first = code >> 3, cnt = (code & 7u) + 1u;
@@ -445,7 +445,7 @@ __device__ __forceinline__ int visit_tri(const SV& sc, const RayPre& r, Trav& t,
     float4 v0 = tr[0], v1 = tr[1], v2 = tr[2];
     float th, b0, b1;
     if (tri_test(xyz(v0), xyz(v1), xyz(v2), r, t.tmax, &th, &b0, &b1)) {
-        if (ANY) {
+        if (any) {
             *occ = true;
             return 0;
         }
@@ -498,7 +498,7 @@ __device__ __forceinline__ bool trav_step(bool active, const SV& sc, const RayPr
             done = true;
     }
     if (active && !done && t.node < 0) {
-        const int rest = visit_tri<ANY, COUNT>(sc, r, t, t.node, vc, occ);
+        const int rest = visit_tri<COUNT>(sc, r, t, t.node, vc, ANY, occ);
         if (ANY && *occ) return true;
         if (rest) t.node = rest;
         else done = !trav_pop<LDS_DEPTH>(t, lds, lds_stride, ovf, ovf_stride);
@@ -511,7 +511,7 @@ __device__ __forceinline__ bool trav_step(bool active, const SV& sc, const RayPr
     } else {
         // one triangle per step: a divergent wave then pays for one node
         // visit plus one triangle test per iteration, not for a whole leaf
-        const int rest = visit_tri<ANY, COUNT>(sc, r, t, t.node, vc, occ);
+        const int rest = visit_tri<COUNT>(sc, r, t, t.node, vc, ANY, occ);
         if (ANY && *occ) return true;
         if (rest) {
             t.node = rest;
@@ -520,6 +520,29 @@ __device__ __forceinline__ bool trav_step(bool active, const SV& sc, const RayPr
     }
     return !trav_pop<LDS_DEPTH>(t, lds, lds_stride, ovf, ovf_stride);
 #endif
+}
+
+// One step of a lane that traces either kind of ray (`any`: stop at the first
+// triangle hit), visiting children in closest-hit order for both: an any-hit
+// answer does not depend on the order.
+template <int LDS_DEPTH, class SV>
+__device__ __forceinline__ bool trav_step_mixed(bool active, bool any, const SV& sc, const RayPre& r, Trav& t,
+                                                const float4* top, uint32_t* lds, int lds_stride, uint32_t* ovf,
+                                                size_t ovf_stride, bool* occ) {
+    VisitCount vc;
+    bool done = false;
+    if (active && t.node >= 0) {
+        if (!visit_node<false, LDS_DEPTH, false>(sc, r, t, top, lds, lds_stride, ovf, ovf_stride, vc) &&
+            !trav_pop<LDS_DEPTH>(t, lds, lds_stride, ovf, ovf_stride))
+            done = true;
+    }
+    if (active && !done && t.node < 0) {
+        const int rest = visit_tri<false>(sc, r, t, t.node, vc, any, occ);
+        if (*occ) return true;
+        if (rest) t.node = rest;
+        else done = !trav_pop<LDS_DEPTH>(t, lds, lds_stride, ovf, ovf_stride);
+    }
+    return done;
 }
 
 }  // namespace xt
