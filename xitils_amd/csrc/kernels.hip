@@ -98,10 +98,19 @@ __device__ __forceinline__ void flush_counts(unsigned long long* totals, const V
 // MULTI: the rays of a unified batch's queue, each traced in its own item's
 // scene (item_of[path id] -> the item's nodes and triangles, per lane).
 // Bounded to 8 waves per SIMD, which every form but the chunked multi-scene
-// and counting ones reaches without spilling; the chunked multi-scene form
-// takes 7, the chunked counting form (run once per scene) is unbounded.
+// one (7, where 8 spills two registers) reaches without spilling.
+//
+// Bound by VALU issue, and for any hit by L1 accesses too: a node visit is some
+// 180 VALU instructions and 4 loads, and the kernel issued 0.76-0.84 G
+// wave-instructions per ms where independent FMAs reach 0.81-0.88.  Lane state
+// kept as masks and counts in scalar registers (the ray id tells an idle lane),
+// the outward push one fma a plane, child counts from the sort's masks and
+// stack reads that stay LDS reads: 1080p field 62.8 -> 61.3 ms a frame, 100 k
+// triangle room 12.85 -> 12.46, 16 rooms batch 4.07 -> 3.84, bounce-ray query
+// 437 -> 427 us.  (Grid steps held as whole floats in the nodes' spare words:
+// 1% faster frames, but the bounce-ray query 450 us.)
 template <bool ANY, int LDS_DEPTH, bool COUNT, bool MULTI, bool DYN>
-__global__ __launch_bounds__(TRACE_BLOCK, DYN && COUNT ? 1 : DYN && MULTI ? 7 : 8) void k_trace(DevScene sc, const float4* __restrict__ ray_o,
+__global__ __launch_bounds__(TRACE_BLOCK, DYN && MULTI ? 7 : 8) void k_trace(DevScene sc, const float4* __restrict__ ray_o,
                                                         const float4* __restrict__ ray_d, int ray_stride,
                                                         const uint32_t* __restrict__ count_ptr, uint32_t count_fixed,
                                                         float4* __restrict__ hits, uint8_t* __restrict__ occluded,
@@ -125,38 +134,39 @@ __global__ __launch_bounds__(TRACE_BLOCK, DYN && COUNT ? 1 : DYN && MULTI ? 7 : 
     const size_t gtid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t* my_lds = lds + threadIdx.x;
     uint32_t* my_ovf = ovf ? ovf + gtid : nullptr;
-    const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)(gtid / 64);
+    const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(gtid / 64));
     RayChunks ch = chunks_first<DYN>(wave, nwaves, n);
     const uint64_t below = (1ull << __lane_id()) - 1ull;
     VisitCount vc;
-    bool active = false;
-    uint32_t rid = 0;
+    uint32_t rid = INVALID;   // the lane's ray; INVALID: none
     RayPre r;
     Trav t;
     TravView view{sc.nodes, sc.tris, MULTI ? 0u : sc.top_nodes};
     while (true) {
-        const uint64_t busy = __ballot(active);
-        const uint32_t nidle = 64u - (uint32_t)__popcll(busy);
-        const bool refill = nidle >= (uint32_t)REFILL_IDLE || busy == 0;
-        if (DYN && refill && ch.next >= ch.end && !ch.exhausted) chunks_refill(ch, dyn);
-        if (refill && ch.next < ch.end) {
-            const uint32_t my = ch.next + (uint32_t)__popcll(~busy & below);
-            if (!active && my < ch.end) {
-                rid = my;
-                float4 o4 = ray_o[(size_t)rid * ray_stride];
-                float4 d4 = ray_d[(size_t)rid * ray_stride];
-                if constexpr (MULTI) {
-                    const MultiItem& it = items[item_of[__float_as_uint(d4.w)]];
-                    view.nodes = it.nodes;
-                    view.tris = it.tris;
+        const uint64_t busy = wave_ballot(rid != INVALID);
+        const uint32_t nidle = 64u - wave_count(busy);
+        if (nidle >= (uint32_t)REFILL_IDLE) {
+            if (DYN && ch.next >= ch.end && !ch.exhausted) chunks_refill(ch, dyn);
+            if (ch.next < ch.end) {
+                const uint32_t my = ch.next + (uint32_t)__popcll(~busy & below);
+                if (rid == INVALID && my < ch.end) {
+                    rid = my;
+                    float4 o4 = ray_o[(size_t)rid * ray_stride];
+                    float4 d4 = ray_d[(size_t)rid * ray_stride];
+                    if constexpr (MULTI) {
+                        const MultiItem& it = items[item_of[__float_as_uint(d4.w)]];
+                        view.nodes = it.nodes;
+                        view.tris = it.tris;
+                    }
+                    r = ray_setup(xyz(o4), xyz(d4));
+                    trav_init(t, tmax_from_ray ? o4.w : INFINITY);   // extension rays: tMax = Infinity (PathTracer.h:167)
                 }
-                r = ray_setup(xyz(o4), xyz(d4));
-                trav_init(t, tmax_from_ray ? o4.w : INFINITY);   // extension rays: tMax = Infinity (PathTracer.h:167)
-                active = true;
+                ch.next = min(ch.next + nidle, ch.end);
+            } else if (busy == 0) {
+                break;
             }
-            ch.next = min(ch.next + nidle, ch.end);
         }
-        if (__ballot(active) == 0) break;
+        const bool active = rid != INVALID;
         bool occ = false;
         bool done;
         if constexpr (MULTI)
@@ -174,7 +184,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, DYN && COUNT ? 1 : DYN && MULTI ? 7 : 
                                                   t.b0, t.b1)
                                     : make_float4(INFINITY, __uint_as_float(INVALID), 0.0f, 0.0f);
                 }
-                active = false;
+                rid = INVALID;
             }
         }
     }
@@ -255,8 +265,8 @@ __device__ __forceinline__ uint32_t block_sort_by_material(const DevScene& sc, c
         const uint32_t slot = __float_as_uint(hits[i].y);
         key = 0;
         if (slot != INVALID) {
-            const uint32_t m = __float_as_uint(sc.tris[(size_t)slot * TRI_F4 + 1].w);
-            key = 1 + min(sc.mats[m].type, (uint32_t)XT_MAT_COUNT_);
+            const uint32_t m = __float_as_uint(in_global(sc.tris)[(size_t)slot * TRI_F4 + 1].w);
+            key = 1 + min(in_global((const uint32_t*)sc.mats)[(size_t)m * (sizeof(xt_material) / 4)], (uint32_t)XT_MAT_COUNT_);
         }
     }
     const uint32_t wave = threadIdx.x / 64, lane = __lane_id();
@@ -382,7 +392,7 @@ __device__ __forceinline__ void shade_vertex(const WaveParams& wp, const DevScen
         bool emissive = false;
         if (hit) {
             s = make_surf<NMAP>(sc, slot, d, h.z, h.w);
-            mat = sc.mats[s.mat];
+            mat = in_global(sc.mats)[s.mat];
             emissive = mat.type == XT_MAT_EMISSION;
         }
         // ---- radiance arriving along the ray that reached this vertex
@@ -410,7 +420,7 @@ __device__ __forceinline__ void shade_vertex(const WaveParams& wp, const DevScen
             } else if (emissive) {                                                     // PathTracer.h:171-189
                 float mis;
                 if (pdf_prev >= 0.0f && can_sample) {
-                    float pl = sc.light_pdf[slot] * p_area;
+                    float pl = in_global(sc.light_pdf)[slot] * p_area;
                     float cosL = fabsf(dot(d, s.sn));
                     float distSq = h.x * h.x;
                     pl *= distSq / cosL;
@@ -529,8 +539,8 @@ __device__ __forceinline__ void shade_vertex(const WaveParams& wp, const DevScen
                         }
                     }
                 } else if (can_sample) {
-                    uint2 lo = sc.light_objs[blk1.y % sc.num_lights];
-                    uint32_t lslot = sc.light_slots[lo.x + blk1.z % lo.y];
+                    uint2 lo = in_global(sc.light_objs)[blk1.y % sc.num_lights];
+                    uint32_t lslot = in_global(sc.light_slots)[lo.x + blk1.z % lo.y];
                     uint4 blk2 = rng.block(v, 2);
                     float t0, t1;
                     if (uniform_bary) {
@@ -548,19 +558,19 @@ __device__ __forceinline__ void shade_vertex(const WaveParams& wp, const DevScen
                         t0 = a * inv;
                         t1 = b * inv;
                     }
-                    const float4* lt = sc.tris + (size_t)lslot * TRI_F4;
+                    const auto lt = in_global(sc.tris) + (size_t)lslot * TRI_F4;
                     float4 l0 = lt[0], l1 = lt[1], l2 = lt[2];
                     f3 q0 = xyz(l0), q1 = xyz(l1), q2 = xyz(l2);
                     f3 lp = lerp3(q0, q1, q2, t0, t1);
                     f3 ln = normalize(cross(q1 - q0, q2 - q0));
                     f3 lsn = ln;
                     if (__float_as_uint(l2.w) & TRI_FLAG_NORMALS) {
-                        const float4* nr = sc.normals + (size_t)lslot * TRI_F4;
+                        const auto nr = in_global(sc.normals) + (size_t)lslot * TRI_F4;
                         lsn = normalize(lerp3(xyz(nr[0]), xyz(nr[1]), xyz(nr[2]), t0, t1));
                     }
                     ln = normalize(ln);
                     lsn = normalize(lsn);
-                    float pdfL = sc.light_pdf[lslot] * p_area;
+                    float pdfL = in_global(sc.light_pdf)[lslot] * p_area;
                     float dist = length(lp - s.p);
                     f3 sd = div(lp - s.p, dist);
                     if (dot(sd, ln) < 0) {
@@ -578,7 +588,7 @@ __device__ __forceinline__ void shade_vertex(const WaveParams& wp, const DevScen
                         }
                         if (mis > 0.0f) {
                             float G = fabsf(dot(-sd, lsn)) / distSq;
-                            const xt_material& lm = sc.mats[__float_as_uint(l1.w)];
+                            const xt_material lm = in_global(sc.mats)[__float_as_uint(l1.w)];
                             f3 c = div(weight * mis * fc * emitted(lm, -sd, ln) * G, pdfL);
                             push_sh = true;
                             sh_d = sd;
@@ -727,8 +737,7 @@ XT_INST_SHADE(true, true, true)
 
 // Any-hit for queued shadow rays; unoccluded contributions go straight to the
 // path radiance, or to pending[] when the path continues (see k_shade).
-// Bounded to 8 waves per SIMD: every form fits 64 VGPRs without spilling (the
-// chunked ones take 71 unbounded and ran 6% slower at 7 waves).
+// Bounded to 8 waves per SIMD, which every form reaches without spilling.
 template <bool COUNT, bool DYN>
 __global__ __launch_bounds__(TRACE_BLOCK, 8) void k_shadow(DevScene sc, ShadowQueue sq, const uint32_t* __restrict__ count,
                                                         float4* __restrict__ radiance, float4* __restrict__ pending,
@@ -747,31 +756,32 @@ __global__ __launch_bounds__(TRACE_BLOCK, 8) void k_shadow(DevScene sc, ShadowQu
     const size_t gtid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t* my_lds = lds + threadIdx.x;
     uint32_t* my_ovf = ovf ? ovf + gtid : nullptr;
-    const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)(gtid / 64);
+    const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(gtid / 64));
     RayChunks ch = chunks_first<DYN>(wave, nwaves, n);
     const uint64_t below = (1ull << __lane_id()) - 1ull;
     VisitCount vc;
-    bool active = false;
-    uint32_t rid = 0;
+    uint32_t rid = INVALID;   // the lane's ray; INVALID: none
     RayPre r;
     Trav t;
     while (true) {
-        const uint64_t busy = __ballot(active);
-        const uint32_t nidle = 64u - (uint32_t)__popcll(busy);
-        const bool refill = nidle >= (uint32_t)REFILL_IDLE || busy == 0;
-        if (DYN && refill && ch.next >= ch.end && !ch.exhausted) chunks_refill(ch, dyn);
-        if (refill && ch.next < ch.end) {
-            const uint32_t my = ch.next + (uint32_t)__popcll(~busy & below);
-            if (!active && my < ch.end) {
-                rid = my;
-                float4 o4 = sq.o[rid], d4 = sq.d[rid];
-                r = ray_setup(xyz(o4), xyz(d4));
-                trav_init(t, o4.w);
-                active = true;
+        const uint64_t busy = wave_ballot(rid != INVALID);
+        const uint32_t nidle = 64u - wave_count(busy);
+        if (nidle >= (uint32_t)REFILL_IDLE) {
+            if (DYN && ch.next >= ch.end && !ch.exhausted) chunks_refill(ch, dyn);
+            if (ch.next < ch.end) {
+                const uint32_t my = ch.next + (uint32_t)__popcll(~busy & below);
+                if (rid == INVALID && my < ch.end) {
+                    rid = my;
+                    float4 o4 = sq.o[rid], d4 = sq.d[rid];
+                    r = ray_setup(xyz(o4), xyz(d4));
+                    trav_init(t, o4.w);
+                }
+                ch.next = min(ch.next + nidle, ch.end);
+            } else if (busy == 0) {
+                break;
             }
-            ch.next = min(ch.next + nidle, ch.end);
         }
-        if (__ballot(active) == 0) break;
+        const bool active = rid != INVALID;
         bool occ = false;
         const bool done = trav_step<true, TRACE_LDS_DEPTH, COUNT>(active, sc, r, t, top, my_lds, TRACE_BLOCK, my_ovf,
                                                                    nthreads, vc, &occ);
@@ -787,7 +797,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, 8) void k_shadow(DevScene sc, ShadowQu
                 } else if (!occ) {
                     radiance[id] = f4(xyz(radiance[id]) + c, 0.0f);
                 }
-                active = false;
+                rid = INVALID;
             }
         }
     }
@@ -1007,10 +1017,9 @@ template __global__ void k_shade_multi<true>(MultiBatch, PathQueue, const uint32
                                              uint32_t*, ShadowQueue, uint32_t*, float4*, float4*);
 
 // Any-hit for a unified batch's shadow queue, each ray in its item's scene.
-// 8 waves per SIMD for the split form, 7 for the chunked one (65 VGPRs; 8
-// would spill).
+// 8 waves per SIMD, without spilling.
 template <bool DYN>
-__global__ __launch_bounds__(TRACE_BLOCK, DYN ? 7 : 8) void k_shadow_multi(ShadowQueue sq, const uint32_t* __restrict__ count,
+__global__ __launch_bounds__(TRACE_BLOCK, 8) void k_shadow_multi(ShadowQueue sq, const uint32_t* __restrict__ count,
                                                               float4* __restrict__ radiance, float4* __restrict__ pending,
                                                               uint32_t* __restrict__ ovf, uint32_t* __restrict__ dyn,
                                                               const uint32_t* __restrict__ item_of,
@@ -1021,36 +1030,37 @@ __global__ __launch_bounds__(TRACE_BLOCK, DYN ? 7 : 8) void k_shadow_multi(Shado
     const size_t gtid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t* my_lds = lds + threadIdx.x;
     uint32_t* my_ovf = ovf ? ovf + gtid : nullptr;
-    const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)(gtid / 64);
+    const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(gtid / 64));
     RayChunks ch = chunks_first<DYN>(wave, nwaves, n);
     const uint64_t below = (1ull << __lane_id()) - 1ull;
     VisitCount vc;
-    bool active = false;
-    uint32_t rid = 0, id = 0;
+    uint32_t rid = INVALID, id = 0;   // the lane's ray (INVALID: none) and its path
     RayPre r;
     Trav t;
     TravView view{nullptr, nullptr, 0u};
     while (true) {
-        const uint64_t busy = __ballot(active);
-        const uint32_t nidle = 64u - (uint32_t)__popcll(busy);
-        const bool refill = nidle >= (uint32_t)REFILL_IDLE || busy == 0;
-        if (DYN && refill && ch.next >= ch.end && !ch.exhausted) chunks_refill(ch, dyn);
-        if (refill && ch.next < ch.end) {
-            const uint32_t my = ch.next + (uint32_t)__popcll(~busy & below);
-            if (!active && my < ch.end) {
-                rid = my;
-                float4 o4 = sq.o[rid], d4 = sq.d[rid];
-                id = __float_as_uint(d4.w);
-                const MultiItem& it = items[item_of[id]];
-                view.nodes = it.nodes;
-                view.tris = it.tris;
-                r = ray_setup(xyz(o4), xyz(d4));
-                trav_init(t, o4.w);
-                active = true;
+        const uint64_t busy = wave_ballot(rid != INVALID);
+        const uint32_t nidle = 64u - wave_count(busy);
+        if (nidle >= (uint32_t)REFILL_IDLE) {
+            if (DYN && ch.next >= ch.end && !ch.exhausted) chunks_refill(ch, dyn);
+            if (ch.next < ch.end) {
+                const uint32_t my = ch.next + (uint32_t)__popcll(~busy & below);
+                if (rid == INVALID && my < ch.end) {
+                    rid = my;
+                    float4 o4 = sq.o[rid], d4 = sq.d[rid];
+                    id = __float_as_uint(d4.w);
+                    const MultiItem& it = items[item_of[id]];
+                    view.nodes = it.nodes;
+                    view.tris = it.tris;
+                    r = ray_setup(xyz(o4), xyz(d4));
+                    trav_init(t, o4.w);
+                }
+                ch.next = min(ch.next + nidle, ch.end);
+            } else if (busy == 0) {
+                break;
             }
-            ch.next = min(ch.next + nidle, ch.end);
         }
-        if (__ballot(active) == 0) break;
+        const bool active = rid != INVALID;
         bool occ = false;
         const bool done = trav_step<true, TRACE_LDS_DEPTH, false>(active, view, r, t, nullptr, my_lds, TRACE_BLOCK,
                                                                    my_ovf, nthreads, vc, &occ);
@@ -1063,7 +1073,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, DYN ? 7 : 8) void k_shadow_multi(Shado
                 } else if (!occ) {
                     radiance[id] = f4(xyz(radiance[id]) + c, 0.0f);
                 }
-                active = false;
+                rid = INVALID;
             }
         }
     }
@@ -1150,7 +1160,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) v
     const size_t gtid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t* my_lds = lds + threadIdx.x;
     uint32_t* my_ovf = a.ovf ? a.ovf + gtid : nullptr;
-    const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)(gtid / 64);
+    const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(gtid / 64));
     const uint32_t lanes = a.lanes, lane = __lane_id();
     const uint64_t below = (1ull << lane) - 1ull;
     RayChunks ch = chunks_first<true>(wave, nwaves, n, lanes);

@@ -328,7 +328,7 @@ XT_HD f3 tex_texel(const TexRef& m, int x, int y) {
         x = min(max(x, 0), m.w - 1);
     }
     y = min(max(y, 0), m.h - 1);
-    const float4 t = m.texels[(size_t)y * m.w + x];
+    const float4 t = in_global(m.texels)[(size_t)y * m.w + x];
     return mk(t.x, t.y, t.z);
 }
 // Texture::rgb(uv), bilinear filter (Texture.h:83-103)
@@ -378,7 +378,8 @@ XT_HD f3 env_radiance(const DevEnv& e, f3 d) {
     return L;
 }
 // largest i in [0, n) with cdf[i] <= u (cdf[0] = 0, cdf[n] = 1)
-XT_HD int cdf_find(const float* cdf, int n, float u) {
+template <class Cdf>
+XT_HD int cdf_find(const Cdf& cdf, int n, float u) {
     int lo = 0, hi = n - 1;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
@@ -392,10 +393,11 @@ XT_HD int cdf_find(const float* cdf, int n, float u) {
 XT_HD f3 env_map_sample(const DevEnv& e, float u1, float u2) {
     const float PI = 3.14159265358979323846f;
     const int W = e.map_w, H = e.map_h;
-    const int y = cdf_find(e.map_marg, H, u1);
-    const float dy = e.map_marg[y + 1] - e.map_marg[y];
-    const float fy = dy > 0.0f ? (u1 - e.map_marg[y]) / dy : 0.5f;
-    const float* c = e.map_cond + (size_t)y * (W + 1);
+    const auto marg = in_global(e.map_marg);
+    const int y = cdf_find(marg, H, u1);
+    const float dy = marg[y + 1] - marg[y];
+    const float fy = dy > 0.0f ? (u1 - marg[y]) / dy : 0.5f;
+    const auto c = in_global(e.map_cond) + (size_t)y * (W + 1);
     const int x = cdf_find(c, W, u2);
     const float dx = c[x + 1] - c[x];
     const float fx = dx > 0.0f ? (u2 - c[x]) / dx : 0.5f;
@@ -410,7 +412,7 @@ XT_HD float env_map_pdf(const DevEnv& e, f3 du) {
     const LatLongUV uv = env_latlong_uv(du);
     const int x = min((int)(uv.u * e.map_w), e.map_w - 1), y = min((int)(uv.v * e.map_h), e.map_h - 1);
     const float st = sqrtf(fmaxf(0.0f, 1.0f - du.y * du.y));
-    return st > 0.0f ? e.map_pdf[(size_t)y * e.map_w + x] / st : 0.0f;
+    return st > 0.0f ? in_global(e.map_pdf)[(size_t)y * e.map_w + x] / st : 0.0f;
 }
 
 // Environment light strategy: pick env vs area lights, then sun cone vs
@@ -463,7 +465,8 @@ __device__ __forceinline__ f3 xyz(float4 v) { return mk(v.x, v.y, v.z); }
 // normal-mapped hits run it.
 static __device__ __noinline__ f3 normal_mapped(const float4* attr, bool tangents, int w, int h, const float4* texels,
                                                 float b0, float b1, f3 sn) {
-    const float4 a0 = attr[0], a1 = attr[1], a2 = attr[2], a3 = attr[3], a4 = attr[4], a5 = attr[5];
+    const auto at = in_global(attr);
+    const float4 a0 = at[0], a1 = at[1], a2 = at[2], a3 = at[3], a4 = at[4], a5 = at[5];
     const f3 uv = lerp3(mk(a0.w, a1.w, 0.0f), mk(a2.w, a3.w, 0.0f), mk(a4.w, a5.w, 0.0f), b0, b1);
     f3 tg = splat(0.0f), bt = splat(0.0f);
     if (tangents) {
@@ -481,7 +484,7 @@ static __device__ __noinline__ f3 normal_mapped(const float4* attr, bool tangent
 // NMAP: the scene has normal maps (the lookup is compiled in only then).
 template <bool NMAP = true>
 __device__ __forceinline__ Surf make_surf(const DevScene& sc, uint32_t slot, f3 d, float b0, float b1) {
-    const float4* tr = sc.tris + (size_t)slot * TRI_F4;
+    const auto tr = in_global(sc.tris) + (size_t)slot * TRI_F4;
     float4 v0 = tr[0], v1 = tr[1], v2 = tr[2];
     f3 p0 = xyz(v0), p1 = xyz(v1), p2 = xyz(v2);
     Surf s;
@@ -492,7 +495,7 @@ __device__ __forceinline__ Surf make_surf(const DevScene& sc, uint32_t slot, f3 
     f3 wo = normalize(-d);
     f3 n;
     if (flags & TRI_FLAG_NORMALS) {
-        const float4* nr = sc.normals + (size_t)slot * TRI_F4;
+        const auto nr = in_global(sc.normals) + (size_t)slot * TRI_F4;
         n = normalize(lerp3(xyz(nr[0]), xyz(nr[1]), xyz(nr[2]), b0, b1));
     } else {
         n = normalize(cross(p1 - p0, p2 - p0));
@@ -500,7 +503,7 @@ __device__ __forceinline__ Surf make_surf(const DevScene& sc, uint32_t slot, f3 
     f3 sn = face_forward(n, wo);
     const uint32_t nm = flags >> TRI_NMAP_SHIFT;
     if (NMAP && nm != 0) {
-        const DevTexture t = sc.textures[nm - 1];
+        const DevTexture t = in_global(sc.textures)[nm - 1];
         sn = normal_mapped(sc.nmap_attr + (size_t)slot * NMAP_F4, (flags & TRI_FLAG_TANGENTS) != 0, t.w, t.h, t.texels,
                            b0, b1, sn);
     }

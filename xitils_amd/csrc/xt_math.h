@@ -19,11 +19,59 @@
 
 namespace xt {
 
+// An array reached through a pointer that was itself read from memory (a scene
+// record, an item table), known to lie in global memory.  The compiler knows
+// that only of kernel arguments; through other pointers it loads with flat
+// instructions, which also check the LDS aperture and return out of order, so
+// that every wait waits for all of them.
+template <class T>
+struct GlobalArray {
+    const T* p;
+    XT_HD GlobalArray operator+(size_t n) const { return GlobalArray{p + n}; }
+    XT_HD T operator[](size_t i) const {
+#ifdef __HIP_DEVICE_COMPILE__
+        constexpr int WORDS = sizeof(T) / 4, STEP = WORDS % 4 == 0 ? 4 : WORDS % 2 == 0 ? 2 : 1;
+        static_assert(sizeof(T) % 4 == 0 && alignof(T) >= 4, "words");
+        typedef uint32_t vec __attribute__((ext_vector_type(STEP == 1 ? 2 : STEP), aligned(alignof(T) < 4 * STEP ? alignof(T) : 4 * STEP)));
+        T r;
+        if constexpr (STEP == 1) {
+            const __attribute__((address_space(1))) uint32_t* q = (const __attribute__((address_space(1))) uint32_t*)(p + i);
+            uint32_t v[WORDS];
+#pragma unroll
+            for (int k = 0; k < WORDS; ++k) v[k] = q[k];
+            __builtin_memcpy(&r, v, sizeof(T));
+        } else {
+            const __attribute__((address_space(1))) vec* q = (const __attribute__((address_space(1))) vec*)(p + i);
+            vec v[WORDS / STEP];
+#pragma unroll
+            for (int k = 0; k < WORDS / STEP; ++k) v[k] = q[k];
+            __builtin_memcpy(&r, v, sizeof(T));
+        }
+        return r;
+#else
+        return p[i];
+#endif
+    }
+};
 struct f3 {
     float x, y, z;
 };
 
 XT_HD f3 mk(float x, float y, float z) { return f3{x, y, z}; }
+template <class T>
+XT_HD GlobalArray<T> in_global(const T* p) {
+    return GlobalArray<T>{p};
+}
+// The first three floats of element i, as one 12-byte load.
+XT_HD f3 global_xyz(const GlobalArray<float4>& a, size_t i) {
+#ifdef __HIP_DEVICE_COMPILE__
+    typedef float vec __attribute__((ext_vector_type(3)));
+    const vec v = *(const __attribute__((address_space(1))) vec*)(a.p + i);
+    return f3{v.x, v.y, v.z};
+#else
+    return f3{a.p[i].x, a.p[i].y, a.p[i].z};
+#endif
+}
 XT_HD f3 splat(float v) { return f3{v, v, v}; }
 XT_HD f3 operator+(f3 a, f3 b) { return f3{a.x + b.x, a.y + b.y, a.z + b.z}; }
 XT_HD f3 operator-(f3 a, f3 b) { return f3{a.x - b.x, a.y - b.y, a.z - b.z}; }

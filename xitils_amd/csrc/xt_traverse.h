@@ -20,6 +20,7 @@ constexpr float BOX_MARGIN = 1.0f + 0x1p-20f;
 struct RayPre {
     f3 o, d;
     float ix, iy, iz;      // 1 / d (Bounds.h:179)
+    float ex, ey, ez;      // 2^-22 with the sign of d: how far a node's offset is pushed outward (node_slabs_q)
     bool sx_neg, sy_neg, sz_neg;
     int px, py, pz;        // float4 index of the near plane per axis: x 0|1, y 2|3, z 4|5
     int kx, ky, kz;        // permutation (TriangleIndexed.h:88-91)
@@ -33,6 +34,9 @@ __device__ __forceinline__ RayPre ray_setup(f3 o, f3 d) {
     r.ix = 1.0f / d.x;
     r.iy = 1.0f / d.y;
     r.iz = 1.0f / d.z;
+    r.ex = copysignf(0x1p-22f, r.ix);
+    r.ey = copysignf(0x1p-22f, r.iy);
+    r.ez = copysignf(0x1p-22f, r.iz);
     r.sx_neg = signbit(d.x);
     r.sy_neg = signbit(d.y);
     r.sz_neg = signbit(d.z);
@@ -96,7 +100,8 @@ struct TraceResult {
 
 
 // One float of row `row` (0..7) for child k of a node.
-__device__ __forceinline__ float node_row(const float4* nd, int row, int k) {
+template <class Node>
+__device__ __forceinline__ float node_row(const Node& nd, int row, int k) {
     const float4 v = nd[row * NODE_ROW_F4 + (k >> 2)];
     const int c = k & 3;
     return c == 0 ? v.x : (c == 1 ? v.y : (c == 2 ? v.z : v.w));
@@ -105,7 +110,8 @@ __device__ __forceinline__ float node_row(const float4* nd, int row, int k) {
 // The node's child slab tests; returns entry distances (inf = miss).  The
 // near and far planes of each axis are picked by address (the ray's
 // direction signs), so no per-child selects are needed.
-__device__ __forceinline__ void node_slabs(const float4* __restrict__ nd, const RayPre& r, float cull,
+template <class Node>
+__device__ __forceinline__ void node_slabs(const Node& nd, const RayPre& r, float cull,
                                            float tn[BVH_WIDTH]) {
     float4 rows[6][NODE_ROW_F4];
     const int pr[6] = {r.px, r.px ^ 1, r.py, r.py ^ 1, r.pz, r.pz ^ 1};
@@ -159,9 +165,9 @@ __device__ __forceinline__ void node_slabs_q(const float4 w0, const float4 w1, c
     ch[3] = __float_as_int(w1.w);
     const float stx = ldexpf(1.0f, ex), sty = ldexpf(1.0f, ey), stz = ldexpf(1.0f, ez);
     const float ox = w0.x - r.o.x, oy = w0.y - r.o.y, oz = w0.z - r.o.z;
-    const float sx = copysignf(fabsf(ox) * 0x1p-22f, r.ix), sy = copysignf(fabsf(oy) * 0x1p-22f, r.iy),
-                sz = copysignf(fabsf(oz) * 0x1p-22f, r.iz);
-    const float nox = ox - sx, fox = ox + sx, noy = oy - sy, foy = oy + sy, noz = oz - sz, foz = oz + sz;
+    const float nox = fmaf(-fabsf(ox), r.ex, ox), fox = fmaf(fabsf(ox), r.ex, ox);
+    const float noy = fmaf(-fabsf(oy), r.ey, oy), foy = fmaf(fabsf(oy), r.ey, oy);
+    const float noz = fmaf(-fabsf(oz), r.ez, oz), foz = fmaf(fabsf(oz), r.ez, oz);
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
         auto q = [&](uint32_t v) { return (float)((v >> (8 * k)) & 255u); };
@@ -185,7 +191,7 @@ constexpr int TOP_F4 = BVH_QUANT && BVH_TOP_MAX_NODES > 0 ? BVH_TOP_MAX_NODES * 
 __device__ __forceinline__ void stage_top_nodes(float4* top, const DevScene& sc) {
     if constexpr (BVH_QUANT && BVH_TOP_MAX_NODES > 0) {
         const uint32_t n = min(sc.top_nodes, (uint32_t)BVH_TOP_MAX_NODES) * NODE_F4;
-        for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) top[i] = sc.nodes[i];
+        for (uint32_t i = threadIdx.x; i < n; i += blockDim.x) top[i] = in_global(sc.nodes)[i];
         __syncthreads();
     }
 }
@@ -215,6 +221,14 @@ struct VisitCount {
 #define XT_REFILL_IDLE 16
 #endif
 constexpr int REFILL_IDLE = XT_REFILL_IDLE;   // 8 and 24: 1080p frame 1.2% and 0.3% slower; 32 no better
+
+// Lanes for which p holds, and how many, both in scalar registers: the ballot
+// builtin takes the compare's mask as it is (__ballot turns it into a number
+// per lane and back), and the count is read as a scalar.
+__device__ __forceinline__ uint64_t wave_ballot(bool p) { return __builtin_amdgcn_ballot_w64(p); }
+__device__ __forceinline__ uint32_t wave_count(uint64_t mask) {
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)__popcll(mask));
+}
 
 // Which rays a wave traces.  DYN = false: an even contiguous share per wave.
 // DYN = true (large queues): the queue is cut into chunks of a quarter of an
@@ -253,12 +267,15 @@ __device__ __forceinline__ RayChunks chunks_first(uint32_t wave, uint32_t nwaves
         c.exhausted = true;
         return c;
     }
+    // (64-bit minima by hand: min() of two uint64_t goes through doubles)
+    auto upto = [&](uint64_t v) { return v < n ? (uint32_t)v : n; };
     const uint64_t quarter = ((uint64_t)n + 4ull * nwaves - 1) / (4ull * nwaves);
-    c.chunk = (uint32_t)min<uint64_t>(max<uint64_t>(quarter, min_chunk), TRAV_CHUNK);
+    c.chunk = max(upto(quarter), min_chunk);
+    if (c.chunk > TRAV_CHUNK) c.chunk = TRAV_CHUNK;
     const uint64_t b = (uint64_t)wave * c.chunk;
-    c.next = (uint32_t)min<uint64_t>(b, n);
-    c.end = (uint32_t)min<uint64_t>(b + c.chunk, n);
-    c.base = (uint32_t)min<uint64_t>((uint64_t)nwaves * c.chunk, n);
+    c.next = upto(b);
+    c.end = upto(b + c.chunk);
+    c.base = upto((uint64_t)nwaves * c.chunk);
     c.n = n;
     c.exhausted = c.base >= n;   // no chunk is left for the cursor
     return c;
@@ -267,12 +284,12 @@ __device__ __forceinline__ RayChunks chunks_first(uint32_t wave, uint32_t nwaves
 __device__ __forceinline__ void chunks_refill(RayChunks& c, uint32_t* dyn) {
     uint32_t got = 0;
     if (__lane_id() == 0) got = atomicAdd(&dyn[0], c.chunk);
-    const uint64_t g = (uint64_t)__builtin_amdgcn_readfirstlane(got) + c.base;
+    const uint64_t g = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)got) + c.base;
     if (g >= c.n) {
         c.exhausted = true;
     } else {
         c.next = (uint32_t)g;
-        c.end = (uint32_t)min<uint64_t>(g + c.chunk, c.n);
+        c.end = g + c.chunk < c.n ? (uint32_t)(g + c.chunk) : c.n;
     }
 }
 // Every thread of the block calls it once its wave has left the loop.
@@ -311,7 +328,7 @@ template <bool ANY, int LDS_DEPTH, bool COUNT, class SV>
 __device__ __forceinline__ bool visit_node(const SV& sc, const RayPre& r, Trav& t, const float4* top,
                                            uint32_t* lds, int lds_stride, uint32_t* ovf, size_t ovf_stride,
                                            VisitCount& vc) {
-    const float4* nd = sc.nodes + (size_t)t.node * NODE_F4;
+    const auto nd = in_global(sc.nodes) + (size_t)t.node * NODE_F4;
     if (COUNT) vc.nodes++;
     float tn[BVH_WIDTH];
     int ch[BVH_WIDTH];
@@ -393,24 +410,23 @@ __device__ __forceinline__ bool visit_node(const SV& sc, const RayPre& r, Trav& 
             XT_CSWAP(1, 2) XT_CSWAP(3, 4) XT_CSWAP(5, 6)
         }
 #undef XT_CSWAP
-        int nhit = 0;
-#pragma unroll
-        for (int k = 0; k < BVH_WIDTH; ++k) nhit += tn[k] < INFINITY;
-        if (nhit > 0) {
+        if (tn[0] < INFINITY) {
             if (BVH_WIDTH == 4 && t.sp + BVH_WIDTH - 1 <= LDS_DEPTH) {
-                // room in LDS: the far-to-near order ch[nhit-1] .. ch[1] goes
-                // to fixed slots sp, sp+1, sp+2 by selects; slots at or above
-                // the new top hold leftovers that are never read
-                const int v0 = nhit == 4 ? ch[3 % BVH_WIDTH] : (nhit == 3 ? ch[2] : ch[1]);
-                const int v1 = nhit == 4 ? ch[2] : ch[1];
+                // room in LDS: the far-to-near order of the hit children but
+                // the nearest goes to fixed slots sp, sp+1, sp+2 by selects;
+                // slots at or above the new top hold leftovers that are never read
+                const bool h1 = tn[1] < INFINITY, h2 = tn[2] < INFINITY, h3 = tn[3 % BVH_WIDTH] < INFINITY;
                 uint32_t* s = lds + t.sp * lds_stride;
-                s[0] = (uint32_t)v0;
-                s[lds_stride] = (uint32_t)v1;
+                s[0] = (uint32_t)(h3 ? ch[3 % BVH_WIDTH] : h2 ? ch[2] : ch[1]);
+                s[lds_stride] = (uint32_t)(h3 ? ch[2] : ch[1]);
                 s[2 * lds_stride] = (uint32_t)ch[1];
-                t.sp += nhit - 1;
+                t.sp += (int)h1 + (int)h2 + (int)h3;
                 t.node = ch[0];
                 return true;
             }
+            int nhit = 0;
+#pragma unroll
+            for (int k = 0; k < BVH_WIDTH; ++k) nhit += tn[k] < INFINITY;
             // far children first; static indices keep ch[] in registers
 #pragma unroll
             for (int k = BVH_WIDTH - 1; k >= 1; --k) {
@@ -430,7 +446,7 @@ __device__ __forceinline__ bool visit_node(const SV& sc, const RayPre& r, Trav& 
 // Primitive id of the triangle in sorted slot `slot` (the w of its first vertex).
 template <class SV>
 __device__ __forceinline__ uint32_t prim_of_slot(const SV& sc, uint32_t slot) {
-    return __float_as_uint(sc.tris[(size_t)slot * TRI_F4].w);
+    return __float_as_uint(in_global((const float*)sc.tris)[(size_t)slot * (4 * TRI_F4) + 3]);
 }
 
 // Tests the first triangle of leaf code `leaf` (< 0); returns the code of the
@@ -439,12 +455,13 @@ template <bool COUNT, class SV>
 __device__ __forceinline__ int visit_tri(const SV& sc, const RayPre& r, Trav& t, int leaf, VisitCount& vc, bool any,
                                          bool* occ) {
     uint32_t code = (uint32_t)(~leaf);
-    uint32_t first = code >> 3, cnt = (code & 7u) + 1u;
+    uint32_t first = code >> 3;
     if (COUNT) vc.tris++;
-    const float4* tr = sc.tris + (size_t)first * TRI_F4;
-    float4 v0 = tr[0], v1 = tr[1], v2 = tr[2];
+    const auto tr = in_global(sc.tris) + (size_t)first * TRI_F4;
+    const float4 v0 = tr[0];
+    const f3 v1 = global_xyz(tr, 1), v2 = global_xyz(tr, 2);
     float th, b0, b1;
-    if (tri_test(xyz(v0), xyz(v1), xyz(v2), r, t.tmax, &th, &b0, &b1)) {
+    if (tri_test(xyz(v0), v1, v2, r, t.tmax, &th, &b0, &b1)) {
         if (any) {
             *occ = true;
             return 0;
@@ -461,17 +478,23 @@ __device__ __forceinline__ int visit_tri(const SV& sc, const RayPre& r, Trav& t,
             t.cull = fminf(t.tmax, th);
         }
     }
-    // rest of the leaf: first + 1, count - 1
-    return cnt > 1 ? ~(int)(((first + 1u) << 3) | (cnt - 2u)) : 0;
+    // rest of the leaf: first + 1, count - 1, so the code (first << 3 | count - 1) plus 7
+    return (code & 7u) ? leaf - 7 : 0;
 }
 
-// Pops the next entry into t.node; false when the stack is empty.
+// Pops the next entry into t.node; false when the stack is empty.  The empty
+// asm keeps the LDS read an LDS read: left to itself the compiler merges it
+// with the spill column's into one flat load, which takes the vector-memory
+// path and its latency.
 template <int LDS_DEPTH>
 __device__ __forceinline__ bool trav_pop(Trav& t, const uint32_t* lds, int lds_stride, const uint32_t* ovf,
                                          size_t ovf_stride) {
     if (t.sp == 0) return false;
     --t.sp;
-    t.node = (int)(t.sp < LDS_DEPTH ? lds[t.sp * lds_stride] : ovf[(size_t)(t.sp - LDS_DEPTH) * ovf_stride]);
+    uint32_t e = lds[min(t.sp, LDS_DEPTH - 1) * lds_stride];
+    asm("" : "+v"(e));
+    if (t.sp >= LDS_DEPTH) e = ovf[(size_t)(t.sp - LDS_DEPTH) * ovf_stride];
+    t.node = (int)e;
     return true;
 }
 
