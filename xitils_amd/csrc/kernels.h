@@ -75,6 +75,14 @@ struct PathQueue {
     float4* e;
     uint32_t* rec;
 };
+// Queue lengths, four words: 2 k is the length of path queue k, 2 k + 1 that of
+// the shadow queue filled beside it.  A pair is one 64-bit counter to the shade
+// kernel, which appends to both with one atomic.
+__host__ __device__ __forceinline__ uint32_t* path_count(uint32_t* counts, int k) { return counts + 2 * k; }
+__host__ __device__ __forceinline__ uint32_t* shadow_count(uint32_t* counts, int k) { return counts + 2 * k + 1; }
+__host__ __device__ __forceinline__ unsigned long long* pair_count(uint32_t* counts, int k) {
+    return (unsigned long long*)(counts + 2 * k);
+}
 constexpr uint32_t QF_PENDING = 1u;   // the previous vertex's NEE result waits in pending[id]
 
 // Shadow-ray queue (48 B per entry):
@@ -188,7 +196,7 @@ __global__ void k_count_from_window(uint32_t* count, const MultiCursor* c);
 __global__ void k_generate_multi(MultiBatch mb, PathQueue q, float4* radiance);
 template <bool NMAP>
 __global__ void k_shade_multi(MultiBatch mb, PathQueue qin, const uint32_t* count_in, const float4* hits,
-                              PathQueue qout, uint32_t* count_out, ShadowQueue sq, uint32_t* count_shadow,
+                              PathQueue qout, unsigned long long* counts_out, ShadowQueue sq,
                               float4* radiance, float4* pending);
 __global__ void k_accumulate_multi(MultiBatch mb, const float4* radiance);
 
@@ -236,11 +244,11 @@ __global__ void k_walk(WalkArgs a);
 __global__ void k_generate(WaveParams wp, PathQueue q, float4* radiance);
 template <bool GUIDE, bool NMAP, bool SORT>
 __global__ void k_shade(WaveParams wp, const DevScene* scene, PathQueue qin, const uint32_t* count_in, const float4* hits,
-                        PathQueue qout, uint32_t* count_out, ShadowQueue sq, uint32_t* count_shadow,
+                        PathQueue qout, unsigned long long* counts_out, ShadowQueue sq,
                         float4* radiance, float4* pending, GuideRender gr);
 template <bool COUNT, bool DYN = false>
 __global__ void k_shadow(DevScene sc, ShadowQueue sq, const uint32_t* count, float4* radiance, float4* pending,
-                         uint32_t* ovf, uint32_t* dyn, unsigned long long* visit_totals, const uint32_t* counts3,
+                         uint32_t* ovf, uint32_t* dyn, unsigned long long* visit_totals, const uint32_t* counts4,
                          uint32_t* counts_out);
 __global__ void k_accumulate(WaveParams wp, const float4* radiance, void* film, int film_f64);
 __global__ void k_zero_u32(uint32_t* p, uint32_t n);

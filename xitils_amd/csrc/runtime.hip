@@ -45,7 +45,7 @@ struct RenderBuffers {
     float4* pending = nullptr;
     uint32_t* rec[2] = {};           // training-record index per path-queue entry (allocated on demand)
     float* lobes = nullptr;          // decoded guide mixtures per path-queue entry (allocated on demand)
-    uint32_t* counts = nullptr;      // [0], [1]: path queues, [2]: shadow queue
+    uint32_t* counts = nullptr;      // queue lengths (path_count, shadow_count)
     uint32_t* host_counts = nullptr; // pinned, RB_RING slots of 4 counts (bounce rounds in flight)
     uint32_t* host_counts_dev = nullptr;  // the same memory's device address (written by k_shadow)
     hipEvent_t round_ev[RB_RING] = {};
@@ -178,8 +178,8 @@ struct xt_scene {
     GuideState guide;
 };
 
-using ShadeKernel = void (*)(WaveParams, const DevScene*, PathQueue, const uint32_t*, const float4*, PathQueue, uint32_t*,
-                            ShadowQueue, uint32_t*, float4*, float4*, GuideRender);
+using ShadeKernel = void (*)(WaveParams, const DevScene*, PathQueue, const uint32_t*, const float4*, PathQueue,
+                            unsigned long long*, ShadowQueue, float4*, float4*, GuideRender);
 // The shade kernel for a render: guided or not, with the normal-mapping
 // materials or not, and with the block-local material partition
 // (XT_FLAG_SORT_MATERIALS) or not -- separate instantiations, so the plain
@@ -1277,7 +1277,7 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                 wa.scene = s->d_ds;
                 if (q >= 0) {
                     wa.q = rb.q[q];
-                    wa.count = rb.counts + q;
+                    wa.count = path_count(rb.counts, q);
                 }
                 wa.pending = rb.pending;
                 wa.radiance = rb.radiance;
@@ -1302,7 +1302,7 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
             } else {
                 hipLaunchKernelGGL(k_generate, dim3(blocks256(wp.num_paths)), dim3(256), 0, s->stream, wp, rb.q[0], rb.radiance);
                 XT_LAUNCHED(result);
-                hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, s->stream, rb.counts + 0, wp.num_paths);
+                hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, s->stream, path_count(rb.counts, 0), wp.num_paths);
                 XT_LAUNCHED(result);
                 tm.add(3, a, tm.mark());
             }
@@ -1341,9 +1341,9 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                                              : (dyn ? k_trace<false, TRACE_LDS_DEPTH, false, false, true>
                                                     : k_trace<false, TRACE_LDS_DEPTH, false, false, false>);
                     hipLaunchKernelGGL(trace, dim3(trace_blocks(s, bound)), dim3(TRACE_BLOCK), 0, s->stream, s->ds,
-                                       rb.q[cur].o, rb.q[cur].d, 1, rb.counts + cur, 0u, rb.hits, nullptr, 0, 0,
-                                       s->d_ovf, rb.dyn, s->counting ? rb.visits : nullptr, rb.counts + (1 - cur),
-                                       rb.counts + 2, nullptr, nullptr);   // also clears the next counters
+                                       rb.q[cur].o, rb.q[cur].d, 1, path_count(rb.counts, cur), 0u, rb.hits, nullptr, 0, 0,
+                                       s->d_ovf, rb.dyn, s->counting ? rb.visits : nullptr,
+                                       path_count(rb.counts, 1 - cur), shadow_count(rb.counts, 1 - cur), nullptr, nullptr);   // also clears the next counters
                     XT_LAUNCHED(result);
                     tm.add(0, a, tm.mark());
                     GuideRender gr{};
@@ -1354,7 +1354,7 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                         uint2* l4 = (uint2*)rb.lobes;
                         float2* l2 = (float2*)(rb.lobes + (size_t)2 * G_LOBES * rb.capacity);
                         hipLaunchKernelGGL(k_guide_infer, dim3(ib), dim3(GI_BLOCK), 0, s->stream, net_r, g.gb, s->ds,
-                                           rb.q[cur], rb.counts + cur, rb.hits, l4, l2, rb.capacity,
+                                           rb.q[cur], path_count(rb.counts, cur), rb.hits, l4, l2, rb.capacity,
                                            g.cfg.max_guided_vertex);
                         XT_LAUNCHED(result);
                         tm.add(4, a, tm.mark());
@@ -1371,15 +1371,15 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                     }
                     a = tm.mark();
                     hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags), dim3(shade_blocks(bound)), dim3(SHADE_BLOCK), 0,
-                                       s->stream, wp, s->d_ds, rb.q[cur], rb.counts + cur, rb.hits, rb.q[1 - cur],
-                                       rb.counts + (1 - cur), rb.sq, rb.counts + 2, rb.radiance, rb.pending, gr);
+                                       s->stream, wp, s->d_ds, rb.q[cur], path_count(rb.counts, cur), rb.hits, rb.q[1 - cur],
+                                       pair_count(rb.counts, 1 - cur), rb.sq, rb.radiance, rb.pending, gr);
                     XT_LAUNCHED(result);
                     tm.add(1, a, tm.mark());
                     a = tm.mark();
                     auto shadow = s->counting ? (dyn ? k_shadow<true, true> : k_shadow<true, false>)
                                               : (dyn ? k_shadow<false, true> : k_shadow<false, false>);
                     hipLaunchKernelGGL(shadow, dim3(trace_blocks(s, bound)), dim3(TRACE_BLOCK), 0, s->stream, s->ds,
-                                       rb.sq, rb.counts + 2, rb.radiance, rb.pending, s->d_ovf, rb.dyn + 2,
+                                       rb.sq, shadow_count(rb.counts, 1 - cur), rb.radiance, rb.pending, s->d_ovf, rb.dyn + 2,
                                        s->counting ? rb.visits + 2 : nullptr, rb.counts,
                                        rb.host_counts_dev + 4 * slot);   // counts -> pinned ring
                     XT_LAUNCHED(result);
@@ -1400,7 +1400,8 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                     }
                     const uint32_t* hc = rb.host_counts + 4 * vs;
                     const uint32_t len = queue_len[vs];
-                    const uint32_t next = hc[(verified & 1) ? 0 : 1], nsh = hc[2];
+                    const int filled = (verified & 1) ? 0 : 1;   // the queues that round filled
+                    const uint32_t next = hc[2 * filled], nsh = hc[2 * filled + 1];
                     if (len > 0) {
                         s->stats.extension_rays += len;
                         s->stats.extend_launches++;
@@ -1550,7 +1551,7 @@ struct BounceBufs {
     float4* hits;
     float4* radiance;
     float4* pending;
-    uint32_t* counts;        // [0], [1]: path queues, [2]: shadow queue
+    uint32_t* counts;        // queue lengths (path_count, shadow_count)
     uint32_t* ovf;           // traversal spill columns for tblocks blocks
     uint32_t* dyn;           // k_walk's chunk cursor and block counter
     uint32_t capacity;       // paths
@@ -1623,17 +1624,17 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
                            dim3(walk_blocks(s, maxpaths, wa.lanes, s->nmap, tmost)), dim3(TRACE_BLOCK), 0, s->stream, wa);
     } else {
         hipLaunchKernelGGL(k_generate, dim3(gblocks), dim3(256), 0, s->stream, wp, b.q[0], b.radiance);
-        hipLaunchKernelGGL(k_count_from_cursor, dim3(1), dim3(1), 0, s->stream, b.counts + 0, cursor);
+        hipLaunchKernelGGL(k_count_from_cursor, dim3(1), dim3(1), 0, s->stream, path_count(b.counts, 0), cursor);
     }
     int cur = 0;
     for (int it = 0; it <= p->max_depth && !whole; ++it) {
         hipLaunchKernelGGL((k_trace<false, TRACE_LDS_DEPTH, false>), dim3(tblocks), dim3(TRACE_BLOCK), 0, s->stream, s->ds,
-                           b.q[cur].o, b.q[cur].d, 1, b.counts + cur, 0u, b.hits, nullptr, 0, 0, b.ovf, nullptr, nullptr,
-                           b.counts + (1 - cur), b.counts + 2);
+                           b.q[cur].o, b.q[cur].d, 1, path_count(b.counts, cur), 0u, b.hits, nullptr, 0, 0, b.ovf, nullptr, nullptr,
+                           path_count(b.counts, 1 - cur), shadow_count(b.counts, 1 - cur));
         GuideRender gr{};
         if (guide) {
             hipLaunchKernelGGL(k_guide_infer, dim3(ib), dim3(GI_BLOCK), 0, s->stream, g.net, g.gb, s->ds, b.q[cur],
-                               b.counts + cur, b.hits, gd.lobes_mk, gd.lobes2, gd.stride, g.cfg.max_guided_vertex);
+                               path_count(b.counts, cur), b.hits, gd.lobes_mk, gd.lobes2, gd.stride, g.cfg.max_guided_vertex);
             gr.lobes_mk = gd.lobes_mk;
             gr.lobes2 = gd.lobes2;
             gr.stride = gd.stride;
@@ -1641,9 +1642,9 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
             gr.max_vertex = g.cfg.max_guided_vertex;
         }
         hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags), dim3(sblocks), dim3(SHADE_BLOCK), 0, s->stream, wp, s->d_ds,
-                           b.q[cur], b.counts + cur, b.hits, b.q[1 - cur], b.counts + (1 - cur), b.sq,
-                           b.counts + 2, b.radiance, b.pending, gr);
-        hipLaunchKernelGGL(k_shadow<false>, dim3(tblocks), dim3(TRACE_BLOCK), 0, s->stream, s->ds, b.sq, b.counts + 2,
+                           b.q[cur], path_count(b.counts, cur), b.hits, b.q[1 - cur], pair_count(b.counts, 1 - cur), b.sq,
+                           b.radiance, b.pending, gr);
+        hipLaunchKernelGGL(k_shadow<false>, dim3(tblocks), dim3(TRACE_BLOCK), 0, s->stream, s->ds, b.sq, shadow_count(b.counts, 1 - cur),
                            b.radiance, b.pending, b.ovf, nullptr, nullptr, b.counts, nullptr);
         cur = 1 - cur;
     }
@@ -1959,7 +1960,7 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
         hipLaunchKernelGGL((nmap ? k_walk<false, true, true> : k_walk<false, false, true>),
                            dim3(tblocks), dim3(TRACE_BLOCK), 0, m.stream, wa);
     } else {
-        hipLaunchKernelGGL(k_count_from_window, dim3(1), dim3(1), 0, m.stream, m.counts, m.cursor);
+        hipLaunchKernelGGL(k_count_from_window, dim3(1), dim3(1), 0, m.stream, path_count(m.counts, 0), m.cursor);
         hipLaunchKernelGGL(k_generate_multi, dim3(gblocks), dim3(256), 0, m.stream, mb, m.q[0], m.radiance);
     }
     int cur = 0;
@@ -1967,18 +1968,18 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
         hipLaunchKernelGGL((dyn ? k_trace<false, TRACE_LDS_DEPTH, false, true, true>
                                 : k_trace<false, TRACE_LDS_DEPTH, false, true, false>),
                            dim3(tblocks), dim3(TRACE_BLOCK), 0, m.stream, s0->ds, m.q[cur].o, m.q[cur].d, 1,
-                           m.counts + cur, 0u, m.hits, nullptr, 0, 0, m.ovf, m.dyn, nullptr, m.counts + (1 - cur),
-                           m.counts + 2, m.item_of, m.items);
+                           path_count(m.counts, cur), 0u, m.hits, nullptr, 0, 0, m.ovf, m.dyn, nullptr,
+                           path_count(m.counts, 1 - cur), shadow_count(m.counts, 1 - cur), m.item_of, m.items);
         if (nmap)
             hipLaunchKernelGGL(k_shade_multi<true>, dim3(sblocks), dim3(SHADE_BLOCK), 0, m.stream, mb, m.q[cur],
-                               m.counts + cur, m.hits, m.q[1 - cur], m.counts + (1 - cur), m.sq, m.counts + 2,
+                               path_count(m.counts, cur), m.hits, m.q[1 - cur], pair_count(m.counts, 1 - cur), m.sq,
                                m.radiance, m.pending);
         else
             hipLaunchKernelGGL(k_shade_multi<false>, dim3(sblocks), dim3(SHADE_BLOCK), 0, m.stream, mb, m.q[cur],
-                               m.counts + cur, m.hits, m.q[1 - cur], m.counts + (1 - cur), m.sq, m.counts + 2,
+                               path_count(m.counts, cur), m.hits, m.q[1 - cur], pair_count(m.counts, 1 - cur), m.sq,
                                m.radiance, m.pending);
         hipLaunchKernelGGL((dyn ? k_shadow_multi<true> : k_shadow_multi<false>), dim3(tblocks), dim3(TRACE_BLOCK), 0,
-                           m.stream, m.sq, m.counts + 2, m.radiance, m.pending, m.ovf, m.dyn + 2, m.item_of, m.items);
+                           m.stream, m.sq, shadow_count(m.counts, 1 - cur), m.radiance, m.pending, m.ovf, m.dyn + 2, m.item_of, m.items);
         cur = 1 - cur;
     }
     hipLaunchKernelGGL(k_accumulate_multi, dim3(gblocks), dim3(256), 0, m.stream, mb, m.radiance);
