@@ -236,8 +236,14 @@ constexpr uint32_t WALK_MAX = 11u << 16;
 constexpr uint32_t WALK_TAIL = 1u << 18;
 // Waves that few paths are spread over, by leaving lanes empty: a wave's step
 // takes as long as the slowest of its rays, so 6 k paths ran in 735 us at 64
-// paths a wave and in 545 / 427 / 413 / 406 us over 512 / 1024 / 2048 / 4096 waves.
+// paths a wave and in 545 / 427 / 413 / 406 us over 512 / 1024 / 2048 / 4096
+// waves (before paths had two lanes).
 constexpr uint32_t WALK_SPREAD = 2048;
+// Paths up to which a wave holds at most 32, each with a second lane for its
+// shadow ray: as many as 4 waves per SIMD hold.  100 k triangle room, us, one
+// lane a path against two: 14 k paths 1111 / 757, 57 k 1763 / 1053, 115 k 2000 /
+// 1364; at 230 k, where two lanes a path need twice the waves, 2220 / 2347.
+constexpr uint32_t WALK_PAIRS = 1u << 17;
 template <bool QUEUE, bool NMAP, bool MULTI>
 __global__ void k_walk(WalkArgs a);
 

@@ -1145,9 +1145,15 @@ __global__ __launch_bounds__(256) void k_accumulate_multi(MultiBatch mb, const f
 // ended take the next path of the wave's chunk.  The same functions in the
 // same order per path as the queued kernels, so the same radiance.
 //
-// Between vertices the wave traces every lane's two rays to their ends (a
-// lane goes on to its extension ray as soon as WALK_SWITCH lanes, or all that
-// are left, have their shadow ray done), then shades together.
+// Between vertices the wave traces every path's two rays to their ends, then
+// shades together.  A full wave's lane traces them one after the other (going
+// on to its extension ray as soon as WALK_SWITCH lanes, or all that are left,
+// have their shadow ray done).  With at most 32 paths -- few in all, or the
+// last of a wave, moved together -- lane l + 32 traces the shadow ray while
+// lane l traces the extension ray: such a wave's time is the chain of its
+// slowest path, some 17 us of traversal and 14 of shading a vertex (1 k
+// triangles), where one ray after the other took 40 us.  96 x 64: 373 -> 293 us;
+// 800 x 800, paths ended by roulette alone: 2.83 -> 2.55 ms.
 #ifndef XT_WALK_SWITCH
 #define XT_WALK_SWITCH 8
 #endif
@@ -1176,18 +1182,18 @@ __global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) v
     if constexpr (!MULTI) c0 = shade_const(wp0, *a.scene);
     // the lane's path: its next extension ray, the sample that made it, the
     // radiance so far and the light sample its shadow ray decides on
-    bool alive = false, has_ext = false, has_pend = false;
+    bool alive = false, has_ext = false, has_sh = false;
     uint32_t id = 0, v = 0, item = 0, n_ext = 0, n_sh = 0;
-    f3 eo = splat(0.0f), ed = eo, weight = eo, meval = eo, rad = eo, c = eo;
-    float pdf = 0.0f, pe = 0.0f;
+    f3 eo = splat(0.0f), ed = eo, weight = eo, meval = eo, rad = eo, c = eo, so = eo, sd = eo;
+    float pdf = 0.0f, pe = 0.0f, stmax = 0.0f;
     enum { IDLE, SHADOW, EXTEND, SWITCH };   // SWITCH: shadow ray done, extension ray next
-    int mode = IDLE;
+    bool pair = lanes <= 32;   // two lanes per path
     RayPre r;
     Trav t;
     TravView view{nullptr, nullptr, 0u};
     while (true) {
-        const uint64_t busy = __ballot(alive);
-        const uint32_t nidle = lanes - (uint32_t)__popcll(busy);
+        uint64_t busy = wave_ballot(alive);
+        const uint32_t nidle = lanes - wave_count(busy);
         const bool refill = busy == 0 || nidle * 4 >= lanes;
         if (refill && ch.next >= ch.end && !ch.exhausted) chunks_refill(ch, a.dyn);
         if (refill && ch.next < ch.end) {
@@ -1198,7 +1204,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) v
                     id = __float_as_uint(d4.w);
                     const uint32_t vf = __float_as_uint(w4.w);
                     v = vf & 0xFFFFFFu;
-                    has_pend = ((vf >> 24) & QF_PENDING) != 0;
+                    const bool has_pend = ((vf >> 24) & QF_PENDING) != 0;
                     const float4 e4 = v > 1 ? a.q.e[my] : make_float4(1.0f, 1.0f, 1.0f, 0.0f);
                     pdf = o4.w;
                     pe = e4.w;
@@ -1224,20 +1230,84 @@ __global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) v
                     v = 1;
                     pdf = pe = 0.0f;
                     weight = meval = splat(1.0f);
-                    rad = splat(0.0f);
-                    has_pend = false;
+                    rad = c = splat(0.0f);
                 }
                 if constexpr (MULTI) {
                     view.nodes = mb.items[item].nodes;
                     view.tris = mb.items[item].tris;
                 }
-                alive = true;
-                mode = SWITCH;
+                alive = has_ext = true;
+                has_sh = false;
             }
             ch.next = min(ch.next + nidle, ch.end);
+            busy = wave_ballot(alive);
         }
-        if (__ballot(alive) == 0) break;
-        // the rays of this vertex
+        if (busy == 0) break;
+        if (!pair && ch.exhausted && ch.next >= ch.end && wave_count(busy) <= 32) {
+            // the wave's last paths, moved to its first lanes
+            pair = true;
+            uint32_t* const from = lds + (threadIdx.x & ~63u);   // the stacks are empty here
+            if (alive) from[__popcll(busy & below)] = lane;
+            const bool keep = lane < wave_count(busy);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const int src = keep ? (int)from[lane] : (int)lane;
+            auto move3 = [&](f3 x) { return mk(__shfl(x.x, src), __shfl(x.y, src), __shfl(x.z, src)); };
+            eo = move3(eo);
+            ed = move3(ed);
+            weight = move3(weight);
+            meval = move3(meval);
+            rad = move3(rad);
+            c = move3(c);
+            so = move3(so);
+            sd = move3(sd);
+            pdf = __shfl(pdf, src);
+            pe = __shfl(pe, src);
+            stmax = __shfl(stmax, src);
+            id = __shfl(id, src);
+            v = __shfl(v, src);
+            if constexpr (MULTI) {
+                item = __shfl(item, src);
+                view.nodes = mb.items[item].nodes;
+                view.tris = mb.items[item].tris;
+            }
+            const uint32_t flags = __shfl((uint32_t)has_ext | (uint32_t)has_sh << 1, src);
+            alive = keep;
+            has_ext = keep && (flags & 1u);
+            has_sh = keep && (flags & 2u);
+        }
+        // the rays of this vertex: a path's light sample c is added now (a path
+        // that ends) or at its next vertex, unless the shadow ray is blocked
+        int mode = !alive ? IDLE : has_sh && !pair ? SHADOW : has_ext ? EXTEND : IDLE;
+        bool occluded = false;
+        n_sh += alive && has_sh ? 1u : 0u;
+        f3 ro = mode == SHADOW ? so : eo, rd = mode == SHADOW ? sd : ed;
+        float rt = mode == SHADOW ? stmax : INFINITY;   // extension rays: tMax = Infinity (PathTracer.h:167)
+        if (pair) {
+            const int owner = (int)(lane & 31u);
+            const bool theirs = __shfl((int)(alive && has_sh), owner) != 0;
+            const f3 o2 = mk(__shfl(so.x, owner), __shfl(so.y, owner), __shfl(so.z, owner));
+            const f3 d2 = mk(__shfl(sd.x, owner), __shfl(sd.y, owner), __shfl(sd.z, owner));
+            const float t2 = __shfl(stmax, owner);
+            if (lane >= 32 && theirs) {
+                mode = SHADOW;
+                ro = o2;
+                rd = d2;
+                rt = t2;
+            }
+            if constexpr (MULTI) {
+                const uint32_t it2 = __shfl(item, owner);
+                if (lane >= 32 && theirs) {
+                    view.nodes = mb.items[it2].nodes;
+                    view.tris = mb.items[it2].tris;
+                }
+            }
+        }
+        n_ext += mode == EXTEND ? 1u : 0u;
+        if (mode != IDLE) {
+            r = ray_setup(ro, rd);
+            trav_init(t, rt);
+        }
         while (true) {
             const uint64_t tracing = __ballot(mode == SHADOW || mode == EXTEND);
             const uint64_t waiting = __ballot(mode == SWITCH);
@@ -1245,7 +1315,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) v
             if (tracing == 0 || __popcll(waiting) >= XT_WALK_SWITCH) {
                 if (mode == SWITCH) {
                     r = ray_setup(eo, ed);
-                    trav_init(t, INFINITY);   // extension rays: tMax = Infinity (PathTracer.h:167)
+                    trav_init(t, INFINITY);
                     mode = EXTEND;
                     ++n_ext;
                 }
@@ -1259,17 +1329,17 @@ __global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) v
                 done = trav_step_mixed<TRACE_LDS_DEPTH>(active, mode == SHADOW, *a.scene, r, t, top, my_lds, TRACE_BLOCK,
                                                         my_ovf, nthreads, &occ);
             if (active && done) {
-                if (mode == EXTEND) {
-                    mode = IDLE;
-                } else {
-                    if (occ) c = splat(0.0f);
-                    mode = has_ext ? SWITCH : IDLE;
-                    if (!has_ext) {
-                        if (!occ) rad += c;
-                        a.radiance[id] = f4(rad, 0.0f);
-                        alive = false;
-                    }
-                }
+                if (mode == SHADOW) occluded = occ;
+                mode = mode == SHADOW && has_ext && alive ? SWITCH : IDLE;
+            }
+        }
+        if (pair) occluded = (wave_ballot(occluded) >> (lane & 31u) >> 32) & 1ull;
+        if (alive && has_sh) {
+            if (occluded) c = splat(0.0f);
+            if (!has_ext) {
+                if (!occluded) rad += c;
+                a.radiance[id] = f4(rad, 0.0f);
+                alive = false;
             }
         }
         if (alive) {
@@ -1280,7 +1350,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) v
             in.pdf_prev = pdf;
             in.pe_prev = pe;
             in.v = v;
-            in.qflags = has_pend ? QF_PENDING : 0u;
+            in.qflags = QF_PENDING;   // c is zero without a light sample
             in.id = id;
             in.h = t.best_slot != INVALID
                        ? make_float4(t.best_t, __uint_as_float(t.best_slot), t.b0, t.b1)
@@ -1297,7 +1367,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) v
                 shade_vertex<false, NMAP>(wp0, *a.scene, c0, in, gr, 0, cmap, put, o);
             }
             has_ext = o.push_ext;
-            has_pend = o.push_ext && o.push_sh;
+            has_sh = o.push_sh;
             eo = o.ext_o;
             ed = o.ext_d;
             weight = o.ext_w;
@@ -1306,14 +1376,10 @@ __global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) v
             pe = o.ext_pe;
             v = o.ext_v;
             c = o.sh_c;
-            if (o.push_sh) {
-                r = ray_setup(o.sh_o, o.sh_d);
-                trav_init(t, o.sh_tmax);
-                mode = SHADOW;
-                ++n_sh;
-            } else if (o.push_ext) {
-                mode = SWITCH;
-            } else {
+            so = o.sh_o;
+            sd = o.sh_d;
+            stmax = o.sh_tmax;
+            if (!has_ext && !has_sh) {
                 a.radiance[id] = f4(rad, 0.0f);
                 alive = false;
             }

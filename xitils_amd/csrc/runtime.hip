@@ -738,7 +738,8 @@ static uint32_t trace_blocks(const xt_scene* s, size_t n) {
 
 // Paths a wave of k_walk follows at a time, of n in all.
 static uint32_t walk_lanes(uint64_t n) {
-    return (uint32_t)std::min<uint64_t>(64, std::max<uint64_t>(1, (n + WALK_SPREAD - 1) / WALK_SPREAD));
+    const uint64_t lanes = std::max<uint64_t>(1, (n + WALK_SPREAD - 1) / WALK_SPREAD);
+    return (uint32_t)std::min<uint64_t>(lanes, n <= WALK_PAIRS ? 32 : 64);
 }
 // Its blocks: as many as have paths, no more than are resident at once.
 static uint32_t walk_blocks(const xt_scene* s, uint64_t n, uint32_t lanes, bool nmap, uint32_t most) {
