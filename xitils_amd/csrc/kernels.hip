@@ -177,9 +177,9 @@ __global__ __launch_bounds__(TRACE_BLOCK, DYN && MULTI ? 7 : 8) void k_trace(Dev
         bool occ = false;
         bool done;
         if constexpr (MULTI)
-            done = trav_step<ANY, LDS_DEPTH, COUNT>(active, view, r, t, top, my_lds, TRACE_BLOCK, my_ovf, nthreads, vc, &occ);
+            done = trav_step<ANY, LDS_DEPTH, COUNT, DYN>(active, view, r, t, top, my_lds, TRACE_BLOCK, my_ovf, nthreads, vc, &occ);
         else
-            done = trav_step<ANY, LDS_DEPTH, COUNT>(active, sc, r, t, top, my_lds, TRACE_BLOCK, my_ovf, nthreads, vc, &occ);
+            done = trav_step<ANY, LDS_DEPTH, COUNT, DYN>(active, sc, r, t, top, my_lds, TRACE_BLOCK, my_ovf, nthreads, vc, &occ);
         if (active) {
             if (done) {
                 if (ANY) {
@@ -790,7 +790,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, 8) void k_shadow(DevScene sc, ShadowQu
         }
         const bool active = rid != INVALID;
         bool occ = false;
-        const bool done = trav_step<true, TRACE_LDS_DEPTH, COUNT>(active, sc, r, t, top, my_lds, TRACE_BLOCK, my_ovf,
+        const bool done = trav_step<true, TRACE_LDS_DEPTH, COUNT, DYN>(active, sc, r, t, top, my_lds, TRACE_BLOCK, my_ovf,
                                                                    nthreads, vc, &occ);
         if (active) {
             if (done) {
@@ -1068,7 +1068,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, 8) void k_shadow_multi(ShadowQueue sq,
         }
         const bool active = rid != INVALID;
         bool occ = false;
-        const bool done = trav_step<true, TRACE_LDS_DEPTH, false>(active, view, r, t, nullptr, my_lds, TRACE_BLOCK,
+        const bool done = trav_step<true, TRACE_LDS_DEPTH, false, DYN>(active, view, r, t, nullptr, my_lds, TRACE_BLOCK,
                                                                    my_ovf, nthreads, vc, &occ);
         if (active) {
             if (done) {

@@ -506,10 +506,17 @@ __device__ __forceinline__ bool trav_pop(Trav& t, const uint32_t* lds, int lds_s
 // the lanes that reach leaves share the triangle code with those already in
 // leaves.  The visits and their order per ray do not change (identical hits
 // and fetch counts), only how they are grouped into wave iterations.
+// TWICE: while at least half of the wave's lanes are at inner nodes after the
+// first visit, they make a second one before the leaves are tested, so the
+// triangle code, which few lanes need at a time, runs less often.  The chunked
+// launches take it (1080p field, 64 samples: 61.3 -> 59.5 ms a frame); a third
+// visit cost 1% there.  In the launches of even shares, which end with their
+// slowest rays, the second visit only lengthens those: 1..2% slower on the
+// room batch, the Cornell box and ray queries, so they test leaves every time.
 #ifndef XT_TRAV_FUSED
 #define XT_TRAV_FUSED 1
 #endif
-template <bool ANY, int LDS_DEPTH, bool COUNT, class SV>
+template <bool ANY, int LDS_DEPTH, bool COUNT, bool TWICE, class SV>
 __device__ __forceinline__ bool trav_step(bool active, const SV& sc, const RayPre& r, Trav& t, const float4* top,
                                           uint32_t* lds, int lds_stride, uint32_t* ovf, size_t ovf_stride,
                                           VisitCount& vc, bool* occ) {
@@ -519,6 +526,13 @@ __device__ __forceinline__ bool trav_step(bool active, const SV& sc, const RayPr
         if (!visit_node<ANY, LDS_DEPTH, COUNT>(sc, r, t, top, lds, lds_stride, ovf, ovf_stride, vc) &&
             !trav_pop<LDS_DEPTH>(t, lds, lds_stride, ovf, ovf_stride))
             done = true;
+    }
+    if (TWICE && wave_count(wave_ballot(active && !done && t.node >= 0)) >= 32u) {
+        if (active && !done && t.node >= 0) {
+            if (!visit_node<ANY, LDS_DEPTH, COUNT>(sc, r, t, top, lds, lds_stride, ovf, ovf_stride, vc) &&
+                !trav_pop<LDS_DEPTH>(t, lds, lds_stride, ovf, ovf_stride))
+                done = true;
+        }
     }
     if (active && !done && t.node < 0) {
         const int rest = visit_tri<COUNT>(sc, r, t, t.node, vc, ANY, occ);
