@@ -96,6 +96,14 @@ def pmc_from_profiles(name):
     return out
 
 
+def traversal_bytes(cst, node_bytes):
+    """Algorithmic bytes of a step's extension and shadow rays, which one launch
+    per round traces together: ray records, node and triangle fetches."""
+    return (cst["extension_rays"] * EXT_RAY_IO_BYTES + cst["shadow_rays"] * SHADOW_RAY_IO_BYTES +
+            (cst["ext_node_fetches"] + cst["shadow_node_fetches"]) * node_bytes +
+            (cst["ext_tri_fetches"] + cst["shadow_tri_fetches"]) * TRI_BYTES)
+
+
 def traffic_from_profiles(kernel_tag, name=None):
     """HBM bytes per launch (rocprofv3 --pmc FETCH_SIZE + WRITE_SIZE, scaled by
     the copy-kernel calibration) from the committed summary, or None."""
@@ -364,9 +372,8 @@ def cornell_main(args):
     torch.cuda.synchronize()
     wall = time.perf_counter() - t0
     paths = W * H * spp * steps
-    n_ext = cst["extension_rays"]
     node_bytes = info["bytes_nodes"] // max(1, info["bvh_nodes"])
-    bytes_ext = n_ext * EXT_RAY_IO_BYTES + cst["ext_node_fetches"] * node_bytes + cst["ext_tri_fetches"] * TRI_BYTES
+    bytes_trav = traversal_bytes(cst, node_bytes)
     launches = agg["extend_launches"] / steps
     out = {
         "metric": "Mpaths/s (Cornell box 256x256, 16 spp)",
@@ -386,8 +393,8 @@ def cornell_main(args):
                    "parallelism": "1 GPU"},
         "mrays_per_s": round((agg["extension_rays"] + agg["shadow_rays"]) / wall / 1e6, 2),
         "stage_ms_per_step": {k: round(agg[k] / steps, 3) for k in ("ms_extend", "ms_shade", "ms_shadow", "ms_other")},
-        "roofline": kernel_roofline("k_trace<closest> (extend)", bytes_ext / launches,
-                                    agg["ms_extend"] / max(1, agg["extend_launches"]), {},
+        "roofline": kernel_roofline("k_trace + k_trace_shadow (extension and shadow rays)", bytes_trav / launches,
+                                    (agg["ms_extend"] + agg["ms_shadow"]) / max(1, agg["extend_launches"]), {},
                                     {"note": "36 triangles: the tree and triangles sit in L1/LDS-sized caches; "
                                              "launch and latency bound, Mrays/s is the figure of merit"}),
     }
@@ -924,19 +931,19 @@ def main():
     paths = W * H * spp * args.steps
     mpaths = paths / wall / 1e6
     rays = agg["extension_rays"] + agg["shadow_rays"]
-    # roofline of the closest-hit traversal (dominant kernel)
-    n_ext = cst["extension_rays"]
+    # roofline of the traversal (dominant kernels)
+    n_rays = cst["extension_rays"] + cst["shadow_rays"]
     node_bytes = info["bytes_nodes"] // max(1, info["bvh_nodes"])
-    bytes_ext = n_ext * EXT_RAY_IO_BYTES + cst["ext_node_fetches"] * node_bytes + cst["ext_tri_fetches"] * TRI_BYTES
-    per_step_ext_bytes = bytes_ext
+    bytes_trav = traversal_bytes(cst, node_bytes)
     launches = agg["extend_launches"] / args.steps
-    pmc = pmc_from_profiles("extend_heightfield1080p_pmc.txt") if (args.cells, W, H, spp) == (1024, 1920, 1080, 64) \
+    pmc = pmc_from_profiles("traverse_heightfield1080p_pmc.txt") if (args.cells, W, H, spp) == (1024, 1920, 1080, 64) \
         else {}
     roofline = kernel_roofline(
-        "k_trace<closest> (extend)", per_step_ext_bytes / launches, agg["ms_extend"] / agg["extend_launches"], pmc,
-        {"per_ray": {"node_fetches": round(cst["ext_node_fetches"] / n_ext, 3),
-                     "tri_fetches": round(cst["ext_tri_fetches"] / n_ext, 3),
-                     "bytes": round(bytes_ext / n_ext, 1)}})
+        "k_trace + k_trace_shadow (extension and shadow rays)", bytes_trav / launches,
+        (agg["ms_extend"] + agg["ms_shadow"]) / agg["extend_launches"], pmc,
+        {"per_ray": {"node_fetches": round((cst["ext_node_fetches"] + cst["shadow_node_fetches"]) / n_rays, 3),
+                     "tri_fetches": round((cst["ext_tri_fetches"] + cst["shadow_tri_fetches"]) / n_rays, 3),
+                     "bytes": round(bytes_trav / n_rays, 1)}})
     out = {
         "metric": "Mpaths/s at 1080p",
         "value": round(mpaths, 3),

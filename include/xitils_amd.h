@@ -175,7 +175,10 @@ typedef struct xt_render_params {
 /* Counters of the last xt_render, xt_trace_closest or xt_trace_any on a
  * scene.  A launch that follows paths to their ends (small renders, the last
  * rounds of large ones; not while fetches are counted) counts as one extend
- * launch and its time as ms_extend.  After a ray query only its fields are set: extension_rays (closest)
+ * launch and its time as ms_extend.  So does the time of a launch that traces a
+ * round's extension rays and the shadow rays of the round before it (not while
+ * fetches are counted or a network is trained); ms_shadow is the time of shadow rays
+ * traced alone.  After a ray query only its fields are set: extension_rays (closest)
  * or shadow_rays (any) = n, ms_extend or ms_shadow = ms_total = the traversal
  * kernel's time, and with counting on its node and triangle fetches. */
 typedef struct xt_render_stats {

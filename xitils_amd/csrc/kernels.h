@@ -189,6 +189,10 @@ __global__ void k_trace(DevScene sc, const float4* ray_o, const float4* ray_d, i
 template <bool DYN>
 __global__ void k_shadow_multi(ShadowQueue sq, const uint32_t* count, float4* radiance, float4* pending, uint32_t* ovf,
                                uint32_t* dyn, const uint32_t* item_of, const MultiItem* items);
+template <bool MULTI, bool DYN>
+__global__ void k_trace_shadow(DevScene sc, const float4* ray_o, const float4* ray_d, float4* hits, ShadowQueue sq,
+                               uint32_t* counts, int cur, float4* radiance, float4* pending, uint32_t* ovf, uint32_t* dyn,
+                               uint32_t* counts_out, const uint32_t* item_of = nullptr, const MultiItem* items = nullptr);
 __global__ void k_window_init(MultiBatch mb);
 __global__ void k_window_plan(MultiBatch mb);
 __global__ void k_window_advance(MultiBatch mb);

@@ -99,6 +99,60 @@ __device__ __forceinline__ void flush_counts(unsigned long long* totals, const V
     }
 }
 
+// The loop of the traversal kernels: the rays of `ch` (and, DYN, of the cursor
+// `dyn`) by persistent waves with in-place lane refill.  load(i) sets up ray i
+// in r and t, finish(i, occluded) takes its result out of t.
+template <bool ANY, int LDS_DEPTH, bool COUNT, bool DYN, class SV, class Load, class Finish>
+__device__ __forceinline__ void trace_queue(RayChunks ch, uint32_t* dyn, const SV& sv, const RayPre& r, Trav& t,
+                                            const float4* top, uint32_t* my_lds, uint32_t* my_ovf, size_t nthreads,
+                                            VisitCount& vc, Load load, Finish finish) {
+    const uint64_t below = (1ull << __lane_id()) - 1ull;
+    uint32_t rid = INVALID;   // the lane's ray; INVALID: none
+    while (true) {
+        const uint64_t busy = wave_ballot(rid != INVALID);
+        const uint32_t nidle = 64u - wave_count(busy);
+        if (nidle >= (uint32_t)REFILL_IDLE) {
+            if (DYN && ch.next >= ch.end && !ch.exhausted) chunks_refill(ch, dyn);
+            if (ch.next < ch.end) {
+                const uint32_t my = ch.next + (uint32_t)__popcll(~busy & below);
+                if (rid == INVALID && my < ch.end) {
+                    rid = my;
+                    load(rid);
+                }
+                ch.next = min(ch.next + nidle, ch.end);
+            } else if (busy == 0) {
+                break;
+            }
+        }
+        const bool active = rid != INVALID;
+        bool occ = false;
+        const bool done = trav_step<ANY, LDS_DEPTH, COUNT, DYN>(active, sv, r, t, top, my_lds, TRACE_BLOCK, my_ovf, nthreads, vc, &occ);
+        if (active && done) {
+            finish(rid, occ);
+            rid = INVALID;
+        }
+    }
+}
+
+// A closest-hit ray's entry of the hit queue.
+__device__ __forceinline__ float4 hit_record(const Trav& t, uint32_t id) {
+    return t.best_slot != INVALID ? make_float4(t.best_t, __uint_as_float(id), t.b0, t.b1)
+                                  : make_float4(INFINITY, __uint_as_float(INVALID), 0.0f, 0.0f);
+}
+
+// What a shadow ray adds: unoccluded contributions go straight to the path
+// radiance, or to pending[] when the path continues (see k_shade).
+__device__ __forceinline__ void shadow_record(const ShadowQueue& sq, uint32_t i, bool occ, float4* radiance, float4* pending) {
+    const float4 c4 = sq.c[i];
+    const uint32_t id = __float_as_uint(sq.d[i].w);
+    const f3 c = occ ? splat(0.0f) : xyz(c4);
+    if (c4.w != 0.0f) {
+        pending[id] = f4(c, 0.0f);
+    } else if (!occ) {
+        radiance[id] = f4(xyz(radiance[id]) + c, 0.0f);
+    }
+}
+
 // Ray queries over a ray array (stride in float4 between rays): closest hit
 // (ANY = false) -> hits[i] = (t, slot or prim id, b0, b1); any hit ->
 // occluded[i].  Persistent waves with in-place lane refill (xt_traverse.h).
@@ -143,58 +197,26 @@ __global__ __launch_bounds__(TRACE_BLOCK, DYN && MULTI ? 7 : 8) void k_trace(Dev
     uint32_t* my_ovf = ovf ? ovf + gtid : nullptr;
     const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(gtid / 64));
     RayChunks ch = chunks_first<DYN>(wave, nwaves, n);
-    const uint64_t below = (1ull << __lane_id()) - 1ull;
     VisitCount vc;
-    uint32_t rid = INVALID;   // the lane's ray; INVALID: none
     RayPre r;
     Trav t;
     TravView view{sc.nodes, sc.tris, MULTI ? 0u : sc.top_nodes};
-    while (true) {
-        const uint64_t busy = wave_ballot(rid != INVALID);
-        const uint32_t nidle = 64u - wave_count(busy);
-        if (nidle >= (uint32_t)REFILL_IDLE) {
-            if (DYN && ch.next >= ch.end && !ch.exhausted) chunks_refill(ch, dyn);
-            if (ch.next < ch.end) {
-                const uint32_t my = ch.next + (uint32_t)__popcll(~busy & below);
-                if (rid == INVALID && my < ch.end) {
-                    rid = my;
-                    float4 o4 = ray_o[(size_t)rid * ray_stride];
-                    float4 d4 = ray_d[(size_t)rid * ray_stride];
-                    if constexpr (MULTI) {
-                        const MultiItem& it = items[item_of[__float_as_uint(d4.w)]];
-                        view.nodes = it.nodes;
-                        view.tris = it.tris;
-                    }
-                    r = ray_setup(xyz(o4), xyz(d4));
-                    trav_init(t, tmax_from_ray ? o4.w : INFINITY);   // extension rays: tMax = Infinity (PathTracer.h:167)
-                }
-                ch.next = min(ch.next + nidle, ch.end);
-            } else if (busy == 0) {
-                break;
-            }
+    auto load = [&](uint32_t i) {
+        const float4 o4 = ray_o[(size_t)i * ray_stride], d4 = ray_d[(size_t)i * ray_stride];
+        if constexpr (MULTI) {
+            const MultiItem& it = items[item_of[__float_as_uint(d4.w)]];
+            view.nodes = it.nodes;
+            view.tris = it.tris;
         }
-        const bool active = rid != INVALID;
-        bool occ = false;
-        bool done;
-        if constexpr (MULTI)
-            done = trav_step<ANY, LDS_DEPTH, COUNT, DYN>(active, view, r, t, top, my_lds, TRACE_BLOCK, my_ovf, nthreads, vc, &occ);
-        else
-            done = trav_step<ANY, LDS_DEPTH, COUNT, DYN>(active, sc, r, t, top, my_lds, TRACE_BLOCK, my_ovf, nthreads, vc, &occ);
-        if (active) {
-            if (done) {
-                if (ANY) {
-                    occluded[rid] = occ ? 1 : 0;
-                } else {
-                    hits[rid] = t.best_slot != INVALID
-                                    ? make_float4(t.best_t, __uint_as_float(hit_prim_ids ? prim_of_slot(view, t.best_slot)
-                                                                                            : t.best_slot),
-                                                  t.b0, t.b1)
-                                    : make_float4(INFINITY, __uint_as_float(INVALID), 0.0f, 0.0f);
-                }
-                rid = INVALID;
-            }
-        }
-    }
+        r = ray_setup(xyz(o4), xyz(d4));
+        trav_init(t, tmax_from_ray ? o4.w : INFINITY);   // extension rays: tMax = Infinity (PathTracer.h:167)
+    };
+    auto finish = [&](uint32_t i, bool occ) {
+        if (ANY) occluded[i] = occ ? 1 : 0;
+        else hits[i] = hit_record(t, hit_prim_ids && t.best_slot != INVALID ? prim_of_slot(view, t.best_slot) : t.best_slot);
+    };
+    if constexpr (MULTI) trace_queue<ANY, LDS_DEPTH, COUNT, DYN>(ch, dyn, view, r, t, top, my_lds, my_ovf, nthreads, vc, load, finish);
+    else trace_queue<ANY, LDS_DEPTH, COUNT, DYN>(ch, dyn, sc, r, t, top, my_lds, my_ovf, nthreads, vc, load, finish);
     if constexpr (DYN) chunks_release(dyn);
     if (COUNT) flush_counts(visit_totals, vc);
 }
@@ -765,49 +787,17 @@ __global__ __launch_bounds__(TRACE_BLOCK, 8) void k_shadow(DevScene sc, ShadowQu
     uint32_t* my_ovf = ovf ? ovf + gtid : nullptr;
     const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(gtid / 64));
     RayChunks ch = chunks_first<DYN>(wave, nwaves, n);
-    const uint64_t below = (1ull << __lane_id()) - 1ull;
     VisitCount vc;
-    uint32_t rid = INVALID;   // the lane's ray; INVALID: none
     RayPre r;
     Trav t;
-    while (true) {
-        const uint64_t busy = wave_ballot(rid != INVALID);
-        const uint32_t nidle = 64u - wave_count(busy);
-        if (nidle >= (uint32_t)REFILL_IDLE) {
-            if (DYN && ch.next >= ch.end && !ch.exhausted) chunks_refill(ch, dyn);
-            if (ch.next < ch.end) {
-                const uint32_t my = ch.next + (uint32_t)__popcll(~busy & below);
-                if (rid == INVALID && my < ch.end) {
-                    rid = my;
-                    float4 o4 = sq.o[rid], d4 = sq.d[rid];
-                    r = ray_setup(xyz(o4), xyz(d4));
-                    trav_init(t, o4.w);
-                }
-                ch.next = min(ch.next + nidle, ch.end);
-            } else if (busy == 0) {
-                break;
-            }
-        }
-        const bool active = rid != INVALID;
-        bool occ = false;
-        const bool done = trav_step<true, TRACE_LDS_DEPTH, COUNT, DYN>(active, sc, r, t, top, my_lds, TRACE_BLOCK, my_ovf,
-                                                                   nthreads, vc, &occ);
-        if (active) {
-            if (done) {
-                // unoccluded contributions go straight to the path radiance, or to
-                // pending[] when the path continues (see k_shade)
-                float4 c4 = sq.c[rid];
-                uint32_t id = __float_as_uint(sq.d[rid].w);
-                f3 c = occ ? splat(0.0f) : xyz(c4);
-                if (c4.w != 0.0f) {
-                    pending[id] = f4(c, 0.0f);
-                } else if (!occ) {
-                    radiance[id] = f4(xyz(radiance[id]) + c, 0.0f);
-                }
-                rid = INVALID;
-            }
-        }
-    }
+    trace_queue<true, TRACE_LDS_DEPTH, COUNT, DYN>(
+        ch, dyn, sc, r, t, top, my_lds, my_ovf, nthreads, vc,
+        [&](uint32_t i) {
+            const float4 o4 = sq.o[i];
+            r = ray_setup(xyz(o4), xyz(sq.d[i]));
+            trav_init(t, o4.w);
+        },
+        [&](uint32_t i, bool occ) { shadow_record(sq, i, occ, radiance, pending); });
     if constexpr (DYN) chunks_release(dyn);
     if (COUNT) flush_counts(visit_totals, vc);
 }
@@ -1038,57 +1028,127 @@ __global__ __launch_bounds__(TRACE_BLOCK, 8) void k_shadow_multi(ShadowQueue sq,
     uint32_t* my_ovf = ovf ? ovf + gtid : nullptr;
     const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(gtid / 64));
     RayChunks ch = chunks_first<DYN>(wave, nwaves, n);
-    const uint64_t below = (1ull << __lane_id()) - 1ull;
     VisitCount vc;
-    uint32_t rid = INVALID, id = 0;   // the lane's ray (INVALID: none) and its path
     RayPre r;
     Trav t;
     TravView view{nullptr, nullptr, 0u};
-    while (true) {
-        const uint64_t busy = wave_ballot(rid != INVALID);
-        const uint32_t nidle = 64u - wave_count(busy);
-        if (nidle >= (uint32_t)REFILL_IDLE) {
-            if (DYN && ch.next >= ch.end && !ch.exhausted) chunks_refill(ch, dyn);
-            if (ch.next < ch.end) {
-                const uint32_t my = ch.next + (uint32_t)__popcll(~busy & below);
-                if (rid == INVALID && my < ch.end) {
-                    rid = my;
-                    float4 o4 = sq.o[rid], d4 = sq.d[rid];
-                    id = __float_as_uint(d4.w);
-                    const MultiItem& it = items[item_of[id]];
-                    view.nodes = it.nodes;
-                    view.tris = it.tris;
-                    r = ray_setup(xyz(o4), xyz(d4));
-                    trav_init(t, o4.w);
-                }
-                ch.next = min(ch.next + nidle, ch.end);
-            } else if (busy == 0) {
-                break;
-            }
-        }
-        const bool active = rid != INVALID;
-        bool occ = false;
-        const bool done = trav_step<true, TRACE_LDS_DEPTH, false, DYN>(active, view, r, t, nullptr, my_lds, TRACE_BLOCK,
-                                                                   my_ovf, nthreads, vc, &occ);
-        if (active) {
-            if (done) {
-                const float4 c4 = sq.c[rid];
-                const f3 c = occ ? splat(0.0f) : xyz(c4);
-                if (c4.w != 0.0f) {
-                    pending[id] = f4(c, 0.0f);
-                } else if (!occ) {
-                    radiance[id] = f4(xyz(radiance[id]) + c, 0.0f);
-                }
-                rid = INVALID;
-            }
-        }
-    }
+    trace_queue<true, TRACE_LDS_DEPTH, false, DYN>(
+        ch, dyn, view, r, t, nullptr, my_lds, my_ovf, nthreads, vc,
+        [&](uint32_t i) {
+            const float4 o4 = sq.o[i], d4 = sq.d[i];
+            const MultiItem& it = items[item_of[__float_as_uint(d4.w)]];
+            view.nodes = it.nodes;
+            view.tris = it.tris;
+            r = ray_setup(xyz(o4), xyz(d4));
+            trav_init(t, o4.w);
+        },
+        [&](uint32_t i, bool occ) { shadow_record(sq, i, occ, radiance, pending); });
     if constexpr (DYN) chunks_release(dyn);
 }
 template __global__ void k_shadow_multi<false>(ShadowQueue, const uint32_t*, float4*, float4*, uint32_t*, uint32_t*,
                                                const uint32_t*, const MultiItem*);
 template __global__ void k_shadow_multi<true>(ShadowQueue, const uint32_t*, float4*, float4*, uint32_t*, uint32_t*,
                                               const uint32_t*, const MultiItem*);
+
+// A round's extension rays and the shadow rays of the round before, which do
+// not depend on each other, in one launch: a launch lasts as long as its slowest
+// rays, so below some millions of paths two launches end with two stretches of
+// a nearly idle chip, and below half a million one queue does not fill it at
+// all.  16 rooms at 128 x 128 in one batch 3.80 -> 2.80 ms, Cornell box at 1 M
+// paths 1511 -> 1247 us, 100 k triangle room at 3.7 M 12.33 -> 10.88 ms (guided
+// 9.17 -> 7.68), normal-mapped plane 8.30 -> 7.96, 1080p field at 132 M 58.9 ->
+// 58.3.  A path's contributions are added in the same order: its shadow ray
+// still ends before its next vertex is shaded.
+// DYN: a wave takes chunks of extension rays while there are any, then of
+// shadow rays.  Otherwise the two queues are one row of rays with an even
+// share per wave, and only the wave at the seam traces both kinds.
+template <bool MULTI, bool DYN>
+__global__ __launch_bounds__(TRACE_BLOCK, DYN && MULTI ? 7 : 8) void k_trace_shadow(
+    DevScene sc, const float4* __restrict__ ray_o, const float4* __restrict__ ray_d, float4* __restrict__ hits, ShadowQueue sq,
+    uint32_t* __restrict__ counts, int cur, float4* __restrict__ radiance, float4* __restrict__ pending,
+    uint32_t* __restrict__ ovf, uint32_t* __restrict__ dyn, uint32_t* __restrict__ counts_out,
+    const uint32_t* __restrict__ item_of, const MultiItem* __restrict__ items) {
+    __shared__ uint32_t lds[TRACE_LDS_DEPTH * TRACE_BLOCK];
+    const uint32_t np = *path_count(counts, cur), ns = *shadow_count(counts, cur);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        // the lengths to the host's pinned ring, and the next round's queues
+        // (last read by the previous round) emptied
+        if (counts_out) {
+            *path_count(counts_out, cur) = np;
+            *shadow_count(counts_out, cur) = ns;
+        }
+        *pair_count(counts, 1 - cur) = 0ull;
+    }
+    __shared__ float4 top[MULTI ? 1 : TOP_F4];
+    if constexpr (!MULTI) stage_top_nodes(top, sc);
+    const size_t nthreads = (size_t)gridDim.x * blockDim.x;
+    const size_t gtid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t* my_lds = lds + threadIdx.x;
+    uint32_t* my_ovf = ovf ? ovf + gtid : nullptr;
+    const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(gtid / 64));
+    RayChunks ext, sha;
+    if constexpr (DYN) {
+        ext = chunks_first<true>(wave, nwaves, np);
+        sha = chunks_queued(nwaves, ns);
+    } else {
+        chunks_joint(wave, nwaves, np, ns, &ext, &sha);
+    }
+    VisitCount vc;
+    auto scene_of = [&](uint32_t id, TravView& view) {
+        if constexpr (MULTI) {
+            const MultiItem& it = items[item_of[id]];
+            view.nodes = it.nodes;
+            view.tris = it.tris;
+        }
+    };
+    auto trace = [&](const auto& sv, TravView& view) {
+        RayPre r;
+        Trav t;
+        trace_queue<false, TRACE_LDS_DEPTH, false, DYN>(
+            ext, dyn, sv, r, t, MULTI ? nullptr : top, my_lds, my_ovf, nthreads, vc,
+            [&](uint32_t i) {
+                const float4 d4 = ray_d[i];
+                scene_of(__float_as_uint(d4.w), view);
+                r = ray_setup(xyz(ray_o[i]), xyz(d4));
+                trav_init(t, INFINITY);   // tMax = Infinity (PathTracer.h:167)
+            },
+            [&](uint32_t i, bool) { hits[i] = hit_record(t, t.best_slot); });
+    };
+    auto trace_shadow = [&](const auto& sv, TravView& view) {
+        RayPre r;
+        Trav t;
+        trace_queue<true, TRACE_LDS_DEPTH, false, DYN>(
+            sha, dyn + 2, sv, r, t, MULTI ? nullptr : top, my_lds, my_ovf, nthreads, vc,
+            [&](uint32_t i) {
+                const float4 o4 = sq.o[i], d4 = sq.d[i];
+                scene_of(__float_as_uint(d4.w), view);
+                r = ray_setup(xyz(o4), xyz(d4));
+                trav_init(t, o4.w);
+            },
+            [&](uint32_t i, bool occ) { shadow_record(sq, i, occ, radiance, pending); });
+    };
+    TravView view{nullptr, nullptr, 0u}, shadow_view{nullptr, nullptr, 0u};
+    if constexpr (MULTI) {
+        trace(view, view);
+        trace_shadow(shadow_view, shadow_view);
+    } else {
+        trace(sc, view);
+        trace_shadow(sc, shadow_view);
+    }
+    if constexpr (DYN) {
+        chunks_release(dyn);
+        chunks_release(dyn + 2);
+    }
+}
+#define XT_INST_TRACE_SHADOW(MULTI, DYN)                                                                              \
+    template __global__ void k_trace_shadow<MULTI, DYN>(DevScene, const float4*, const float4*, float4*, ShadowQueue,  \
+                                                        uint32_t*, int, float4*, float4*, uint32_t*, uint32_t*,        \
+                                                        uint32_t*, const uint32_t*, const MultiItem*);
+XT_INST_TRACE_SHADOW(false, false)
+XT_INST_TRACE_SHADOW(false, true)
+XT_INST_TRACE_SHADOW(true, false)
+XT_INST_TRACE_SHADOW(true, true)
+#undef XT_INST_TRACE_SHADOW
 
 // film[pixel] += the window's samples of that pixel, in sample order, for
 // every item the window overlaps (one thread per item pixel).

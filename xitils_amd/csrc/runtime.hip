@@ -1322,6 +1322,24 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
             uint32_t rec_base = 0;
             bool launch = !whole;
             queue_len[0] = wp.num_paths;
+            // A round's shadow rays go with the next round's extension rays,
+            // except where each round's counts are read before the next and
+            // where the two kinds' fetches are counted.
+            const bool joint = !train && !s->counting;
+            // shadow rays of round `rd` alone; counts -> pinned ring
+            auto shadow_round = [&](int rd, int filled) {
+                const int slot = rd % RB_RING;
+                const bool dyn = bound >= TRAV_DYN_MIN;
+                auto shadow = s->counting ? (dyn ? k_shadow<true, true> : k_shadow<true, false>)
+                                          : (dyn ? k_shadow<false, true> : k_shadow<false, false>);
+                hipEvent_t b = tm.mark();
+                hipLaunchKernelGGL(shadow, dim3(trace_blocks(s, bound)), dim3(TRACE_BLOCK), 0, s->stream, s->ds, rb.sq,
+                                   shadow_count(rb.counts, filled), rb.radiance, rb.pending, s->d_ovf, rb.dyn + 2,
+                                   s->counting ? rb.visits + 2 : nullptr, rb.counts, rb.host_counts_dev + 4 * slot);
+                XT_LAUNCHED(result);
+                tm.add(2, b, tm.mark());
+                if (hipEventRecord(rb.round_ev[slot], s->stream) != hipSuccess) result = fail(XT_ERR_DEVICE, "hipEventRecord failed");
+            };
             // a path adds one extension ray per round, so max_depth + 1 rounds hold every live queue
             const int max_rounds = p->max_depth > 0 ? p->max_depth + 2 + lag : (1 << 16);
             // Once a read count is zero every later round is empty: the host
@@ -1332,19 +1350,31 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                     break;
                 }
                 {
-                    const int slot = round % RB_RING;
                     a = tm.mark();
                     // large queues: rays handed out in chunks from a cursor (the
                     // round's shadow queue is no longer than its path queue)
                     const bool dyn = bound >= TRAV_DYN_MIN;
-                    auto trace = s->counting ? (dyn ? k_trace<false, TRACE_LDS_DEPTH, true, false, true>
-                                                    : k_trace<false, TRACE_LDS_DEPTH, true, false, false>)
-                                             : (dyn ? k_trace<false, TRACE_LDS_DEPTH, false, false, true>
-                                                    : k_trace<false, TRACE_LDS_DEPTH, false, false, false>);
-                    hipLaunchKernelGGL(trace, dim3(trace_blocks(s, bound)), dim3(TRACE_BLOCK), 0, s->stream, s->ds,
-                                       rb.q[cur].o, rb.q[cur].d, 1, path_count(rb.counts, cur), 0u, rb.hits, nullptr, 0, 0,
-                                       s->d_ovf, rb.dyn, s->counting ? rb.visits : nullptr,
-                                       path_count(rb.counts, 1 - cur), shadow_count(rb.counts, 1 - cur), nullptr, nullptr);   // also clears the next counters
+                    // both forms also clear the next round's counters
+                    if (joint && round > 0) {
+                        const int slot = (round - 1) % RB_RING;
+                        hipLaunchKernelGGL((dyn ? k_trace_shadow<false, true> : k_trace_shadow<false, false>),
+                                           dim3(trace_blocks(s, 2 * (size_t)bound)), dim3(TRACE_BLOCK), 0, s->stream, s->ds,
+                                           rb.q[cur].o, rb.q[cur].d, rb.hits, rb.sq, rb.counts, cur, rb.radiance, rb.pending,
+                                           s->d_ovf, rb.dyn, rb.host_counts_dev + 4 * slot, nullptr, nullptr);
+                        if (hipEventRecord(rb.round_ev[slot], s->stream) != hipSuccess) {
+                            result = fail(XT_ERR_DEVICE, "hipEventRecord failed");
+                            break;
+                        }
+                    } else {
+                        auto trace = s->counting ? (dyn ? k_trace<false, TRACE_LDS_DEPTH, true, false, true>
+                                                        : k_trace<false, TRACE_LDS_DEPTH, true, false, false>)
+                                                 : (dyn ? k_trace<false, TRACE_LDS_DEPTH, false, false, true>
+                                                        : k_trace<false, TRACE_LDS_DEPTH, false, false, false>);
+                        hipLaunchKernelGGL(trace, dim3(trace_blocks(s, bound)), dim3(TRACE_BLOCK), 0, s->stream, s->ds,
+                                           rb.q[cur].o, rb.q[cur].d, 1, path_count(rb.counts, cur), 0u, rb.hits, nullptr, 0, 0,
+                                           s->d_ovf, rb.dyn, s->counting ? rb.visits : nullptr,
+                                           path_count(rb.counts, 1 - cur), shadow_count(rb.counts, 1 - cur), nullptr, nullptr);
+                    }
                     XT_LAUNCHED(result);
                     tm.add(0, a, tm.mark());
                     GuideRender gr{};
@@ -1376,19 +1406,8 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                                        pair_count(rb.counts, 1 - cur), rb.sq, rb.radiance, rb.pending, gr);
                     XT_LAUNCHED(result);
                     tm.add(1, a, tm.mark());
-                    a = tm.mark();
-                    auto shadow = s->counting ? (dyn ? k_shadow<true, true> : k_shadow<true, false>)
-                                              : (dyn ? k_shadow<false, true> : k_shadow<false, false>);
-                    hipLaunchKernelGGL(shadow, dim3(trace_blocks(s, bound)), dim3(TRACE_BLOCK), 0, s->stream, s->ds,
-                                       rb.sq, shadow_count(rb.counts, 1 - cur), rb.radiance, rb.pending, s->d_ovf, rb.dyn + 2,
-                                       s->counting ? rb.visits + 2 : nullptr, rb.counts,
-                                       rb.host_counts_dev + 4 * slot);   // counts -> pinned ring
-                    XT_LAUNCHED(result);
-                    tm.add(2, a, tm.mark());
-                    if (hipEventRecord(rb.round_ev[slot], s->stream) != hipSuccess) {
-                        result = fail(XT_ERR_DEVICE, "hipEventRecord failed");
-                        break;
-                    }
+                    if (!joint) shadow_round(round, 1 - cur);
+                    if (result != XT_OK) break;
                     ++round;
                     cur = 1 - cur;
                 }
@@ -1421,6 +1440,7 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                 if (launch && can_walk && bound <= WALK_TAIL && result == XT_OK) {
                     // few paths are left: the queue of the next round, whose
                     // length is at most `bound`, in one launch
+                    if (joint) shadow_round(round - 1, cur);
                     walk(cur, bound);
                     while (verified < round)
                         if (!read_round()) break;
@@ -1603,9 +1623,11 @@ struct BounceGuide {
 // max_depth + 1 rounds of extend / (guide) / shade / shadow, accumulate,
 // advance the cursor.  Every kernel reads its queue length from device memory.
 static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const WaveParams& wp, const BounceBufs& b,
-                                 const BatchPlan& plan, BatchCursor* cursor, uint32_t tblocks, uint32_t tmost,
+                                 const BatchPlan& plan, BatchCursor* cursor, uint32_t tmost,
                                  const BounceGuide& gd, void* d_film, int f64) {
     const uint32_t maxpaths = plan.pix_chunk * plan.S;
+    const uint32_t tblocks = std::min(trace_blocks(s, maxpaths), tmost);
+    const uint32_t jblocks = std::min(trace_blocks(s, 2 * (size_t)maxpaths), tmost);   // launches of two queues
     const uint32_t gblocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((maxpaths + 255) / 256, (uint64_t)s->dev->num_cu * 8));
     const uint32_t ablocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((plan.pix_chunk + 255) / 256, (uint64_t)s->dev->num_cu * 8));
     const uint32_t sblocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((maxpaths + SHADE_BLOCK - 1) / SHADE_BLOCK, s->shade_grid));
@@ -1629,9 +1651,14 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
     }
     int cur = 0;
     for (int it = 0; it <= p->max_depth && !whole; ++it) {
-        hipLaunchKernelGGL((k_trace<false, TRACE_LDS_DEPTH, false>), dim3(tblocks), dim3(TRACE_BLOCK), 0, s->stream, s->ds,
-                           b.q[cur].o, b.q[cur].d, 1, path_count(b.counts, cur), 0u, b.hits, nullptr, 0, 0, b.ovf, nullptr, nullptr,
-                           path_count(b.counts, 1 - cur), shadow_count(b.counts, 1 - cur));
+        if (it == 0)
+            hipLaunchKernelGGL((k_trace<false, TRACE_LDS_DEPTH, false>), dim3(tblocks), dim3(TRACE_BLOCK), 0, s->stream, s->ds,
+                               b.q[0].o, b.q[0].d, 1, path_count(b.counts, 0), 0u, b.hits, nullptr, 0, 0, b.ovf, nullptr, nullptr,
+                               path_count(b.counts, 1), shadow_count(b.counts, 1));
+        else
+            hipLaunchKernelGGL((k_trace_shadow<false, false>), dim3(jblocks), dim3(TRACE_BLOCK), 0, s->stream, s->ds, b.q[cur].o,
+                               b.q[cur].d, b.hits, b.sq, b.counts, cur, b.radiance, b.pending, b.ovf, nullptr, nullptr, nullptr,
+                               nullptr);
         GuideRender gr{};
         if (guide) {
             hipLaunchKernelGGL(k_guide_infer, dim3(ib), dim3(GI_BLOCK), 0, s->stream, g.net, g.gb, s->ds, b.q[cur],
@@ -1645,10 +1672,11 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
         hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags), dim3(sblocks), dim3(SHADE_BLOCK), 0, s->stream, wp, s->d_ds,
                            b.q[cur], path_count(b.counts, cur), b.hits, b.q[1 - cur], pair_count(b.counts, 1 - cur), b.sq,
                            b.radiance, b.pending, gr);
-        hipLaunchKernelGGL(k_shadow<false>, dim3(tblocks), dim3(TRACE_BLOCK), 0, s->stream, s->ds, b.sq, shadow_count(b.counts, 1 - cur),
-                           b.radiance, b.pending, b.ovf, nullptr, nullptr, b.counts, nullptr);
         cur = 1 - cur;
     }
+    if (!whole)
+        hipLaunchKernelGGL(k_shadow<false>, dim3(tblocks), dim3(TRACE_BLOCK), 0, s->stream, s->ds, b.sq, shadow_count(b.counts, cur),
+                           b.radiance, b.pending, b.ovf, nullptr, nullptr, b.counts, nullptr);
     hipLaunchKernelGGL(k_accumulate, dim3(ablocks), dim3(256), 0, s->stream, wp, b.radiance, d_film, f64);
     hipLaunchKernelGGL(k_advance_cursor, dim3(1), dim3(1), 0, s->stream, cursor, plan);
 }
@@ -1678,9 +1706,8 @@ static xt_status capture_graph(xt_scene* s, const xt_camera* cam, const xt_rende
         gd.lobes2 = (float2*)(rb.lobes + (size_t)2 * G_LOBES * rb.capacity);
         gd.stride = rb.capacity;
     }
-    const uint32_t tblocks = trace_blocks(s, plan.pix_chunk * plan.S);
     XT_HIP(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_cursor_batch(s, p, wp, b, plan, s->d_cursor, tblocks, s->trace_grid_max, gd, d_film, f64);
+    enqueue_cursor_batch(s, p, wp, b, plan, s->d_cursor, s->trace_grid_max, gd, d_film, f64);
     hipError_t launch_err = hipGetLastError();
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(s->stream, &graph);
@@ -1903,9 +1930,9 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
     xt_scene* s0 = sc_list[0];
     const bool whole = window <= WALK_MAX;   // each path in one launch
     const uint32_t lanes = walk_lanes(window);
-    const uint32_t tblocks = whole ? walk_blocks(s0, window, lanes, nmap, s0->trace_grid_max)
-                                   : std::max(1u, std::min(s0->trace_grid, (window + TRACE_BLOCK - 1) / TRACE_BLOCK));
-    const size_t ovf_need = (size_t)ovf_depth * tblocks * TRACE_BLOCK;
+    const uint32_t tblocks = whole ? walk_blocks(s0, window, lanes, nmap, s0->trace_grid_max) : trace_blocks(s0, window);
+    const uint32_t jblocks = trace_blocks(s0, 2 * (size_t)window);   // launches of two queues
+    const size_t ovf_need = (size_t)ovf_depth * std::max(tblocks, jblocks) * TRACE_BLOCK;
     if (m.ovf_entries < ovf_need) {
         hipStreamSynchronize(m.stream);
         hipFree(m.ovf);
@@ -1966,11 +1993,16 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
     }
     int cur = 0;
     for (int it = 0; it <= max_depth && !whole; ++it) {
-        hipLaunchKernelGGL((dyn ? k_trace<false, TRACE_LDS_DEPTH, false, true, true>
-                                : k_trace<false, TRACE_LDS_DEPTH, false, true, false>),
-                           dim3(tblocks), dim3(TRACE_BLOCK), 0, m.stream, s0->ds, m.q[cur].o, m.q[cur].d, 1,
-                           path_count(m.counts, cur), 0u, m.hits, nullptr, 0, 0, m.ovf, m.dyn, nullptr,
-                           path_count(m.counts, 1 - cur), shadow_count(m.counts, 1 - cur), m.item_of, m.items);
+        if (it == 0)
+            hipLaunchKernelGGL((dyn ? k_trace<false, TRACE_LDS_DEPTH, false, true, true>
+                                    : k_trace<false, TRACE_LDS_DEPTH, false, true, false>),
+                               dim3(tblocks), dim3(TRACE_BLOCK), 0, m.stream, s0->ds, m.q[0].o, m.q[0].d, 1,
+                               path_count(m.counts, 0), 0u, m.hits, nullptr, 0, 0, m.ovf, m.dyn, nullptr,
+                               path_count(m.counts, 1), shadow_count(m.counts, 1), m.item_of, m.items);
+        else
+            hipLaunchKernelGGL((dyn ? k_trace_shadow<true, true> : k_trace_shadow<true, false>), dim3(jblocks), dim3(TRACE_BLOCK),
+                               0, m.stream, s0->ds, m.q[cur].o, m.q[cur].d, m.hits, m.sq, m.counts, cur, m.radiance, m.pending,
+                               m.ovf, m.dyn, nullptr, m.item_of, m.items);
         if (nmap)
             hipLaunchKernelGGL(k_shade_multi<true>, dim3(sblocks), dim3(SHADE_BLOCK), 0, m.stream, mb, m.q[cur],
                                path_count(m.counts, cur), m.hits, m.q[1 - cur], pair_count(m.counts, 1 - cur), m.sq,
@@ -1979,10 +2011,11 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
             hipLaunchKernelGGL(k_shade_multi<false>, dim3(sblocks), dim3(SHADE_BLOCK), 0, m.stream, mb, m.q[cur],
                                path_count(m.counts, cur), m.hits, m.q[1 - cur], pair_count(m.counts, 1 - cur), m.sq,
                                m.radiance, m.pending);
-        hipLaunchKernelGGL((dyn ? k_shadow_multi<true> : k_shadow_multi<false>), dim3(tblocks), dim3(TRACE_BLOCK), 0,
-                           m.stream, m.sq, shadow_count(m.counts, 1 - cur), m.radiance, m.pending, m.ovf, m.dyn + 2, m.item_of, m.items);
         cur = 1 - cur;
     }
+    if (!whole)
+        hipLaunchKernelGGL((dyn ? k_shadow_multi<true> : k_shadow_multi<false>), dim3(tblocks), dim3(TRACE_BLOCK), 0, m.stream,
+                           m.sq, shadow_count(m.counts, cur), m.radiance, m.pending, m.ovf, m.dyn + 2, m.item_of, m.items);
     hipLaunchKernelGGL(k_accumulate_multi, dim3(gblocks), dim3(256), 0, m.stream, mb, m.radiance);
     hipLaunchKernelGGL(k_window_advance, dim3(1), dim3(1), 0, m.stream, mb);
     hipError_t launch_err = hipGetLastError();
@@ -2296,12 +2329,11 @@ xt_status xt_render_static(xt_scene* s, const xt_camera* cam, const xt_render_pa
     uint32_t nbatches = 0;
     const BatchPlan plan = cursor_plan(p, cap, &nbatches);
     const WaveParams wp = cursor_wave_params(cam, p, cursor);
-    const uint32_t tblocks = std::min(trace_blocks(s, (size_t)plan.pix_chunk * plan.S), tcap);
     // the cursor is written by k_cursor_init and the counters by the kernels
     // (k_count_from_cursor, k_trace), so nothing needs clearing beforehand
     hipLaunchKernelGGL(k_cursor_init, dim3(1), dim3(1), 0, s->stream, cursor, plan, b.dyn);
     for (uint32_t k = 0; k < nbatches; ++k)
-        enqueue_cursor_batch(s, p, wp, b, plan, cursor, tblocks, tcap, BounceGuide{}, film, film_f64);
+        enqueue_cursor_batch(s, p, wp, b, plan, cursor, tcap, BounceGuide{}, film, film_f64);
     hipError_t le = hipGetLastError();
     hipError_t se = hipStreamSynchronize(s->stream);
     if (le != hipSuccess) return fail(XT_ERR_DEVICE, std::string("xt_render_static launch failed: ") + hipGetErrorString(le));

@@ -280,6 +280,26 @@ __device__ __forceinline__ RayChunks chunks_first(uint32_t wave, uint32_t nwaves
     c.exhausted = c.base >= n;   // no chunk is left for the cursor
     return c;
 }
+// The same (DYN) with every chunk from the cursor: waves come to the queue one
+// by one, when another has run out.
+__device__ __forceinline__ RayChunks chunks_queued(uint32_t nwaves, uint32_t n) {
+    RayChunks c = chunks_first<true>(nwaves, nwaves, n);
+    c.next = c.end = n;
+    c.base = 0u;
+    c.exhausted = n == 0u;
+    return c;
+}
+// Even shares of two queues as one row of na + nb rays.
+__device__ __forceinline__ void chunks_joint(uint32_t wave, uint32_t nwaves, uint32_t na, uint32_t nb, RayChunks* a, RayChunks* b) {
+    const uint64_t n = (uint64_t)na + nb, per = (n + nwaves - 1) / nwaves, lo = wave * per, hi = lo + per;
+    auto upto = [](uint64_t v, uint32_t most) { return v < most ? (uint32_t)v : most; };
+    a->next = upto(lo, na);
+    a->end = upto(hi, na);
+    b->next = lo > na ? upto(lo - na, nb) : 0u;
+    b->end = hi > na ? upto(hi - na, nb) : 0u;
+    a->exhausted = b->exhausted = true;
+    a->chunk = b->chunk = a->base = b->base = a->n = b->n = 0u;
+}
 // Wave-uniform: the whole wave calls it, with every lane active.
 __device__ __forceinline__ void chunks_refill(RayChunks& c, uint32_t* dyn) {
     uint32_t got = 0;
