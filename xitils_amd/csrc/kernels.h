@@ -224,19 +224,23 @@ struct WalkArgs {
 // waves per SIMD of k_walk (at 3 instead of 4, with no spill instead of 28
 // registers', it measured the same; the normal-mapping form needs 256 VGPRs)
 constexpr int WALK_WAVES = 4, WALK_WAVES_NMAP = 2;
-// Paths from which a batch is queued instead of walked.  A walked path costs
-// the longest of its wave's rays at every vertex, a queued one its share of
-// three launches per round: below some half a million paths the launches, their
-// gaps and the slowest ray of each cost more.  Walked against queued, us, 100 k
-// triangle room (depth 16): 1111 / 3354 at 14 k paths, 2605 / 4055 at 230 k,
-// 4694 / 4898 at 460 k, 7452 / 6205 at 921 k; Cornell box (depth 8): 353 / 890,
-// 689 / 1003, 1168 / 1231, 1802 / 1612; 0.5 M triangle field 453 / 997,
-// 862 / 1618, 1200 / 1771, 1782 / 2137; normal-mapped plane 333 / 922,
-// 785 / 1339, 1152 / 1651, 2081 / 2313.
-constexpr uint32_t WALK_MAX = 11u << 16;
+// Most paths of a batch that are walked instead of queued.  A walked path costs
+// the longest of its wave's rays at every vertex, a queued one its share of two
+// launches per round; where a batch has few paths the launches, their gaps and
+// the slowest ray of each cost more.  They cost more again where rounds are
+// short: most paths leave for a sky early, and without a depth cap the last
+// paths go on for many rounds.  Walked against queued, us, 100 k triangle room
+// (depth 16): 769 / 962 at 14 k paths, 1359 / 1540 at 115 k, 2221 / 2334 at
+// 230 k, 3925 / 3267 at 460 k; material zoo 1133 / 1193 at 230 k, 1782 / 1574;
+// Cornell box (depth 8) 560 / 609, 1007 / 861.  Under a sky: 0.5 M triangle
+// field 971 / 1141 at 460 k, 1175 / 1266 at 691 k, 1475 / 1412 at 921 k;
+// normal-mapped plane 1058 / 1251, 1621 / 1522, 1914 / 1763.  Roulette only: zoo
+// 2437 / 2563, 2948 / 2955, 3409 / 3288, room 4375 / 4630 at 230 k, 6390 / 6045.
+constexpr uint32_t WALK_MAX = 5u << 16, WALK_MAX_SHORT_ROUNDS = 10u << 16;
 // Paths of a queue that are walked to their ends instead of queued on: the
-// last rounds of a large batch (Cornell box 1 M paths: 1671 us without, 1641
-// at 256 Ki, 1820 at 1 Mi).
+// last rounds of a large batch (material zoo at 460 k paths, us: 1782 from
+// 32 Ki, 1646 from 128 Ki, 1577 from 256 Ki, 1519 from 384 Ki; 100 k triangle
+// room at 460 k: 3326, 3328, 3272, 3671).
 constexpr uint32_t WALK_TAIL = 1u << 18;
 // Waves that few paths are spread over, by leaving lanes empty: a wave's step
 // takes as long as the slowest of its rays, so 6 k paths ran in 735 us at 64

@@ -736,6 +736,12 @@ static uint32_t trace_blocks(const xt_scene* s, size_t n) {
     return (uint32_t)std::max<size_t>(1, std::min<size_t>(b, s->trace_grid));
 }
 
+// Most paths that k_walk follows from their camera rays.
+static uint32_t walk_max(const xt_scene* s, int max_depth) {
+    return s->ds.env.has_sky || max_depth <= 0 ? WALK_MAX_SHORT_ROUNDS : WALK_MAX;
+}
+
+
 // Paths a wave of k_walk follows at a time, of n in all.
 static uint32_t walk_lanes(uint64_t n) {
     const uint64_t lanes = std::max<uint64_t>(1, (n + WALK_SPREAD - 1) / WALK_SPREAD);
@@ -1297,7 +1303,7 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                 s->stats.extend_launches++;
             };
             const bool can_walk = !guide && !s->counting;
-            const bool whole = can_walk && wp.num_paths <= WALK_MAX;
+            const bool whole = can_walk && wp.num_paths <= walk_max(s, p->max_depth);
             if (whole) {
                 walk(-1, wp.num_paths);
             } else {
@@ -1634,7 +1640,7 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
     const bool guide = gd.lobes_mk != nullptr;
     GuideState& g = s->guide;
     const uint32_t ib = std::max(1u, std::min((maxpaths + GI_BLOCK - 1) / GI_BLOCK, (uint32_t)s->dev->num_cu * 4));
-    const bool whole = !guide && maxpaths <= WALK_MAX;   // each path in one launch
+    const bool whole = !guide && maxpaths <= walk_max(s, p->max_depth);   // each path in one launch
     if (whole) {
         WalkArgs wa{};
         wa.wp = wp;
@@ -1879,6 +1885,7 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
     uint64_t total = 0;
     int max_depth = 1;
     bool nmap = false;
+    uint32_t wmax = WALK_MAX_SHORT_ROUNDS;   // paths up to which the window is walked
     uint32_t ovf_depth = 0;
     for (uint32_t i : which) {
         const xt_batch_item& it = items[i];
@@ -1890,6 +1897,7 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
             sc_list.push_back(s);
             ds.push_back(s->ds);
             nmap |= s->nmap;
+            wmax = std::min(wmax, walk_max(s, it.params.max_depth));
             ovf_depth = std::max(ovf_depth, s->ovf_depth);
         }
         MultiItem e{};
@@ -1928,7 +1936,7 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
         m.capacity = window;
     }
     xt_scene* s0 = sc_list[0];
-    const bool whole = window <= WALK_MAX;   // each path in one launch
+    const bool whole = window <= wmax;   // each path in one launch
     const uint32_t lanes = walk_lanes(window);
     const uint32_t tblocks = whole ? walk_blocks(s0, window, lanes, nmap, s0->trace_grid_max) : trace_blocks(s0, window);
     const uint32_t jblocks = trace_blocks(s0, 2 * (size_t)window);   // launches of two queues
