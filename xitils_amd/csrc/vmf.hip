@@ -428,18 +428,22 @@ const FitLauncher kFit[VMF_MAX_LOBES + 1] = {nullptr,         launch_fit<1>,  la
 
 // Device copies of host arrays (or the caller's device pointers).
 struct Staged {
+    xt_device* dev;
+    hipStream_t st;
     std::vector<void*> owned;
+    Staged(xt_device* d, hipStream_t stream) : dev(d), st(stream) {}
     ~Staged() {
-        for (void* p : owned) hipFree(p);
+        if (!owned.empty()) hipStreamSynchronize(st);   // also after an error halfway
+        for (void* p : owned) dev->stage.give(p);
     }
     template <class T>
-    hipError_t in(const T* src, size_t count, bool on_device, const T** dst, hipStream_t st) {
+    hipError_t in(const T* src, size_t count, bool on_device, const T** dst) {
         if (on_device || count == 0 || !src) {
             *dst = src;
             return hipSuccess;
         }
         T* d = nullptr;
-        hipError_t e = dalloc(&d, count);
+        hipError_t e = dev->stage.take(count * sizeof(T), (void**)&d);
         if (e != hipSuccess) return e;
         owned.push_back(d);
         *dst = d;
@@ -452,7 +456,7 @@ struct Staged {
             return hipSuccess;
         }
         T* d = nullptr;
-        hipError_t e = dalloc(&d, count);
+        hipError_t e = dev->stage.take(count * sizeof(T), (void**)&d);
         if (e != hipSuccess) return e;
         owned.push_back(d);
         *dst = d;
@@ -479,14 +483,14 @@ xt_status xt_vmf_eval(xt_device* dev, uint32_t num_lobes, const float* encoded, 
     if (n == 0) return XT_OK;
     if (!encoded || !dirs || !pdf || num_dists == 0) return xt_fail(XT_ERR_INVALID_ARGUMENT, "NULL or empty argument");
     const hipStream_t st = hipStreamPerThread;
-    Staged sg;
+    Staged sg(dev, st);
     const float *d_enc, *d_dirs;
     const uint32_t* d_dist;
     float* d_out;
     const size_t E = 5 * num_lobes - 1;
-    XT_HIP(sg.in(encoded, E * num_dists, on_device, &d_enc, st));
-    XT_HIP(sg.in(dist_of_dir, dist_of_dir ? (size_t)n : 0, on_device, &d_dist, st));
-    XT_HIP(sg.in(dirs, 3 * (size_t)n, on_device, &d_dirs, st));
+    XT_HIP(sg.in(encoded, E * num_dists, on_device, &d_enc));
+    XT_HIP(sg.in(dist_of_dir, dist_of_dir ? (size_t)n : 0, on_device, &d_dist));
+    XT_HIP(sg.in(dirs, 3 * (size_t)n, on_device, &d_dirs));
     XT_HIP(sg.out(pdf, n, on_device, &d_out));
     hipLaunchKernelGGL(k_vmf_eval, dim3((n + 255) / 256), dim3(256), 0, st, (int)num_lobes, d_enc, num_dists, d_dist,
                        d_dirs, n, d_out);
@@ -503,14 +507,14 @@ xt_status xt_vmf_sample(xt_device* dev, uint32_t num_lobes, const float* encoded
     if (n == 0) return XT_OK;
     if (!encoded || !uniforms || !dirs || num_dists == 0) return xt_fail(XT_ERR_INVALID_ARGUMENT, "NULL or empty argument");
     const hipStream_t st = hipStreamPerThread;
-    Staged sg;
+    Staged sg(dev, st);
     const float *d_enc, *d_u;
     const uint32_t* d_dist;
     float* d_out;
     const size_t E = 5 * num_lobes - 1;
-    XT_HIP(sg.in(encoded, E * num_dists, on_device, &d_enc, st));
-    XT_HIP(sg.in(dist_of_sample, dist_of_sample ? (size_t)n : 0, on_device, &d_dist, st));
-    XT_HIP(sg.in(uniforms, 4 * (size_t)n, on_device, &d_u, st));
+    XT_HIP(sg.in(encoded, E * num_dists, on_device, &d_enc));
+    XT_HIP(sg.in(dist_of_sample, dist_of_sample ? (size_t)n : 0, on_device, &d_dist));
+    XT_HIP(sg.in(uniforms, 4 * (size_t)n, on_device, &d_u));
     XT_HIP(sg.out(dirs, 3 * (size_t)n, on_device, &d_out));
     hipLaunchKernelGGL(k_vmf_sample, dim3((n + 255) / 256), dim3(256), 0, st, (int)num_lobes, d_enc, num_dists, d_dist,
                        d_u, n, d_out);
@@ -536,15 +540,15 @@ xt_status xt_vmf_fit(xt_device* dev, uint32_t num_lobes, const float* samples, u
     for (uint32_t f = 0; f < num_fits; ++f)
         if (hoff[f + 1] < hoff[f]) return xt_fail(XT_ERR_INVALID_ARGUMENT, "offsets must be non-decreasing");
     if (hoff[num_fits] > num_samples) return xt_fail(XT_ERR_INVALID_ARGUMENT, "offsets exceed num_samples");
-    Staged sg;
+    Staged sg(dev, st);
     const float *d_smp, *d_iu;
     const uint32_t* d_off;
     float* d_enc;
     int32_t* d_steps = nullptr;
     const size_t E = 5 * num_lobes - 1;
-    XT_HIP(sg.in(samples, 3 * (size_t)num_samples, on_device, &d_smp, st));
-    XT_HIP(sg.in(offsets, (size_t)num_fits + 1, on_device, &d_off, st));
-    XT_HIP(sg.in(init_uniforms, (size_t)2 * num_lobes * num_fits, on_device, &d_iu, st));
+    XT_HIP(sg.in(samples, 3 * (size_t)num_samples, on_device, &d_smp));
+    XT_HIP(sg.in(offsets, (size_t)num_fits + 1, on_device, &d_off));
+    XT_HIP(sg.in(init_uniforms, (size_t)2 * num_lobes * num_fits, on_device, &d_iu));
     XT_HIP(sg.out(encoded, E * num_fits, on_device, &d_enc));
     if (steps) XT_HIP(sg.out(steps, num_fits, on_device, &d_steps));
     kFit[num_lobes](fit_in_blocks(num_fits, hoff[num_fits] - hoff[0]), st, d_smp, d_off, num_fits, d_iu, d_enc, d_steps);
