@@ -256,7 +256,10 @@ template <bool QUEUE, bool NMAP, bool MULTI>
 __global__ void k_walk(WalkArgs a);
 
 __global__ void k_generate(WaveParams wp, PathQueue q, float4* radiance);
-template <bool GUIDE, bool NMAP, bool SORT>
+template <bool DYN>
+__global__ void k_trace_camera(DevScene sc, WaveParams wp, float4* hits, uint32_t* ovf, uint32_t* dyn,
+                               unsigned long long* clear);
+template <bool GUIDE, bool NMAP, bool SORT, bool FIRST>
 __global__ void k_shade(WaveParams wp, const DevScene* scene, PathQueue qin, const uint32_t* count_in, const float4* hits,
                         PathQueue qout, unsigned long long* counts_out, ShadowQueue sq,
                         float4* radiance, float4* pending, GuideRender gr);

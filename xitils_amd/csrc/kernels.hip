@@ -351,6 +351,43 @@ struct CursorMap {
     }
 };
 
+// The batch's camera rays, made where they are traced and again where their
+// hits are shaded (k_shade's FIRST form), so the first round has no ray queue:
+// writing and reading one cost 144 bytes a path and a launch, making the rays
+// twice some 300 VALU instructions (1080p field, 132 M paths: 58.06 -> 57.32 ms a
+// frame, of which k_generate 1.44, while the camera rays' trace went from 12.9
+// to 13.6; Cornell box 1239 -> 1232 us).
+template <bool DYN>
+__global__ __launch_bounds__(TRACE_BLOCK, 8) void k_trace_camera(DevScene sc, WaveParams wp, float4* __restrict__ hits,
+                                                                 uint32_t* __restrict__ ovf, uint32_t* __restrict__ dyn,
+                                                                 unsigned long long* __restrict__ clear) {
+    __shared__ uint32_t lds[TRACE_LDS_DEPTH * TRACE_BLOCK];
+    if (blockIdx.x == 0 && threadIdx.x == 0) *clear = 0ull;   // the next round's queues
+    __shared__ float4 top[TOP_F4];
+    stage_top_nodes(top, sc);
+    const size_t nthreads = (size_t)gridDim.x * blockDim.x;
+    const size_t gtid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t nwaves = (uint32_t)(nthreads / 64), wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(gtid / 64));
+    const RayChunks ch = chunks_first<DYN>(wave, nwaves, batch_of(wp).num_paths);
+    const CursorMap pmap{wp};
+    VisitCount vc;
+    RayPre r;
+    Trav t;
+    trace_queue<false, TRACE_LDS_DEPTH, false, DYN>(
+        ch, dyn, sc, r, t, top, lds + threadIdx.x, ovf ? ovf + gtid : nullptr, nthreads, vc,
+        [&](uint32_t i) {
+            f3 o, d;
+            const uint2 ps = pmap(i);
+            camera_ray(wp, ps.x, ps.y, &o, &d);
+            r = ray_setup(o, d);
+            trav_init(t, INFINITY);   // tMax = Infinity (PathTracer.h:167)
+        },
+        [&](uint32_t i, bool) { hits[i] = hit_record(t, t.best_slot); });
+    if constexpr (DYN) chunks_release(dyn);
+}
+template __global__ void k_trace_camera<false>(DevScene, WaveParams, float4*, uint32_t*, uint32_t*, unsigned long long*);
+template __global__ void k_trace_camera<true>(DevScene, WaveParams, float4*, uint32_t*, uint32_t*, unsigned long long*);
+
 // One StandardPathTracer / NaivePathTracer loop step (PathTracer.h:147-246 /
 // 65-101) for queue entry i: emission at the new vertex, roulette, BSDF
 // sample -> extension ray, light sample -> shadow ray.
@@ -654,32 +691,45 @@ __device__ __forceinline__ void shade_vertex(const WaveParams& wp, const DevScen
 }
 
 // shade_vertex of queue entry i.
-template <bool GUIDE, bool NMAP, class PathMap>
+// FIRST: the camera ray of path i, as k_trace_camera traced it.
+template <bool GUIDE, bool NMAP, bool FIRST, class PathMap>
 __device__ __forceinline__ void shade_entry(const WaveParams& wp, const DevScene& sc, const ShadeConst& sc0,
                                             const PathQueue& qin, const float4* __restrict__ hits,
                                             float4* __restrict__ radiance, float4* __restrict__ pending,
                                             const GuideRender& gr, uint32_t i, const PathMap& pmap, ShadeOut& out) {
-    const float4 o4 = qin.o[i], d4 = qin.d[i], w4 = qin.w[i];
     VertexIn in;
     in.h = hits[i];
-    in.id = __float_as_uint(d4.w);
-    const uint32_t vf = __float_as_uint(w4.w);
-    in.v = vf & 0xFFFFFFu;
-    in.qflags = vf >> 24;
-    // a camera ray (vertex 1) has no sampling record and no radiance yet:
-    // the generate step writes neither
-    const float4 e4 = in.v > 1 ? qin.e[i] : make_float4(1.0f, 1.0f, 1.0f, 0.0f);
-    in.pdf_prev = o4.w;
-    in.pe_prev = e4.w;
-    in.d = xyz(d4);
-    in.meval = xyz(e4);
-    in.weight = xyz(w4);
-    in.rad = in.v > 1 ? xyz(radiance[in.id]) : splat(0.0f);
-    in.pend = (in.qflags & QF_PENDING) ? xyz(pending[in.id]) : splat(0.0f);
-    if (GUIDE && gr.recs) {
-        // the vertex that sampled this ray: radiance up to and including its light sample
-        const uint32_t rin = qin.rec[i];
-        if (rin != INVALID) gr.recs[rin].f = f4(in.rad + in.pend, 0.0f);
+    if constexpr (FIRST) {
+        f3 o;
+        const uint2 ps = pmap(i);
+        camera_ray(wp, ps.x, ps.y, &o, &in.d);
+        in.id = i;
+        in.v = 1u;
+        in.qflags = 0u;
+        in.pdf_prev = in.pe_prev = 0.0f;
+        in.weight = in.meval = splat(1.0f);
+        in.rad = in.pend = splat(0.0f);
+    } else {
+        const float4 o4 = qin.o[i], d4 = qin.d[i], w4 = qin.w[i];
+        in.id = __float_as_uint(d4.w);
+        const uint32_t vf = __float_as_uint(w4.w);
+        in.v = vf & 0xFFFFFFu;
+        in.qflags = vf >> 24;
+        // a camera ray (vertex 1) has no sampling record and no radiance yet:
+        // the generate step writes neither
+        const float4 e4 = in.v > 1 ? qin.e[i] : make_float4(1.0f, 1.0f, 1.0f, 0.0f);
+        in.pdf_prev = o4.w;
+        in.pe_prev = e4.w;
+        in.d = xyz(d4);
+        in.meval = xyz(e4);
+        in.weight = xyz(w4);
+        in.rad = in.v > 1 ? xyz(radiance[in.id]) : splat(0.0f);
+        in.pend = (in.qflags & QF_PENDING) ? xyz(pending[in.id]) : splat(0.0f);
+        if (GUIDE && gr.recs) {
+            // the vertex that sampled this ray: radiance up to and including its light sample
+            const uint32_t rin = qin.rec[i];
+            if (rin != INVALID) gr.recs[rin].f = f4(in.rad + in.pend, 0.0f);
+        }
     }
     const uint32_t id = in.id;
     shade_vertex<GUIDE, NMAP>(wp, sc, sc0, in, gr, i, pmap, [&](f3 rad) { radiance[id] = f4(rad, 0.0f); }, out);
@@ -725,7 +775,9 @@ __device__ __forceinline__ void shade_emit(ShadeOut& o, const PathQueue& qout,
 
 // The forms without normal mapping (but the guided sorted one, at 144 VGPRs)
 // are bounded to 4 waves per SIMD, which they reach without spilling.
-template <bool GUIDE, bool NMAP, bool SORT>
+// FIRST: the first round of an unguided render, whose queue is the batch's
+// paths themselves.
+template <bool GUIDE, bool NMAP, bool SORT, bool FIRST>
 __global__ __launch_bounds__(SHADE_BLOCK, NMAP || (GUIDE && SORT) ? 1 : 4) void k_shade(WaveParams wp, const DevScene* __restrict__ scene, PathQueue qin,
                                                const uint32_t* __restrict__ count_in, const float4* __restrict__ hits,
                                                PathQueue qout, unsigned long long* __restrict__ counts_out,
@@ -735,7 +787,7 @@ __global__ __launch_bounds__(SHADE_BLOCK, NMAP || (GUIDE && SORT) ? 1 : 4) void 
     // occupy scalar registers for the whole kernel and spill (111 SGPR
     // spills, 556 lane reads, 112 VGPRs; through the pointer 32, 80, 103)
     const DevScene& sc = *scene;
-    const uint32_t n = *count_in;
+    const uint32_t n = FIRST ? batch_of(wp).num_paths : *count_in;
     const uint32_t stride = gridDim.x * blockDim.x;
     __shared__ uint32_t append_lds[2 * (SHADE_BLOCK / 64) + 2];
     __shared__ uint32_t sort_lds[SORT ? (SHADE_BLOCK / 64 + 1) * SHADE_KEYS + SHADE_BLOCK : 1];
@@ -745,23 +797,27 @@ __global__ __launch_bounds__(SHADE_BLOCK, NMAP || (GUIDE && SORT) ? 1 : 4) void 
     for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
         const uint32_t i = base + (SORT ? block_sort_by_material<SHADE_BLOCK>(sc, hits, base, n, sort_lds) : threadIdx.x);
         ShadeOut o;
-        if (i < n) shade_entry<GUIDE, NMAP>(wp, sc, c0, qin, hits, radiance, pending, gr, i, pmap, o);
+        if (i < n) shade_entry<GUIDE, NMAP, FIRST>(wp, sc, c0, qin, hits, radiance, pending, gr, i, pmap, o);
         shade_emit<GUIDE>(o, qout, counts_out, sq, gr, append_lds);
     }
 }
 
-#define XT_INST_SHADE(G, N, S)                                                                                   \
-    template __global__ void k_shade<G, N, S>(WaveParams, const DevScene*, PathQueue, const uint32_t*, const float4*,        \
-                                              PathQueue, unsigned long long*, ShadowQueue, float4*, float4*,          \
-                                              GuideRender);
-XT_INST_SHADE(false, false, false)
-XT_INST_SHADE(true, false, false)
-XT_INST_SHADE(false, true, false)
-XT_INST_SHADE(true, true, false)
-XT_INST_SHADE(false, false, true)
-XT_INST_SHADE(true, false, true)
-XT_INST_SHADE(false, true, true)
-XT_INST_SHADE(true, true, true)
+#define XT_INST_SHADE(G, N, S, F)                                                                                \
+    template __global__ void k_shade<G, N, S, F>(WaveParams, const DevScene*, PathQueue, const uint32_t*, const float4*,     \
+                                                 PathQueue, unsigned long long*, ShadowQueue, float4*, float4*,       \
+                                                 GuideRender);
+XT_INST_SHADE(false, false, false, false)
+XT_INST_SHADE(true, false, false, false)
+XT_INST_SHADE(false, true, false, false)
+XT_INST_SHADE(true, true, false, false)
+XT_INST_SHADE(false, false, true, false)
+XT_INST_SHADE(true, false, true, false)
+XT_INST_SHADE(false, true, true, false)
+XT_INST_SHADE(true, true, true, false)
+XT_INST_SHADE(false, false, false, true)
+XT_INST_SHADE(false, true, false, true)
+XT_INST_SHADE(false, false, true, true)
+XT_INST_SHADE(false, true, true, true)
 #undef XT_INST_SHADE
 
 // Any-hit for queued shadow rays; unoccluded contributions go straight to the
@@ -1001,7 +1057,7 @@ __global__ __launch_bounds__(SHADE_BLOCK, NMAP ? 1 : 4) void k_shade_multi(Multi
         if (i < n) {
             const MultiItem& it = mb.items[mb.item_of[__float_as_uint(qin.d[i].w)]];
             const DevScene& sc = mb.scenes[it.scene];
-            shade_entry<false, NMAP>(it.wp, sc, shade_const(it.wp, sc), qin, hits, radiance, pending, gr, i,
+            shade_entry<false, NMAP, false>(it.wp, sc, shade_const(it.wp, sc), qin, hits, radiance, pending, gr, i,
                                      ItemMap{it, g0}, o);
         }
         shade_emit<false>(o, qout, counts_out, sq, gr, append_lds);

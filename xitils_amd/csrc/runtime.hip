@@ -188,13 +188,14 @@ using ShadeKernel = void (*)(WaveParams, const DevScene*, PathQueue, const uint3
 // materials or not, and with the block-local material partition
 // (XT_FLAG_SORT_MATERIALS) or not -- separate instantiations, so the plain
 // kernel carries none of the others' registers.
-static ShadeKernel shade_kernel(bool guide, bool nmap, uint32_t flags) {
-    if (flags & XT_FLAG_SORT_MATERIALS) {
-        if (nmap) return guide ? k_shade<true, true, true> : k_shade<false, true, true>;
-        return guide ? k_shade<true, false, true> : k_shade<false, false, true>;
-    }
-    if (nmap) return guide ? k_shade<true, true, false> : k_shade<false, true, false>;
-    return guide ? k_shade<true, false, false> : k_shade<false, false, false>;
+template <bool SORT>
+static ShadeKernel shade_kernel(bool guide, bool nmap, bool first) {
+    if (first) return nmap ? k_shade<false, true, SORT, true> : k_shade<false, false, SORT, true>;
+    if (nmap) return guide ? k_shade<true, true, SORT, false> : k_shade<false, true, SORT, false>;
+    return guide ? k_shade<true, false, SORT, false> : k_shade<false, false, SORT, false>;
+}
+static ShadeKernel shade_kernel(bool guide, bool nmap, uint32_t flags, bool first) {
+    return flags & XT_FLAG_SORT_MATERIALS ? shade_kernel<true>(guide, nmap, first) : shade_kernel<false>(guide, nmap, first);
 }
 
 extern "C" {
@@ -1352,11 +1353,14 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                 s->stats.extend_launches++;
             };
             const bool can_walk = !guide && !s->counting;
+            // the first round makes its rays itself, unless the network reads
+            // their queue or fetches are counted
+            const bool camera = !guide && !s->counting;
             const bool whole = can_walk && wp.num_paths <= walk_max(s, p->max_depth);
             if (whole) {
                 walk(-1, wp.num_paths);
                 if (result == XT_OK) result = send_film();
-            } else {
+            } else if (!camera) {
                 hipLaunchKernelGGL(k_generate, dim3(blocks256(wp.num_paths)), dim3(256), 0, s->stream, wp, rb.q[0], rb.radiance);
                 XT_LAUNCHED(result);
                 hipLaunchKernelGGL(k_set_u32, dim3(1), dim3(1), 0, s->stream, path_count(rb.counts, 0), wp.num_paths);
@@ -1411,7 +1415,11 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                     // round's shadow queue is no longer than its path queue)
                     const bool dyn = bound >= TRAV_DYN_MIN;
                     // both forms also clear the next round's counters
-                    if (joint && round > 0) {
+                    if (camera && round == 0) {
+                        hipLaunchKernelGGL((dyn ? k_trace_camera<true> : k_trace_camera<false>), dim3(trace_blocks(s, bound)),
+                                           dim3(TRACE_BLOCK), 0, s->stream, s->ds, wp, rb.hits, s->d_ovf, rb.dyn,
+                                           pair_count(rb.counts, 1 - cur));
+                    } else if (joint && round > 0) {
                         const int slot = (round - 1) % RB_RING;
                         hipLaunchKernelGGL((dyn ? k_trace_shadow<false, true> : k_trace_shadow<false, false>),
                                            dim3(trace_blocks(s, 2 * (size_t)bound)), dim3(TRACE_BLOCK), 0, s->stream, s->ds,
@@ -1457,7 +1465,7 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                         }
                     }
                     a = tm.mark();
-                    hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags), dim3(shade_blocks(bound)), dim3(SHADE_BLOCK), 0,
+                    hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags, camera && round == 0), dim3(shade_blocks(bound)), dim3(SHADE_BLOCK), 0,
                                        s->stream, wp, s->d_ds, rb.q[cur], path_count(rb.counts, cur), rb.hits, rb.q[1 - cur],
                                        pair_count(rb.counts, 1 - cur), rb.sq, rb.radiance, rb.pending, gr);
                     XT_LAUNCHED(result);
@@ -1703,13 +1711,16 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
         wa.dyn = b.dyn;
         hipLaunchKernelGGL((s->nmap ? k_walk<false, true, false> : k_walk<false, false, false>),
                            dim3(walk_blocks(s, maxpaths, wa.lanes, s->nmap, tmost)), dim3(TRACE_BLOCK), 0, s->stream, wa);
-    } else {
+    } else if (guide) {
         hipLaunchKernelGGL(k_generate, dim3(gblocks), dim3(256), 0, s->stream, wp, b.q[0], b.radiance);
         hipLaunchKernelGGL(k_count_from_cursor, dim3(1), dim3(1), 0, s->stream, path_count(b.counts, 0), cursor);
     }
     int cur = 0;
     for (int it = 0; it <= p->max_depth && !whole; ++it) {
-        if (it == 0)
+        if (it == 0 && !guide)
+            hipLaunchKernelGGL(k_trace_camera<false>, dim3(tblocks), dim3(TRACE_BLOCK), 0, s->stream, s->ds, wp, b.hits, b.ovf,
+                               nullptr, pair_count(b.counts, 1));
+        else if (it == 0)
             hipLaunchKernelGGL((k_trace<false, TRACE_LDS_DEPTH, false>), dim3(tblocks), dim3(TRACE_BLOCK), 0, s->stream, s->ds,
                                b.q[0].o, b.q[0].d, 1, path_count(b.counts, 0), 0u, b.hits, nullptr, 0, 0, b.ovf, nullptr, nullptr,
                                path_count(b.counts, 1), shadow_count(b.counts, 1));
@@ -1727,7 +1738,7 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
             gr.prob = g.cfg.guide_prob;
             gr.max_vertex = g.cfg.max_guided_vertex;
         }
-        hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags), dim3(sblocks), dim3(SHADE_BLOCK), 0, s->stream, wp, s->d_ds,
+        hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags, it == 0 && !guide), dim3(sblocks), dim3(SHADE_BLOCK), 0, s->stream, wp, s->d_ds,
                            b.q[cur], path_count(b.counts, cur), b.hits, b.q[1 - cur], pair_count(b.counts, 1 - cur), b.sq,
                            b.radiance, b.pending, gr);
         cur = 1 - cur;
