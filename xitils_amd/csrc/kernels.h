@@ -202,6 +202,10 @@ template <bool NMAP>
 __global__ void k_shade_multi(MultiBatch mb, PathQueue qin, const uint32_t* count_in, const float4* hits,
                               PathQueue qout, unsigned long long* counts_out, ShadowQueue sq,
                               float4* radiance, float4* pending);
+template <bool NMAP>
+__global__ void k_shade_multi_open(MultiBatch mb, PathQueue qin, const uint32_t* count_in, const float4* hits,
+                                   PathQueue qout, unsigned long long* counts_out, ShadowQueue sq, float4* radiance,
+                                   float4* pending);
 __global__ void k_accumulate_multi(MultiBatch mb, const float4* radiance);
 
 // Arguments of k_walk.  MULTI uses mb, the others wp and scene; QUEUE (paths
@@ -263,6 +267,10 @@ template <bool GUIDE, bool NMAP, bool SORT, bool FIRST>
 __global__ void k_shade(WaveParams wp, const DevScene* scene, PathQueue qin, const uint32_t* count_in, const float4* hits,
                         PathQueue qout, unsigned long long* counts_out, ShadowQueue sq,
                         float4* radiance, float4* pending, GuideRender gr);
+template <bool NMAP>
+__global__ void k_shade_open(WaveParams wp, const DevScene* scene, PathQueue qin, const uint32_t* count_in,
+                             const float4* hits, PathQueue qout, unsigned long long* counts_out, ShadowQueue sq,
+                             float4* radiance, float4* pending, GuideRender gr);
 template <bool COUNT, bool DYN = false>
 __global__ void k_shadow(DevScene sc, ShadowQueue sq, const uint32_t* count, float4* radiance, float4* pending,
                          uint32_t* ovf, uint32_t* dyn, unsigned long long* visit_totals, const uint32_t* counts4,

@@ -194,7 +194,9 @@ static ShadeKernel shade_kernel(bool guide, bool nmap, bool first) {
     if (nmap) return guide ? k_shade<true, true, SORT, false> : k_shade<false, true, SORT, false>;
     return guide ? k_shade<true, false, SORT, false> : k_shade<false, false, SORT, false>;
 }
-static ShadeKernel shade_kernel(bool guide, bool nmap, uint32_t flags, bool first) {
+// open: a round of bounced rays, many of which may leave for a sky.
+static ShadeKernel shade_kernel(bool guide, bool nmap, uint32_t flags, bool first, bool open) {
+    if (open && !guide && !first && !(flags & XT_FLAG_SORT_MATERIALS)) return nmap ? k_shade_open<true> : k_shade_open<false>;
     return flags & XT_FLAG_SORT_MATERIALS ? shade_kernel<true>(guide, nmap, first) : shade_kernel<false>(guide, nmap, first);
 }
 
@@ -1465,7 +1467,7 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                         }
                     }
                     a = tm.mark();
-                    hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags, camera && round == 0), dim3(shade_blocks(bound)), dim3(SHADE_BLOCK), 0,
+                    hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags, camera && round == 0, !s->counting && s->ds.env.has_sky), dim3(shade_blocks(bound)), dim3(SHADE_BLOCK), 0,
                                        s->stream, wp, s->d_ds, rb.q[cur], path_count(rb.counts, cur), rb.hits, rb.q[1 - cur],
                                        pair_count(rb.counts, 1 - cur), rb.sq, rb.radiance, rb.pending, gr);
                     XT_LAUNCHED(result);
@@ -1738,7 +1740,7 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
             gr.prob = g.cfg.guide_prob;
             gr.max_vertex = g.cfg.max_guided_vertex;
         }
-        hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags, it == 0 && !guide), dim3(sblocks), dim3(SHADE_BLOCK), 0, s->stream, wp, s->d_ds,
+        hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags, it == 0 && !guide, s->ds.env.has_sky), dim3(sblocks), dim3(SHADE_BLOCK), 0, s->stream, wp, s->d_ds,
                            b.q[cur], path_count(b.counts, cur), b.hits, b.q[1 - cur], pair_count(b.counts, 1 - cur), b.sq,
                            b.radiance, b.pending, gr);
         cur = 1 - cur;
@@ -1947,7 +1949,7 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
     std::vector<DevScene>& ds = run.ds;
     uint64_t total = 0;
     int max_depth = 1;
-    bool nmap = false;
+    bool nmap = false, open = false;   // some scene has normal maps, a sky
     uint32_t wmax = WALK_MAX_SHORT_ROUNDS;   // paths up to which the window is walked
     uint32_t ovf_depth = 0;
     for (uint32_t i : which) {
@@ -1960,6 +1962,7 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
             sc_list.push_back(s);
             ds.push_back(s->ds);
             nmap |= s->nmap;
+            open |= s->ds.env.has_sky != 0;
             wmax = std::min(wmax, walk_max(s, it.params.max_depth));
             ovf_depth = std::max(ovf_depth, s->ovf_depth);
         }
@@ -2074,14 +2077,10 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
             hipLaunchKernelGGL((dyn ? k_trace_shadow<true, true> : k_trace_shadow<true, false>), dim3(jblocks), dim3(TRACE_BLOCK),
                                0, m.stream, s0->ds, m.q[cur].o, m.q[cur].d, m.hits, m.sq, m.counts, cur, m.radiance, m.pending,
                                m.ovf, m.dyn, nullptr, m.item_of, m.items);
-        if (nmap)
-            hipLaunchKernelGGL(k_shade_multi<true>, dim3(sblocks), dim3(SHADE_BLOCK), 0, m.stream, mb, m.q[cur],
-                               path_count(m.counts, cur), m.hits, m.q[1 - cur], pair_count(m.counts, 1 - cur), m.sq,
-                               m.radiance, m.pending);
-        else
-            hipLaunchKernelGGL(k_shade_multi<false>, dim3(sblocks), dim3(SHADE_BLOCK), 0, m.stream, mb, m.q[cur],
-                               path_count(m.counts, cur), m.hits, m.q[1 - cur], pair_count(m.counts, 1 - cur), m.sq,
-                               m.radiance, m.pending);
+        auto shade = open && it > 0 ? (nmap ? k_shade_multi_open<true> : k_shade_multi_open<false>)
+                                    : (nmap ? k_shade_multi<true> : k_shade_multi<false>);
+        hipLaunchKernelGGL(shade, dim3(sblocks), dim3(SHADE_BLOCK), 0, m.stream, mb, m.q[cur], path_count(m.counts, cur), m.hits,
+                           m.q[1 - cur], pair_count(m.counts, 1 - cur), m.sq, m.radiance, m.pending);
         cur = 1 - cur;
     }
     if (!whole)
