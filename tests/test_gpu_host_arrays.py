@@ -50,3 +50,27 @@ def test_host_films_equal_device_films(f64):
         sc.render(w, h, spp, film=film, f64=f64, **kw)
         sc.render_device(ref.data_ptr(), w, h, spp, f64=f64, **kw)
         assert np.array_equal(film, ref.cpu().numpy())
+
+
+def test_host_queries_of_several_threads():
+    """Each thread its own scene: one query at a time has the mapped buffer, the others copy."""
+    import threading
+    dev, n = api.Device(0), 3000
+    jobs = []
+    for k in range(4):
+        sc, rays = api.Scene(dev, scenes.material_zoo(64, 64)), _rays(n, k)
+        jobs.append((sc, rays, sc.trace_closest(rays).tobytes(), sc.trace_any(rays).tobytes()))
+    print("[gpu] host queries of four threads", flush=True)
+    wrong = []
+
+    def work(sc, rays, hits, occ):
+        for _ in range(20):
+            if sc.trace_closest(rays).tobytes() != hits or sc.trace_any(rays).tobytes() != occ:
+                wrong.append(sc)
+
+    threads = [threading.Thread(target=work, args=j) for j in jobs]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong

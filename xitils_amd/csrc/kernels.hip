@@ -1431,7 +1431,6 @@ __global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) v
                     c = has_pend ? xyz(a.pending[id]) : splat(0.0f);
                     eo = xyz(o4);
                     ed = xyz(d4);
-                    if constexpr (MULTI) item = mb.item_of[id];
                 } else {
                     id = my;
                     if constexpr (MULTI) {
@@ -1635,8 +1634,6 @@ template __global__ void k_walk<true, false, false>(WalkArgs);
 template __global__ void k_walk<false, true, false>(WalkArgs);
 template __global__ void k_walk<true, true, false>(WalkArgs);
 template __global__ void k_walk<false, false, true>(WalkArgs);
-template __global__ void k_walk<true, false, true>(WalkArgs);
 template __global__ void k_walk<false, true, true>(WalkArgs);
-template __global__ void k_walk<true, true, true>(WalkArgs);
 
 }  // namespace xt

@@ -9,7 +9,6 @@
 #include "../../include/xitils_amd.h"
 
 #include <mutex>
-#include <vector>
 
 struct MultiState;   // unified-batch buffers (runtime.hip)
 struct RenderPool;   // xt_render's path buffers, shared by the device's scenes (runtime.hip)
@@ -25,7 +24,7 @@ public:
         std::lock_guard<std::mutex> lock(mu);
         Block* best = nullptr;
         for (Block& b : blocks)
-            if (!b.busy && b.bytes >= bytes && (!best || b.bytes < best->bytes)) best = &b;
+            if (b.p && !b.busy && b.bytes >= bytes && (!best || b.bytes < best->bytes)) best = &b;
         if (best) {
             best->busy = true;
             *p = best->p;
@@ -33,15 +32,18 @@ public:
         }
         if (held + bytes > KEEP) drop_free();
         hipError_t e = hipMalloc(p, bytes);
-        if (e == hipErrorOutOfMemory && !blocks.empty()) {
+        if (e == hipErrorOutOfMemory && held > 0) {
             (void)hipGetLastError();
             drop_free();
             e = hipMalloc(p, bytes);
         }
-        if (e == hipSuccess && held + bytes <= KEEP) {
-            blocks.push_back({*p, bytes, true});
-            held += bytes;
-        }
+        if (e == hipSuccess && held + bytes <= KEEP)
+            for (Block& b : blocks)
+                if (!b.p) {
+                    b = {*p, bytes, true};
+                    held += bytes;
+                    break;
+                }
         return e;
     }
     // The caller's work on p has ended.
@@ -61,24 +63,20 @@ public:
 
 private:
     struct Block {
-        void* p;
-        size_t bytes;
-        bool busy;
+        void* p = nullptr;
+        size_t bytes = 0;
+        bool busy = false;
     };
     void drop_free() {
-        size_t kept = 0;
-        for (Block& b : blocks) {
-            if (b.busy) {
-                blocks[kept++] = b;
-            } else {
+        for (Block& b : blocks)
+            if (b.p && !b.busy) {
                 held -= b.bytes;
                 hipFree(b.p);
+                b = Block{};
             }
-        }
-        blocks.resize(kept);
     }
     std::mutex mu;
-    std::vector<Block> blocks;
+    Block blocks[64];
     size_t held = 0;
 };
 
@@ -90,6 +88,10 @@ struct xt_device {
     RenderPool* pool = nullptr;         // created by the first xt_render
     std::mutex pool_mu;                 // guards creating `pool`
     StagePool stage;                    // copies of host arrays
+    unsigned char* query_io = nullptr;      // pinned rays and results of small host queries
+    unsigned char* query_io_dev = nullptr;  // the same memory's device address
+    bool query_busy = false;                // in some thread's query
+    std::mutex query_mu;                    // guards the three
     unsigned char* scratch = nullptr;   // this device's address of the static scratch array (xt_render_static)
 };
 

@@ -155,8 +155,6 @@ struct xt_scene {
     float* d_map_marg = nullptr;
     float* d_map_cond = nullptr;
     uint32_t ovf_depth = 0;           // entries per lane beyond the LDS part
-    unsigned char* h_query = nullptr;       // pinned rays and results of small host queries
-    unsigned char* h_query_dev = nullptr;   // the same memory's device address
     hipStream_t copy_stream = nullptr;      // uploads of host films
     hipEvent_t copy_ev = nullptr;
     uint32_t trace_grid_max = 0;      // blocks of the traversal kernels (sizes the spill columns)
@@ -247,6 +245,7 @@ xt_status xt_device_close(xt_device* dev) {
         hipSetDevice(dev->ordinal);
         hipDeviceSynchronize();
         delete dev->pool;
+        if (dev->query_io) hipHostFree(dev->query_io);
     }
     delete dev;
     return XT_OK;
@@ -291,7 +290,6 @@ xt_status xt_scene_destroy(xt_scene* s) {
     for (float4* t : s->d_texels) hipFree(t);
     hipFree(s->d_light_pdf); hipFree(s->d_light_objs); hipFree(s->d_light_slots); hipFree(s->d_ovf);
     hipFree(s->d_qrays); hipFree(s->d_qhits); hipFree(s->d_qocc); hipFree(s->d_qvisits); hipFree(s->d_qdyn);
-    if (s->h_query) hipHostFree(s->h_query);
     if (s->copy_ev) hipEventDestroy(s->copy_ev);
     if (s->copy_stream) hipStreamDestroy(s->copy_stream);
     hipFree(s->d_map); hipFree(s->d_map_pdf); hipFree(s->d_map_marg); hipFree(s->d_map_cond);
@@ -772,22 +770,47 @@ static uint32_t walk_blocks(const xt_scene* s, uint64_t n, uint32_t lanes, bool 
 // 194 against 308 / 180 for 128 Ki.
 constexpr uint32_t QUERY_MAPPED = 1u << 15;
 
+// The device's one mapped buffer, for a query at a time (take() is false when
+// another thread's has it: that query copies, as a larger one does).
+struct MappedQuery {
+    xt_device* dev = nullptr;
+    bool take(xt_device* d) {
+        std::lock_guard<std::mutex> lock(d->query_mu);
+        if (d->query_busy) return false;
+        if (!d->query_io) {
+            void *h = nullptr, *p = nullptr;
+            if (hipHostMalloc(&h, QUERY_MAPPED * (sizeof(xt_ray) + sizeof(xt_hit)), hipHostMallocMapped | hipHostMallocCoherent) !=
+                    hipSuccess ||
+                hipHostGetDevicePointer(&p, h, 0) != hipSuccess) {
+                (void)hipGetLastError();
+                if (h) hipHostFree(h);
+                return false;
+            }
+            d->query_io = (unsigned char*)h;
+            d->query_io_dev = (unsigned char*)p;
+        }
+        dev = d;
+        return d->query_busy = true;
+    }
+    ~MappedQuery() {
+        if (!dev) return;
+        std::lock_guard<std::mutex> lock(dev->query_mu);
+        dev->query_busy = false;
+    }
+};
+
 static xt_status query(xt_scene* s, const xt_ray* rays, uint32_t n, void* out, int on_device, bool any) {
     if (!s || (n && (!rays || !out))) return fail(XT_ERR_INVALID_ARGUMENT, "NULL argument");
     if (n == 0) return XT_OK;
     XT_HIP(hipSetDevice(s->dev->ordinal));
     const float4* d_rays = (const float4*)rays;
     void* d_out = out;
-    const bool mapped = !on_device && n <= QUERY_MAPPED;
+    MappedQuery io;
+    const bool mapped = !on_device && n <= QUERY_MAPPED && io.take(s->dev);
     if (mapped) {
-        if (!s->h_query) {
-            XT_HIP(hipHostMalloc((void**)&s->h_query, QUERY_MAPPED * (sizeof(xt_ray) + sizeof(xt_hit)),
-                                 hipHostMallocMapped | hipHostMallocCoherent));
-            XT_HIP(hipHostGetDevicePointer((void**)&s->h_query_dev, s->h_query, 0));
-        }
-        std::memcpy(s->h_query, rays, (size_t)n * sizeof(xt_ray));
-        d_rays = (const float4*)s->h_query_dev;
-        d_out = s->h_query_dev + QUERY_MAPPED * sizeof(xt_ray);
+        std::memcpy(s->dev->query_io, rays, (size_t)n * sizeof(xt_ray));
+        d_rays = (const float4*)s->dev->query_io_dev;
+        d_out = s->dev->query_io_dev + QUERY_MAPPED * sizeof(xt_ray);
     } else if (!on_device) {
         if (s->qrays_cap < n) {
             hipFree(s->d_qrays);
@@ -851,7 +874,7 @@ static xt_status query(xt_scene* s, const xt_ray* rays, uint32_t n, void* out, i
     if (le == hipSuccess && se == hipSuccess) hipEventElapsedTime(&ms, ev[0], ev[1]);
     if (le != hipSuccess) return fail(XT_ERR_DEVICE, std::string("ray query failed: ") + hipGetErrorString(le));
     if (se != hipSuccess) return fail(XT_ERR_DEVICE, std::string("ray query failed: ") + hipGetErrorString(se));
-    if (mapped) std::memcpy(out, s->h_query + QUERY_MAPPED * sizeof(xt_ray), out_bytes);
+    if (mapped) std::memcpy(out, s->dev->query_io + QUERY_MAPPED * sizeof(xt_ray), out_bytes);
     s->stats = xt_render_stats{};
     s->stats.ms_total = ms;
     unsigned long long v[2] = {0, 0};
