@@ -47,7 +47,7 @@ struct RenderBuffers {
     float* lobes = nullptr;          // decoded guide mixtures per path-queue entry (allocated on demand)
     uint32_t* counts = nullptr;      // queue lengths (path_count, shadow_count)
     uint32_t* host_counts = nullptr; // pinned, RB_RING slots of 4 counts (bounce rounds in flight)
-    uint32_t* host_counts_dev = nullptr;  // the same memory's device address (written by k_shadow)
+    uint32_t* host_counts_dev = nullptr;  // the same memory's device address (written by k_shadow and k_trace_shadow)
     hipEvent_t round_ev[RB_RING] = {};
     unsigned long long* visits = nullptr;  // node, tri fetches: extension [0..1], shadow [2..3]
     uint32_t* dyn = nullptr;               // chunk cursors of the traversal kernels: extension [0..1], shadow [2..3]
