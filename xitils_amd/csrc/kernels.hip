@@ -277,7 +277,7 @@ __global__ __launch_bounds__(256) void k_generate(WaveParams wp, PathQueue q, fl
 }
 
 // Material-sorted shading (XT_FLAG_SORT_MATERIALS): the block's queue
-// entries [base, base + SHADE_BLOCK) are partitioned by shading key (miss,
+// entries [base, base + blockDim.x) are partitioned by shading key (miss,
 // then 1 + material type of the hit) before they are shaded, stably, so each
 // wave of the block mostly shades one kind of BSDF instead of every kind the
 // queue mixes.  Returns this thread's entry offset within the block; every
@@ -739,13 +739,13 @@ __device__ __forceinline__ void shade_entry(const WaveParams& wp, const DevScene
 
 // Compacted appends of a block's shaded entries (every thread of the block
 // calls it): the extension ray with its training record, the shadow ray.
-template <bool GUIDE>
+template <bool GUIDE, int BLOCK>
 __device__ __forceinline__ void shade_emit(ShadeOut& o, const PathQueue& qout,
                                            unsigned long long* __restrict__ counts_out, const ShadowQueue& sq,
                                            const GuideRender& gr, uint32_t* append_lds) {
     // guided light samples: a non-finite contribution is dropped, never summed
     if (GUIDE && o.push_sh && !finite3(o.sh_c)) o.push_sh = false;
-    const uint2 slots = block_append2<SHADE_BLOCK>(counts_out, o.push_ext, o.push_sh, append_lds);
+    const uint2 slots = block_append2<BLOCK>(counts_out, o.push_ext, o.push_sh, append_lds);
     const uint32_t ei = slots.x, si = slots.y;
     if (o.push_ext) {
         uint32_t fl = o.push_sh ? QF_PENDING : 0u;
@@ -780,7 +780,7 @@ __device__ __forceinline__ void shade_emit(ShadeOut& o, const PathQueue& qout,
 // FIRST: the first round of an unguided render, whose queue is the batch's
 // paths themselves.
 template <bool GUIDE, bool NMAP, bool SORT, bool FIRST>
-__global__ __launch_bounds__(SHADE_BLOCK, NMAP || (GUIDE && SORT) ? 1 : 4) void k_shade(WaveParams wp, const DevScene* __restrict__ scene, PathQueue qin,
+__global__ __launch_bounds__(shade_block(GUIDE, NMAP), NMAP || (GUIDE && SORT) ? 1 : 4) void k_shade(WaveParams wp, const DevScene* __restrict__ scene, PathQueue qin,
                                                const uint32_t* __restrict__ count_in, const float4* __restrict__ hits,
                                                PathQueue qout, unsigned long long* __restrict__ counts_out,
                                                ShadowQueue sq, float4* __restrict__ radiance,
@@ -791,16 +791,17 @@ __global__ __launch_bounds__(SHADE_BLOCK, NMAP || (GUIDE && SORT) ? 1 : 4) void 
     const DevScene& sc = *scene;
     const uint32_t n = FIRST ? batch_of(wp).num_paths : *count_in;
     const uint32_t stride = gridDim.x * blockDim.x;
-    __shared__ uint32_t append_lds[2 * (SHADE_BLOCK / 64) + 2];
-    __shared__ uint32_t sort_lds[SORT ? (SHADE_BLOCK / 64 + 1) * SHADE_KEYS + SHADE_BLOCK : 1];
+    constexpr int BLOCK = shade_block(GUIDE, NMAP);
+    __shared__ uint32_t append_lds[2 * (BLOCK / 64) + 2];
+    __shared__ uint32_t sort_lds[SORT ? (BLOCK / 64 + 1) * SHADE_KEYS + BLOCK : 1];
     const CursorMap pmap{wp};
     const ShadeConst c0 = shade_const(wp, sc);
     // whole-block iterations so the appends below always see every thread
     for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
-        const uint32_t i = base + (SORT ? block_sort_by_material<SHADE_BLOCK>(sc, hits, base, n, sort_lds) : threadIdx.x);
+        const uint32_t i = base + (SORT ? block_sort_by_material<BLOCK>(sc, hits, base, n, sort_lds) : threadIdx.x);
         ShadeOut o;
         if (i < n) shade_entry<GUIDE, NMAP, FIRST>(wp, sc, c0, qin, hits, radiance, pending, gr, i, pmap, o);
-        shade_emit<GUIDE>(o, qout, counts_out, sq, gr, append_lds);
+        shade_emit<GUIDE, BLOCK>(o, qout, counts_out, sq, gr, append_lds);
     }
 }
 
@@ -812,14 +813,14 @@ __global__ __launch_bounds__(SHADE_BLOCK, NMAP || (GUIDE && SORT) ? 1 : 4) void 
 // second round 6.1 -> 4.3 ms, now some 3.3 TB/s; plane at 6.2 M paths 8.0 -> 6.8.
 // A first round, whose camera rays miss together, is faster in queue order
 // (plane 6.72 against 6.87 ms).
-// list: 2 * SHADE_BLOCK entries, wave_hits: one count per wave.
-template <class Miss, class Hit>
+// list: 2 * BLOCK entries, wave_hits: one count per wave.
+template <int BLOCK, class Miss, class Hit>
 __device__ __forceinline__ void shade_open(uint32_t n, const float4* __restrict__ hits, const PathQueue& qout,
                                            unsigned long long* __restrict__ counts_out, const ShadowQueue& sq,
                                            uint32_t* append_lds, uint32_t* list, uint32_t* wave_hits, Miss miss, Hit hit) {
     const GuideRender gr{};
     const uint32_t stride = gridDim.x * blockDim.x, wave = threadIdx.x / 64;
-    uint32_t waiting = 0;   // entries of list: below SHADE_BLOCK between iterations
+    uint32_t waiting = 0;   // entries of list: below BLOCK between iterations
     for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
         const uint32_t i = base + threadIdx.x;
         const bool hits_i = i < n && __float_as_uint(hits[i].y) != INVALID;
@@ -828,7 +829,7 @@ __device__ __forceinline__ void shade_open(uint32_t n, const float4* __restrict_
         if (__lane_id() == 0) wave_hits[wave] = (uint32_t)__popcll(mask);
         __syncthreads();
         uint32_t at = waiting;
-        for (uint32_t w = 0; w < SHADE_BLOCK / 64; ++w) {
+        for (uint32_t w = 0; w < BLOCK / 64; ++w) {
             const uint32_t c = wave_hits[w];
             if (w < wave) at += c;
             waiting += c;
@@ -836,28 +837,29 @@ __device__ __forceinline__ void shade_open(uint32_t n, const float4* __restrict_
         if (hits_i) list[at + (uint32_t)__popcll(mask & ((1ull << __lane_id()) - 1ull))] = i;
         __syncthreads();
         const bool last = n - base <= stride;
-        while (waiting >= (uint32_t)SHADE_BLOCK || (last && waiting)) {
-            const uint32_t take = min(waiting, (uint32_t)SHADE_BLOCK);
+        while (waiting >= (uint32_t)BLOCK || (last && waiting)) {
+            const uint32_t take = min(waiting, (uint32_t)BLOCK);
             waiting -= take;
             ShadeOut o;
             if (threadIdx.x < take) hit(list[waiting + threadIdx.x], o);
-            shade_emit<false>(o, qout, counts_out, sq, gr, append_lds);   // ends with every list entry read
+            shade_emit<false, BLOCK>(o, qout, counts_out, sq, gr, append_lds);   // ends with every list entry read
         }
     }
 }
 
 template <bool NMAP>
-__global__ __launch_bounds__(SHADE_BLOCK, NMAP ? 1 : 4) void k_shade_open(WaveParams wp, const DevScene* __restrict__ scene,
+__global__ __launch_bounds__(shade_block(false, NMAP), NMAP ? 1 : 4) void k_shade_open(WaveParams wp, const DevScene* __restrict__ scene,
                                                                        PathQueue qin, const uint32_t* __restrict__ count_in,
                                                                        const float4* __restrict__ hits, PathQueue qout,
                                                                        unsigned long long* __restrict__ counts_out,
                                                                        ShadowQueue sq, float4* __restrict__ radiance,
                                                                        float4* __restrict__ pending, GuideRender gr) {
-    __shared__ uint32_t append_lds[2 * (SHADE_BLOCK / 64) + 2], list[2 * SHADE_BLOCK], wave_hits[SHADE_BLOCK / 64];
+    constexpr int BLOCK = shade_block(false, NMAP);
+    __shared__ uint32_t append_lds[2 * (BLOCK / 64) + 2], list[2 * BLOCK], wave_hits[BLOCK / 64];
     const DevScene& sc = *scene;
     const CursorMap pmap{wp};
     const ShadeConst c0 = shade_const(wp, sc);
-    shade_open(
+    shade_open<BLOCK>(
         *count_in, hits, qout, counts_out, sq, append_lds, list, wave_hits,
         [&](uint32_t i) {
             ShadeOut o;
@@ -1113,7 +1115,7 @@ struct ItemMap {
 // The shade step of a unified batch: each entry with its item's parameters
 // and scene (unguided).
 template <bool NMAP>
-__global__ __launch_bounds__(SHADE_BLOCK, NMAP ? 1 : 4) void k_shade_multi(MultiBatch mb, PathQueue qin,
+__global__ __launch_bounds__(shade_block(false, NMAP), NMAP ? 1 : 4) void k_shade_multi(MultiBatch mb, PathQueue qin,
                                                              const uint32_t* __restrict__ count_in,
                                                              const float4* __restrict__ hits, PathQueue qout,
                                                              unsigned long long* __restrict__ counts_out, ShadowQueue sq,
@@ -1121,7 +1123,8 @@ __global__ __launch_bounds__(SHADE_BLOCK, NMAP ? 1 : 4) void k_shade_multi(Multi
     const uint32_t n = *count_in;
     const uint64_t g0 = mb.cursor->g0;
     const uint32_t stride = gridDim.x * blockDim.x;
-    __shared__ uint32_t append_lds[2 * (SHADE_BLOCK / 64) + 2];
+    constexpr int BLOCK = shade_block(false, NMAP);
+    __shared__ uint32_t append_lds[2 * (BLOCK / 64) + 2];
     const GuideRender gr{};
     for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += stride) {
         const uint32_t i = base + threadIdx.x;
@@ -1132,19 +1135,20 @@ __global__ __launch_bounds__(SHADE_BLOCK, NMAP ? 1 : 4) void k_shade_multi(Multi
             shade_entry<false, NMAP, false>(it.wp, sc, shade_const(it.wp, sc), qin, hits, radiance, pending, gr, i,
                                      ItemMap{it, g0}, o);
         }
-        shade_emit<false>(o, qout, counts_out, sq, gr, append_lds);
+        shade_emit<false, BLOCK>(o, qout, counts_out, sq, gr, append_lds);
     }
 }
 template <bool NMAP>
-__global__ __launch_bounds__(SHADE_BLOCK, NMAP ? 1 : 4) void k_shade_multi_open(MultiBatch mb, PathQueue qin,
+__global__ __launch_bounds__(shade_block(false, NMAP), NMAP ? 1 : 4) void k_shade_multi_open(MultiBatch mb, PathQueue qin,
                                                              const uint32_t* __restrict__ count_in,
                                                              const float4* __restrict__ hits, PathQueue qout,
                                                              unsigned long long* __restrict__ counts_out, ShadowQueue sq,
                                                              float4* __restrict__ radiance, float4* __restrict__ pending) {
-    __shared__ uint32_t append_lds[2 * (SHADE_BLOCK / 64) + 2], list[2 * SHADE_BLOCK], wave_hits[SHADE_BLOCK / 64];
+    constexpr int BLOCK = shade_block(false, NMAP);
+    __shared__ uint32_t append_lds[2 * (BLOCK / 64) + 2], list[2 * BLOCK], wave_hits[BLOCK / 64];
     const uint64_t g0 = mb.cursor->g0;
     const GuideRender gr{};
-    shade_open(
+    shade_open<BLOCK>(
         *count_in, hits, qout, counts_out, sq, append_lds, list, wave_hits,
         [&](uint32_t i) {
             const MultiItem& it = mb.items[mb.item_of[__float_as_uint(qin.d[i].w)]];

@@ -744,6 +744,12 @@ static uint32_t trace_blocks(const xt_scene* s, size_t n) {
     return (uint32_t)std::max<size_t>(1, std::min<size_t>(b, s->trace_grid));
 }
 
+// Blocks of `block` threads for n queue entries: no more threads than `grid`
+// blocks of SHADE_BLOCK.
+static uint32_t shade_blocks_for(uint64_t n, uint32_t grid, uint32_t block) {
+    return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((n + block - 1) / block, (uint64_t)grid * SHADE_BLOCK / block));
+}
+
 // Most paths that k_walk follows from their camera rays.
 static uint32_t walk_max(const xt_scene* s, int max_depth) {
     return s->ds.env.has_sky || max_depth <= 0 ? WALK_MAX_SHORT_ROUNDS : WALK_MAX;
@@ -1319,9 +1325,9 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
     hipEvent_t t_begin = tm.mark();
     const uint32_t gblocks_max = (uint32_t)s->dev->num_cu * 8;
     auto blocks256 = [&](uint64_t n) { return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((n + 255) / 256, gblocks_max)); };
-    const uint32_t shade_max = s->shade_grid;
+    const uint32_t shade_max = s->shade_grid, sblock = shade_block(guide, s->nmap);
     auto shade_blocks = [&](uint64_t n) {
-        return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((n + SHADE_BLOCK - 1) / SHADE_BLOCK, shade_max));
+        return shade_blocks_for(n, shade_max, sblock);
     };
     // batches: S samples of a pixel range, S * pixels <= capacity
     const uint32_t S = npix_all <= cap ? (uint32_t)std::min<uint64_t>(cap / npix_all, p->spp) : 1u;
@@ -1490,7 +1496,7 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                         }
                     }
                     a = tm.mark();
-                    hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags, camera && round == 0, !s->counting && s->ds.env.has_sky), dim3(shade_blocks(bound)), dim3(SHADE_BLOCK), 0,
+                    hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags, camera && round == 0, !s->counting && s->ds.env.has_sky), dim3(shade_blocks(bound)), dim3(sblock), 0,
                                        s->stream, wp, s->d_ds, rb.q[cur], path_count(rb.counts, cur), rb.hits, rb.q[1 - cur],
                                        pair_count(rb.counts, 1 - cur), rb.sq, rb.radiance, rb.pending, gr);
                     XT_LAUNCHED(result);
@@ -1721,8 +1727,8 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
     const uint32_t jblocks = std::min(trace_blocks(s, 2 * (size_t)maxpaths), tmost);   // launches of two queues
     const uint32_t gblocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((maxpaths + 255) / 256, (uint64_t)s->dev->num_cu * 8));
     const uint32_t ablocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((plan.pix_chunk + 255) / 256, (uint64_t)s->dev->num_cu * 8));
-    const uint32_t sblocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((maxpaths + SHADE_BLOCK - 1) / SHADE_BLOCK, s->shade_grid));
     const bool guide = gd.lobes_mk != nullptr;
+    const uint32_t sblock = shade_block(guide, s->nmap), sblocks = shade_blocks_for(maxpaths, s->shade_grid, sblock);
     GuideState& g = s->guide;
     const uint32_t ib = std::max(1u, std::min((maxpaths + GI_BLOCK - 1) / GI_BLOCK, (uint32_t)s->dev->num_cu * 4));
     const bool whole = !guide && maxpaths <= walk_max(s, p->max_depth);   // each path in one launch
@@ -1763,7 +1769,7 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
             gr.prob = g.cfg.guide_prob;
             gr.max_vertex = g.cfg.max_guided_vertex;
         }
-        hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags, it == 0 && !guide, s->ds.env.has_sky), dim3(sblocks), dim3(SHADE_BLOCK), 0, s->stream, wp, s->d_ds,
+        hipLaunchKernelGGL(shade_kernel(guide, s->nmap, p->flags, it == 0 && !guide, s->ds.env.has_sky), dim3(sblocks), dim3(sblock), 0, s->stream, wp, s->d_ds,
                            b.q[cur], path_count(b.counts, cur), b.hits, b.q[1 - cur], pair_count(b.counts, 1 - cur), b.sq,
                            b.radiance, b.pending, gr);
         cur = 1 - cur;
@@ -2069,7 +2075,7 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
     mb.units = m.units;
     const uint32_t ncu = (uint32_t)dev->num_cu;
     const uint32_t gblocks = std::max(1u, std::min((window + 255u) / 256u, ncu * 8));
-    const uint32_t sblocks = std::max(1u, std::min((window + SHADE_BLOCK - 1) / SHADE_BLOCK, s0->shade_grid));
+    const uint32_t sblock = shade_block(false, nmap), sblocks = shade_blocks_for(window, s0->shade_grid, sblock);
     // capture one window's bounce loop (windows of many paths hand the
     // traversal kernels' rays out in chunks from a cursor)
     const bool dyn = window >= TRAV_DYN_MIN;
@@ -2102,7 +2108,7 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
                                m.ovf, m.dyn, nullptr, m.item_of, m.items);
         auto shade = open && it > 0 ? (nmap ? k_shade_multi_open<true> : k_shade_multi_open<false>)
                                     : (nmap ? k_shade_multi<true> : k_shade_multi<false>);
-        hipLaunchKernelGGL(shade, dim3(sblocks), dim3(SHADE_BLOCK), 0, m.stream, mb, m.q[cur], path_count(m.counts, cur), m.hits,
+        hipLaunchKernelGGL(shade, dim3(sblocks), dim3(sblock), 0, m.stream, mb, m.q[cur], path_count(m.counts, cur), m.hits,
                            m.q[1 - cur], pair_count(m.counts, 1 - cur), m.sq, m.radiance, m.pending);
         cur = 1 - cur;
     }
