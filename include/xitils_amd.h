@@ -161,7 +161,8 @@ typedef struct xt_render_params {
     uint32_t width, height;
     uint32_t spp;            /* samples per pixel in this call */
     uint32_t spp_offset;     /* index of the first sample (progressive rendering) */
-    int32_t max_depth;       /* bounce cap; <= 0: unbounded, roulette only (as the reference) */
+    int32_t max_depth;       /* bounce cap; <= 0: none, roulette only (as the reference), and XT_ERR_DEVICE
+                              * when a path goes on past 65,534 vertices */
     uint32_t seed;           /* Philox key word 0 */
     uint32_t stream;         /* Philox key word 1 */
     uint32_t integrator;     /* XT_INTEGRATOR_* */

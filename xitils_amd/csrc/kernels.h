@@ -228,8 +228,10 @@ struct WalkArgs {
     uint32_t lanes;                 // rays a wave keeps in flight (1..64)
     uint32_t* ovf;                  // traversal spill columns
     uint32_t* dyn;                  // chunk cursor and block counter, zero between launches
+    uint32_t max_vertex = 0xFFFFFFFFu;   // a path that goes on past it is left there and sets *overrun
+    uint32_t* overrun;              // null: the depth cap ends every path
     unsigned long long* rays;       // null, or running totals of extension and shadow rays
-    unsigned long long* rays_out;   // where the launch leaves them (mapped host memory)
+    unsigned long long* rays_out;   // where the launch leaves them, and *overrun (mapped host memory)
 };
 // waves per SIMD of k_walk (at 3 instead of 4, with no spill instead of 28
 // registers', it measured the same; the normal-mapping form needs 256 VGPRs)
@@ -281,7 +283,7 @@ template <bool COUNT, bool DYN = false>
 __global__ void k_shadow(DevScene sc, ShadowQueue sq, const uint32_t* count, float4* radiance, float4* pending,
                          uint32_t* ovf, uint32_t* dyn, unsigned long long* visit_totals, const uint32_t* counts4,
                          uint32_t* counts_out);
-__global__ void k_accumulate(WaveParams wp, const float4* radiance, void* film, int film_f64);
+__global__ void k_accumulate(WaveParams wp, const float4* radiance, void* film, int film_f64, const uint32_t* overrun);
 __global__ void k_zero_u32(uint32_t* p, uint32_t n);
 constexpr int VALU_PROBE_CHAINS = 16;   // FMA chains per lane of k_valu_probe
 __global__ void k_valu_probe(uint32_t iters, float* out);

@@ -940,9 +940,12 @@ XT_INST_SHADOW(false, true)
 XT_INST_SHADOW(true, true)
 #undef XT_INST_SHADOW
 
-// film[pixel] += radiance of each of the batch's samples, in sample order.
+// film[pixel] += radiance of each of the batch's samples, in sample order
+// (overrun: null, or set when paths of the batch were left unfinished, and the
+// film then stays as it is).
 __global__ __launch_bounds__(256) void k_accumulate(WaveParams wp, const float4* __restrict__ radiance, void* film,
-                                                    int film_f64) {
+                                                    int film_f64, const uint32_t* __restrict__ overrun) {
+    if (overrun && *overrun) return;
     const BatchCursor bc = batch_of(wp);
     const uint32_t np = bc.num_pixels, S = bc.num_paths / bc.num_pixels;
     for (uint32_t p = blockIdx.x * blockDim.x + threadIdx.x; p < np; p += gridDim.x * blockDim.x) {
@@ -1388,7 +1391,8 @@ __global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) v
     if (threadIdx.x < 2) counted[threadIdx.x] = 0u;
     if constexpr (!MULTI) stage_top_nodes(top, *a.scene);
     __syncthreads();
-    const uint32_t n = QUEUE ? *a.count : MULTI ? mb.cursor->n : batch_of(wp0).num_paths;
+    uint32_t n = QUEUE ? *a.count : MULTI ? mb.cursor->n : batch_of(wp0).num_paths;
+    if (a.overrun && *a.overrun) n = 0u;   // the render has failed
     const size_t nthreads = (size_t)gridDim.x * blockDim.x;
     const size_t gtid = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint32_t* my_lds = lds + threadIdx.x;
@@ -1599,6 +1603,12 @@ __global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) v
             so = o.sh_o;
             sd = o.sh_d;
             stmax = o.sh_tmax;
+            if (has_ext && v > a.max_vertex) {
+                // the render fails, and no wave takes another chunk
+                atomicOr(a.overrun, 1u);
+                atomicMax(&a.dyn[0], ch.n);
+                has_ext = has_sh = false;
+            }
             if (!has_ext && !has_sh) {
                 a.radiance[id] = f4(rad, 0.0f);
                 alive = false;
@@ -1629,6 +1639,7 @@ __global__ __launch_bounds__(TRACE_BLOCK, NMAP ? WALK_WAVES_NMAP : WALK_WAVES) v
             if (a.rays) {
                 a.rays_out[0] = atomicAdd(&a.rays[0], 0ull);
                 a.rays_out[1] = atomicAdd(&a.rays[1], 0ull);
+                a.rays_out[2] = a.overrun ? atomicOr(a.overrun, 0u) : 0u;
             }
         }
     }

@@ -35,6 +35,11 @@ xt_status xt_fail(xt_status s, const std::string& msg) {
 static xt_status fail(xt_status s, const std::string& msg) { return xt_fail(s, msg); }
 
 constexpr int RB_RING = 4;   // bounce rounds whose queue counts can be in flight to the host
+// Bounce rounds of a render without a depth cap.  The host reads counts `lag`
+// rounds late, so a path fails the render when it goes on past vertex
+// ROUNDS_MAX - lag, in the rounds and in k_walk alike.
+constexpr int ROUNDS_MAX = 1 << 16;
+constexpr const char* NOT_DRAINED = "bounce loop did not drain its queue";
 
 struct RenderBuffers {
     uint32_t capacity = 0;
@@ -52,9 +57,10 @@ struct RenderBuffers {
     unsigned long long* visits = nullptr;  // node, tri fetches: extension [0..1], shadow [2..3]
     uint32_t* dyn = nullptr;               // chunk cursors of the traversal kernels: extension [0..1], shadow [2..3]
     unsigned long long* rays = nullptr;    // extension and shadow rays traced by k_walk, ever
-    unsigned long long* host_rays = nullptr;      // its last totals (pinned, behind host_counts)
+    unsigned long long* host_rays = nullptr;      // its last totals, and *overrun (pinned, behind host_counts)
     unsigned long long* host_rays_dev = nullptr;
     unsigned long long rays_seen[2] = {0, 0};     // totals already in some render's stats
+    uint32_t* overrun = nullptr;           // set by k_walk: paths were left unfinished (behind rays; zero between renders)
     void release() {
         for (int k = 0; k < 2; ++k) {
             hipFree(q[k].o); hipFree(q[k].d); hipFree(q[k].w); hipFree(q[k].e);
@@ -933,16 +939,17 @@ static xt_status alloc_buffers(RenderBuffers& rb, uint32_t capacity) {
     XT_HIP(dalloc(&rb.visits, 4));
     XT_HIP(dalloc(&rb.dyn, 4));
     XT_HIP(hipMemset(rb.dyn, 0, 4 * sizeof(uint32_t)));
-    XT_HIP(dalloc(&rb.rays, 2));
-    XT_HIP(hipMemset(rb.rays, 0, 2 * sizeof(unsigned long long)));
+    XT_HIP(dalloc(&rb.rays, 3));
+    rb.overrun = (uint32_t*)(rb.rays + 2);
+    XT_HIP(hipMemset(rb.rays, 0, 3 * sizeof(unsigned long long)));
     XT_HIP(hipStreamSynchronize(nullptr));   // the scenes' streams do not wait for the default stream
     constexpr size_t ring_words = RB_RING * 4;
-    XT_HIP(hipHostMalloc((void**)&rb.host_counts, ring_words * sizeof(uint32_t) + 2 * sizeof(unsigned long long),
+    XT_HIP(hipHostMalloc((void**)&rb.host_counts, ring_words * sizeof(uint32_t) + 3 * sizeof(unsigned long long),
                          hipHostMallocMapped | hipHostMallocCoherent));
     XT_HIP(hipHostGetDevicePointer((void**)&rb.host_counts_dev, rb.host_counts, 0));
     rb.host_rays = (unsigned long long*)(rb.host_counts + ring_words);
     rb.host_rays_dev = (unsigned long long*)(rb.host_counts_dev + ring_words);
-    rb.host_rays[0] = rb.host_rays[1] = 0;
+    rb.host_rays[0] = rb.host_rays[1] = rb.host_rays[2] = 0;
     for (hipEvent_t& e : rb.round_ev) XT_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     rb.capacity = capacity;
     return XT_OK;
@@ -1357,6 +1364,7 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
             }
             hipEvent_t a = tm.mark();
             s->stats.camera_rays += wp.num_paths;
+            const int lag = train ? 0 : 2;   // of the host behind the bounce rounds, below
             // the rest of the batch in one launch: at most n paths, of the
             // queue `q` or (q < 0) from their camera rays
             auto walk = [&](int q, uint64_t n) {
@@ -1374,6 +1382,10 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                 wa.dyn = rb.dyn;
                 wa.rays = rb.rays;
                 wa.rays_out = rb.host_rays_dev;
+                if (p->max_depth <= 0) {
+                    wa.max_vertex = ROUNDS_MAX - lag;
+                    wa.overrun = rb.overrun;
+                }
                 auto kernel = s->nmap ? (q >= 0 ? k_walk<true, true, false> : k_walk<false, true, false>)
                                       : (q >= 0 ? k_walk<true, false, false> : k_walk<false, false, false>);
                 hipEvent_t w = tm.mark();
@@ -1383,10 +1395,12 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                 tm.add(0, w, tm.mark());
                 s->stats.extend_launches++;
             };
-            const bool can_walk = !guide && !s->counting;
             // the first round makes its rays itself, unless the network reads
             // their queue or fetches are counted
             const bool camera = !guide && !s->counting;
+            // one launch follows a path for at most 64 Ki vertices (0.7 s between two
+            // mirrors, 2 s at the 31 us a vertex of the material zoo)
+            const bool can_walk = camera && p->max_depth <= ROUNDS_MAX;
             const bool whole = can_walk && wp.num_paths <= walk_max(s, p->max_depth);
             if (whole) {
                 walk(-1, wp.num_paths);
@@ -1406,7 +1420,6 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
             // and one shadow ray per round).  Rounds launched after the queue
             // ran empty exit at once.  Training renders read each round's
             // counts before the next (the record offsets must be exact).
-            const int lag = train ? 0 : 2;
             uint32_t bound = wp.num_paths;         // >= every queue length from here on
             uint32_t queue_len[RB_RING];           // queue length of each unverified round
             int round = 0, verified = 0, cur = 0;
@@ -1432,12 +1445,12 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                 if (hipEventRecord(rb.round_ev[slot], s->stream) != hipSuccess) result = fail(XT_ERR_DEVICE, "hipEventRecord failed");
             };
             // a path adds one extension ray per round, so max_depth + 1 rounds hold every live queue
-            const int max_rounds = p->max_depth > 0 ? p->max_depth + 2 + lag : (1 << 16);
+            const int max_rounds = p->max_depth > 0 ? p->max_depth + 2 + lag : ROUNDS_MAX;
             // Once a read count is zero every later round is empty: the host
             // moves on (accumulate, next batch) without waiting for them.
             while (result == XT_OK && launch) {
                 if (round >= max_rounds) {
-                    result = fail(XT_ERR_DEVICE, "bounce loop did not drain its queue");
+                    result = fail(XT_ERR_DEVICE, NOT_DRAINED);
                     break;
                 }
                 {
@@ -1551,7 +1564,8 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                 break;
             }
             a = tm.mark();
-            hipLaunchKernelGGL(k_accumulate, dim3(blocks256(np)), dim3(256), 0, s->stream, wp, rb.radiance, d_film, film_f64);
+            hipLaunchKernelGGL(k_accumulate, dim3(blocks256(np)), dim3(256), 0, s->stream, wp, rb.radiance, d_film, film_f64,
+                               rb.overrun);
             XT_LAUNCHED(result);
             tm.add(3, a, tm.mark());
             if (train && rec_base > 0 && result == XT_OK) {
@@ -1607,6 +1621,12 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
     hipError_t e = hipStreamSynchronize(s->stream);
     if (result == XT_OK && e != hipSuccess) result = fail(XT_ERR_DEVICE, std::string("render failed: ") + hipGetErrorString(e));
     if (result == XT_OK && hipGetLastError() != hipSuccess) result = fail(XT_ERR_DEVICE, "kernel launch failed");
+    if (rb.host_rays[2] != 0) {   // k_walk met max_vertex
+        rb.host_rays[2] = 0;
+        hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s->stream, rb.overrun, 1u);
+        hipStreamSynchronize(s->stream);
+        if (result == XT_OK) result = fail(XT_ERR_DEVICE, NOT_DRAINED);
+    }
     if (result == XT_OK) {
         float ms = 0;
         hipEventElapsedTime(&ms, t_begin, t_end);
@@ -1777,7 +1797,8 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
     if (!whole)
         hipLaunchKernelGGL(k_shadow<false>, dim3(tblocks), dim3(TRACE_BLOCK), 0, s->stream, s->ds, b.sq, shadow_count(b.counts, cur),
                            b.radiance, b.pending, b.ovf, nullptr, nullptr, b.counts, nullptr);
-    hipLaunchKernelGGL(k_accumulate, dim3(ablocks), dim3(256), 0, s->stream, wp, b.radiance, d_film, f64);
+    hipLaunchKernelGGL(k_accumulate, dim3(ablocks), dim3(256), 0, s->stream, wp, b.radiance, d_film, f64,
+                       (const uint32_t*)nullptr);
     hipLaunchKernelGGL(k_advance_cursor, dim3(1), dim3(1), 0, s->stream, cursor, plan);
 }
 
