@@ -87,3 +87,13 @@ def test_depth_cap_above_the_limit():
     film = np.full((h, w, 3), 3.0, np.float32)
     assert _render(sc, w, h, film, _kw(LAST + 100, max_depth=70000)) is None
     assert sc.stats()["extension_rays"] == w * h * (LAST + 100) and np.all(film == 3.0)
+
+
+def test_ray_counts_after_a_failed_render():
+    """The rays of the failed render are not counted again by the next one."""
+    w, h = 8, 4
+    sc = _mirrors(w, h, 2e-6)
+    print("[gpu] path limit: ray counts after a failed render", flush=True)
+    assert _render(sc, w, h, np.zeros((h, w, 3), np.float32), _kw(LAST + 1)) is not None
+    sc.render(w, h, 1, **_kw(100))
+    assert sc.stats()["extension_rays"] == w * h * 100

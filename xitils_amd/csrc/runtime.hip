@@ -1621,6 +1621,10 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
     hipError_t e = hipStreamSynchronize(s->stream);
     if (result == XT_OK && e != hipSuccess) result = fail(XT_ERR_DEVICE, std::string("render failed: ") + hipGetErrorString(e));
     if (result == XT_OK && hipGetLastError() != hipSuccess) result = fail(XT_ERR_DEVICE, "kernel launch failed");
+    // the rays walked, also by a render that fails: the next one's start here
+    s->stats.extension_rays += rb.host_rays[0] - rb.rays_seen[0];
+    s->stats.shadow_rays += rb.host_rays[1] - rb.rays_seen[1];
+    for (int k = 0; k < 2; ++k) rb.rays_seen[k] = rb.host_rays[k];
     if (rb.host_rays[2] != 0) {   // k_walk met max_vertex
         rb.host_rays[2] = 0;
         hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, s->stream, rb.overrun, 1u);
@@ -1630,9 +1634,6 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
     if (result == XT_OK) {
         float ms = 0;
         hipEventElapsedTime(&ms, t_begin, t_end);
-        s->stats.extension_rays += rb.host_rays[0] - rb.rays_seen[0];
-        s->stats.shadow_rays += rb.host_rays[1] - rb.rays_seen[1];
-        for (int k = 0; k < 2; ++k) rb.rays_seen[k] = rb.host_rays[k];
         s->stats.ms_total = ms;
         s->stats.ms_extend = tm.total(0);
         s->stats.ms_shade = tm.total(1);
