@@ -1990,7 +1990,8 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
         XT_HIP(dalloc(&dev->multi->counts, 4));
         XT_HIP(dalloc(&dev->multi->cursor, 1));
         XT_HIP(dalloc(&dev->multi->dyn, 4));
-        XT_HIP(hipMemset(dev->multi->dyn, 0, 4 * sizeof(uint32_t)));
+        // on the batch's own stream, which does not wait for the default stream
+        XT_HIP(hipMemsetAsync(dev->multi->dyn, 0, 4 * sizeof(uint32_t), dev->multi->stream));
     }
     MultiState& m = *dev->multi;
     // item and scene tables (items without samples are left out)
