@@ -299,7 +299,8 @@ xt_status xt_render_static(xt_scene* scene, const xt_camera* camera, const xt_re
                            int film_is_f64);
 /* Autotuner: renders one batch of (camera, params) as a graph under 9
  * launch shapes and keeps the fastest for this scene's later renders;
- * out = {traversal blocks per CU, shade blocks per CU}. */
+ * out = {traversal blocks per CU, shade blocks per CU}.  A batch small enough
+ * to follow its paths in one launch has no shape and leaves the scene's. */
 xt_status xt_scene_autotune(xt_scene* scene, const xt_camera* camera, const xt_render_params* params, uint32_t out[2]);
 
 /* Measurement hook (no reference counterpart): renders and ray queries of

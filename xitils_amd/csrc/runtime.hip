@@ -1730,6 +1730,11 @@ static BatchPlan cursor_plan(const xt_render_params* p, uint32_t cap, uint32_t* 
     return plan;
 }
 
+// Whether a count-driven batch of up to maxpaths paths follows each in one launch.
+static bool batch_walked(const xt_scene* s, const xt_render_params* p, uint32_t maxpaths) {
+    return !(p->flags & XT_FLAG_GUIDE) && maxpaths <= walk_max(s, p->max_depth);
+}
+
 // Guide inputs of a count-driven batch (lobes_mk == nullptr: unguided).
 struct BounceGuide {
     uint2* lobes_mk = nullptr;
@@ -1752,7 +1757,7 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
     const uint32_t sblock = shade_block(guide, s->nmap), sblocks = shade_blocks_for(maxpaths, s->shade_grid, sblock);
     GuideState& g = s->guide;
     const uint32_t ib = std::max(1u, std::min((maxpaths + GI_BLOCK - 1) / GI_BLOCK, (uint32_t)s->dev->num_cu * 4));
-    const bool whole = !guide && maxpaths <= walk_max(s, p->max_depth);   // each path in one launch
+    const bool whole = batch_walked(s, p, maxpaths);
     if (whole) {
         WalkArgs wa{};
         wa.wp = wp;
@@ -2467,7 +2472,9 @@ xt_status xt_render_static(xt_scene* s, const xt_camera* cam, const xt_render_pa
 
 
 // Times the graph-replayed render of one batch for a few launch shapes and
-// keeps the fastest (traversal blocks per CU x shade blocks per CU).
+// keeps the fastest (traversal blocks per CU x shade blocks per CU).  A batch
+// whose paths are followed in one launch has neither shape: it keeps the
+// scene's, which its larger renders and its ray queries use.
 xt_status xt_scene_autotune(xt_scene* s, const xt_camera* cam, const xt_render_params* p, uint32_t out[2]) {
     xt_render_params q = *p;
     xt_status st = check_render_args(s, cam, &q);
@@ -2476,9 +2483,18 @@ xt_status xt_scene_autotune(xt_scene* s, const xt_camera* cam, const xt_render_p
     const uint64_t npix = (uint64_t)q.width * q.height;
     const uint32_t cap = graph_capacity(npix, std::max(1u, q.spp));
     q.spp = std::max(1u, (uint32_t)std::min<uint64_t>(std::max<uint64_t>(cap / npix, 1), std::max(1u, p->spp)));
+    const uint32_t ncu = (uint32_t)s->dev->num_cu;
+    uint32_t nbatches = 0;
+    const BatchPlan plan = cursor_plan(&q, cap, &nbatches);
+    if (batch_walked(s, &q, plan.pix_chunk * plan.S)) {
+        if (out) {
+            out[0] = s->trace_grid / ncu;
+            out[1] = s->shade_grid / ncu;
+        }
+        return XT_OK;
+    }
     void* d_film = nullptr;
     XT_HIP(hipMalloc(&d_film, npix * 3 * sizeof(float)));
-    const uint32_t ncu = (uint32_t)s->dev->num_cu;
     const uint32_t tcand[3] = {2, 4, 8}, scand[3] = {2, 4, 8};
     float best = INFINITY;
     uint32_t bt = s->trace_grid, bs = s->shade_grid;
