@@ -211,7 +211,7 @@ extern "C" {
 const char* xt_version(void) { return "xitils_amd 0.1.0 (gfx950, BVH" XT_STR(XT_BVH_WIDTH) " wavefront)"; }
 const char* xt_last_error(void) { return g_last_error.c_str(); }
 
-// Static scratch of xt_render_static: every buffer of its bounce loop is
+// Static scratch of xt_render_static: every buffer of its batches is
 // carved from this array, so that entry point allocates nothing.  Each GPU
 // the library runs on holds its own copy from code-object load until the
 // process ends.  In host code `scratch` names a host-side stand-in, not
@@ -1682,8 +1682,9 @@ static uint32_t graph_capacity(uint64_t npix, uint32_t spp) {
     return (uint32_t)std::min<uint64_t>(std::min<uint32_t>(path_capacity(), 1u << 22), npix * spp);
 }
 
-// Path state of one count-driven batch (the graph renders' buffers, or the
-// static scratch of xt_render_static).
+// Path state of one count-driven batch: the graph renders' buffers, or the
+// static scratch of xt_render_static, whose walked batches need no more than
+// radiance, ovf and dyn.
 struct BounceBufs {
     PathQueue q[2];
     ShadowQueue sq;
@@ -2399,11 +2400,13 @@ xt_status xt_render_batch(xt_batch_item* items, uint32_t n) {
 // ---------------------------------------------------------------- render without allocation
 
 // xt_render_static's carving of the static scratch: a 256-byte header (batch
-// cursor at 0, queue counters at 64), at most 16 MiB of traversal spill
-// columns, then 14 float4 arrays of `capacity` paths (224 bytes per path).
+// cursor at 0, k_walk's chunk cursor and block counter at 128), at most 16 MiB
+// of traversal spill columns, then the radiance of a batch's paths, all that
+// k_walk keeps of them in memory.  Batches are no larger than it takes.
 constexpr size_t STATIC_HEADER = 256;
 constexpr size_t STATIC_SPILL_MAX = (size_t)16 << 20;
-constexpr size_t STATIC_PATH_BYTES = 14 * sizeof(float4);
+static_assert(XT_STATIC_SCRATCH_BYTES - STATIC_HEADER - STATIC_SPILL_MAX >= WALK_MAX_SHORT_ROUNDS * sizeof(float4),
+              "the largest walked batch fits");
 
 xt_status xt_render_static(xt_scene* s, const xt_camera* cam, const xt_render_params* p, void* film, int film_f64) {
     xt_status st = check_render_args(s, cam, p);
@@ -2426,38 +2429,25 @@ xt_status xt_render_static(xt_scene* s, const xt_camera* cam, const xt_render_pa
                                           " spill entries per lane) exceeds the static scratch");
     const size_t spill_bytes = ((per_block * tcap + 255) / 256) * 256;
     const uint64_t npix = (uint64_t)p->width * p->height;
-    const uint64_t fit = (XT_STATIC_SCRATCH_BYTES - STATIC_HEADER - spill_bytes) / STATIC_PATH_BYTES;
-    const uint32_t cap = (uint32_t)std::min<uint64_t>(fit, npix * p->spp);
+    // as few batches as the walk allows, of even sizes: a batch takes as long as
+    // its slowest paths (256 x 256 x 16 of the Cornell box in 4, 4, 4 and 4 samples
+    // 2.0 ms, in 5, 5, 5 and 1 2.5)
+    const uint32_t most = walk_max(s, p->max_depth);
+    auto even = [](uint64_t n, uint64_t at_most) {
+        const uint64_t parts = (n + at_most - 1) / at_most;
+        return (n + parts - 1) / parts;
+    };
+    const uint32_t cap = (uint32_t)(npix <= most ? npix * even(p->spp, most / npix) : even(npix, most));
     BatchCursor* cursor = (BatchCursor*)base;
     BounceBufs b{};
-    b.counts = (uint32_t*)(base + 64);
     b.dyn = (uint32_t*)(base + 128);
     b.ovf = per_block ? (uint32_t*)(base + STATIC_HEADER) : nullptr;
     b.capacity = cap;
-    float4* arr = (float4*)(base + STATIC_HEADER + spill_bytes);
-    auto take = [&]() {
-        float4* r = arr;
-        arr += cap;
-        return r;
-    };
-    for (int k = 0; k < 2; ++k) {
-        b.q[k].o = take();
-        b.q[k].d = take();
-        b.q[k].w = take();
-        b.q[k].e = take();
-        b.q[k].rec = nullptr;
-    }
-    b.sq.o = take();
-    b.sq.d = take();
-    b.sq.c = take();
-    b.hits = take();
-    b.radiance = take();
-    b.pending = take();
+    b.radiance = (float4*)(base + STATIC_HEADER + spill_bytes);
     uint32_t nbatches = 0;
     const BatchPlan plan = cursor_plan(p, cap, &nbatches);
     const WaveParams wp = cursor_wave_params(cam, p, cursor);
-    // the cursor is written by k_cursor_init and the counters by the kernels
-    // (k_count_from_cursor, k_trace), so nothing needs clearing beforehand
+    // k_cursor_init writes the batch cursor and clears k_walk's
     hipLaunchKernelGGL(k_cursor_init, dim3(1), dim3(1), 0, s->stream, cursor, plan, b.dyn);
     for (uint32_t k = 0; k < nbatches; ++k)
         enqueue_cursor_batch(s, p, wp, b, plan, cursor, tcap, BounceGuide{}, film, film_f64);
