@@ -233,10 +233,9 @@ xt_status xt_device_open(int ordinal, xt_device** out) {
     void* scratch_ptr = nullptr;   // this device's copy of the static scratch (the device is current)
     XT_HIP(hipGetSymbolAddress(&scratch_ptr, HIP_SYMBOL(scratch)));
     if (!scratch_ptr) return fail(XT_ERR_DEVICE, "hipGetSymbolAddress returned no address for the static scratch");
-    xt_device* d = new (std::nothrow) xt_device();
+    xt_device* d = new (std::nothrow) xt_device(ordinal);
     if (!d) return fail(XT_ERR_OUT_OF_MEMORY, "host allocation failed");
     d->scratch = (unsigned char*)scratch_ptr;
-    d->ordinal = ordinal;
     d->num_cu = prop.multiProcessorCount;
     d->arch = arch;
     *out = d;
@@ -2241,7 +2240,7 @@ xt_status xt_render_batch(xt_batch_item* items, uint32_t n) {
                 d_films[i] = d_films[j];
                 continue;
             }
-            if (hipMalloc(&q.d_film, q.bytes) != hipSuccess) {
+            if (device_malloc(&q.d_film, q.bytes) != hipSuccess) {
                 result = fail(XT_ERR_OUT_OF_MEMORY, "film allocation failed");
                 break;
             }
@@ -2484,7 +2483,7 @@ xt_status xt_scene_autotune(xt_scene* s, const xt_camera* cam, const xt_render_p
         return XT_OK;
     }
     void* d_film = nullptr;
-    XT_HIP(hipMalloc(&d_film, npix * 3 * sizeof(float)));
+    XT_HIP(device_malloc(&d_film, npix * 3 * sizeof(float)));
     const uint32_t tcand[3] = {2, 4, 8}, scand[3] = {2, 4, 8};
     float best = INFINITY;
     uint32_t bt = s->trace_grid, bs = s->shade_grid;
@@ -2605,7 +2604,7 @@ xt_status xt_guide_init(xt_scene* s, const xt_guide_config* cfg) {
         off[k] = total;
         total += (sizes[k] + 255) / 256 * 256;
     }
-    chk(hipMalloc(&g.net_mem, total));
+    chk(device_malloc(&g.net_mem, total));
     chk(hipStreamCreateWithFlags(&g.train_stream, hipStreamNonBlocking));
     for (int k = 0; k < 2; ++k) {
         chk(hipEventCreateWithFlags(&g.pub_ev[k], hipEventDisableTiming));
