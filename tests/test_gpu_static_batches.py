@@ -1,4 +1,4 @@
-"""xt_render_static over several walked batches: even shares of the samples, the
+"""xt_render_static over one and several batches: even shares of the samples, the
 last one smaller, and of the pixels."""
 import numpy as np
 import pytest
@@ -9,7 +9,7 @@ from xitils_amd import api, scenes
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("w,h,spp", [(201, 199, 11), (573, 571, 2), (577, 571, 3), (1201, 1103, 1)])
+@pytest.mark.parametrize("w,h,spp", [(201, 199, 11), (1501, 997, 7), (2311, 2111, 1)]   # one batch; samples; pixels)
 @pytest.mark.parametrize("make", [scenes.cornell, lambda w, h: scenes.heightfield(48, w, h)])
 def test_static_batches_equal_rounds(make, w, h, spp):
     print(f"[gpu] static batches {w}x{h}x{spp}", flush=True)

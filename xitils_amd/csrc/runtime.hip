@@ -1745,9 +1745,10 @@ struct BounceGuide {
 // Enqueues the bounce loop of the cursor's batch on s->stream: generate,
 // max_depth + 1 rounds of extend / (guide) / shade / shadow, accumulate,
 // advance the cursor.  Every kernel reads its queue length from device memory.
+// whole: k_walk in place of the rounds.
 static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const WaveParams& wp, const BounceBufs& b,
                                  const BatchPlan& plan, BatchCursor* cursor, uint32_t tmost,
-                                 const BounceGuide& gd, void* d_film, int f64) {
+                                 const BounceGuide& gd, void* d_film, int f64, bool whole) {
     const uint32_t maxpaths = plan.pix_chunk * plan.S;
     const uint32_t tblocks = std::min(trace_blocks(s, maxpaths), tmost);
     const uint32_t jblocks = std::min(trace_blocks(s, 2 * (size_t)maxpaths), tmost);   // launches of two queues
@@ -1757,7 +1758,6 @@ static void enqueue_cursor_batch(xt_scene* s, const xt_render_params* p, const W
     const uint32_t sblock = shade_block(guide, s->nmap), sblocks = shade_blocks_for(maxpaths, s->shade_grid, sblock);
     GuideState& g = s->guide;
     const uint32_t ib = std::max(1u, std::min((maxpaths + GI_BLOCK - 1) / GI_BLOCK, (uint32_t)s->dev->num_cu * 4));
-    const bool whole = batch_walked(s, p, maxpaths);
     if (whole) {
         WalkArgs wa{};
         wa.wp = wp;
@@ -1834,7 +1834,8 @@ static xt_status capture_graph(xt_scene* s, const xt_camera* cam, const xt_rende
         gd.stride = rb.capacity;
     }
     XT_HIP(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_cursor_batch(s, p, wp, b, plan, s->d_cursor, s->trace_grid_max, gd, d_film, f64);
+    enqueue_cursor_batch(s, p, wp, b, plan, s->d_cursor, s->trace_grid_max, gd, d_film, f64,
+                         batch_walked(s, p, plan.pix_chunk * plan.S));
     hipError_t launch_err = hipGetLastError();
     hipGraph_t graph = nullptr;
     hipError_t e = hipStreamEndCapture(s->stream, &graph);
@@ -2401,11 +2402,9 @@ xt_status xt_render_batch(xt_batch_item* items, uint32_t n) {
 // xt_render_static's carving of the static scratch: a 256-byte header (batch
 // cursor at 0, k_walk's chunk cursor and block counter at 128), at most 16 MiB
 // of traversal spill columns, then the radiance of a batch's paths, all that
-// k_walk keeps of them in memory.  Batches are no larger than it takes.
+// k_walk keeps of them in memory.
 constexpr size_t STATIC_HEADER = 256;
 constexpr size_t STATIC_SPILL_MAX = (size_t)16 << 20;
-static_assert(XT_STATIC_SCRATCH_BYTES - STATIC_HEADER - STATIC_SPILL_MAX >= WALK_MAX_SHORT_ROUNDS * sizeof(float4),
-              "the largest walked batch fits");
 
 xt_status xt_render_static(xt_scene* s, const xt_camera* cam, const xt_render_params* p, void* film, int film_f64) {
     xt_status st = check_render_args(s, cam, p);
@@ -2428,15 +2427,15 @@ xt_status xt_render_static(xt_scene* s, const xt_camera* cam, const xt_render_pa
                                           " spill entries per lane) exceeds the static scratch");
     const size_t spill_bytes = ((per_block * tcap + 255) / 256) * 256;
     const uint64_t npix = (uint64_t)p->width * p->height;
-    // as few batches as the walk allows, of even sizes: a batch takes as long as
-    // its slowest paths (256 x 256 x 16 of the Cornell box in 4, 4, 4 and 4 samples
-    // 2.0 ms, in 5, 5, 5 and 1 2.5)
-    const uint32_t most = walk_max(s, p->max_depth);
+    // as few batches as fit, of even sizes: a batch takes as long as its slowest
+    // paths (256 x 256 x 16 of the Cornell box at once 1.57 ms, in 8 and 8 samples
+    // 1.89, in 4, 4, 4 and 4 2.01, in 5, 5, 5 and 1 2.5)
+    const uint64_t fit = (XT_STATIC_SCRATCH_BYTES - STATIC_HEADER - spill_bytes) / sizeof(float4);
     auto even = [](uint64_t n, uint64_t at_most) {
         const uint64_t parts = (n + at_most - 1) / at_most;
         return (n + parts - 1) / parts;
     };
-    const uint32_t cap = (uint32_t)(npix <= most ? npix * even(p->spp, most / npix) : even(npix, most));
+    const uint32_t cap = (uint32_t)(npix <= fit ? npix * even(p->spp, fit / npix) : even(npix, fit));
     BatchCursor* cursor = (BatchCursor*)base;
     BounceBufs b{};
     b.dyn = (uint32_t*)(base + 128);
@@ -2449,7 +2448,7 @@ xt_status xt_render_static(xt_scene* s, const xt_camera* cam, const xt_render_pa
     // k_cursor_init writes the batch cursor and clears k_walk's
     hipLaunchKernelGGL(k_cursor_init, dim3(1), dim3(1), 0, s->stream, cursor, plan, b.dyn);
     for (uint32_t k = 0; k < nbatches; ++k)
-        enqueue_cursor_batch(s, p, wp, b, plan, cursor, tcap, BounceGuide{}, film, film_f64);
+        enqueue_cursor_batch(s, p, wp, b, plan, cursor, tcap, BounceGuide{}, film, film_f64, true);
     hipError_t le = hipGetLastError();
     hipError_t se = hipStreamSynchronize(s->stream);
     if (le != hipSuccess) return fail(XT_ERR_DEVICE, std::string("xt_render_static launch failed: ") + hipGetErrorString(le));
