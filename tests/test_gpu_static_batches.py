@@ -9,7 +9,8 @@ from xitils_amd import api, scenes
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("w,h,spp", [(201, 199, 11), (1501, 997, 7), (2311, 2111, 1)]   # one batch; samples; pixels)
+# one batch; shares of the samples; of the pixels
+@pytest.mark.parametrize("w,h,spp", [(201, 199, 11), (1501, 997, 7), (2311, 2111, 1)])
 @pytest.mark.parametrize("make", [scenes.cornell, lambda w, h: scenes.heightfield(48, w, h)])
 def test_static_batches_equal_rounds(make, w, h, spp):
     print(f"[gpu] static batches {w}x{h}x{spp}", flush=True)
