@@ -31,7 +31,7 @@ def _counted(sc, w, h, spp, kw):
     return film
 
 
-@pytest.mark.parametrize("w,h,spp", [(641, 513, 1), (823, 797, 1), (641, 383, 5)])   # just above the walked sizes, and more
+@pytest.mark.parametrize("w,h,spp", [(513, 512, 1), (823, 797, 1), (641, 383, 5)])   # just above what is walked, closed and open, and more
 @pytest.mark.parametrize("kind", [*SCENES, "plane"])
 def test_item_graphs_equal_rounds(monkeypatch, kind, w, h, spp):
     monkeypatch.setenv("XITILS_AMD_BATCH", "items")
@@ -48,16 +48,16 @@ def test_item_graphs_equal_rounds(monkeypatch, kind, w, h, spp):
 
 
 def _windows(plane):
-    """Scenes of odd sizes, 250 k to 300 k paths in all."""
+    """Scenes of odd sizes, 200 k to 250 k paths in all."""
     dev, jobs, ref = api.Device(0), [], []
     makes = [*SCENES.values(), PLANE] if plane else list(SCENES.values())
     for k, (make, kw) in enumerate(makes * 2):
-        w, h, spp = 83 + 9 * k, 131 - 9 * k, 3
+        w, h, spp = 75 + 8 * k, 117 - 8 * k, 3
         sc, kw = api.Scene(dev, make(w, h)), {"seed": 5 + k, "max_depth": 7, **kw}
         jobs.append((sc, w, h, spp, None, kw))
         ref.append(_counted(sc, w, h, spp, kw))
     paths = sum(j[1] * j[2] * j[3] for j in jobs)
-    assert (1 << 17) < paths <= 5 << 16
+    assert (1 << 17) < paths <= 1 << 18
     for rep in range(2):
         films, _ = api.render_batch(jobs)
         for a, b in zip(films, ref):

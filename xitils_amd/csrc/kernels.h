@@ -239,16 +239,27 @@ constexpr int WALK_WAVES = 4, WALK_WAVES_NMAP = 2;
 // Most paths of a batch that are walked instead of queued.  A walked path costs
 // the longest of its wave's rays at every vertex, a queued one its share of two
 // launches per round; where a batch has few paths the launches, their gaps and
-// the slowest ray of each cost more.  They cost more again where rounds are
-// short: most paths leave for a sky early, and without a depth cap the last
-// paths go on for many rounds.  Walked against queued, us, 100 k triangle room
-// (depth 16): 769 / 962 at 14 k paths, 1359 / 1540 at 115 k, 2221 / 2334 at
-// 230 k, 3925 / 3267 at 460 k; material zoo 1133 / 1193 at 230 k, 1782 / 1574;
-// Cornell box (depth 8) 560 / 609, 1007 / 861.  Under a sky: 0.5 M triangle
-// field 971 / 1141 at 460 k, 1175 / 1266 at 691 k, 1475 / 1412 at 921 k;
-// normal-mapped plane 1058 / 1251, 1621 / 1522, 1914 / 1763.  Roulette only: zoo
-// 2437 / 2563, 2948 / 2955, 3409 / 3288, room 4375 / 4630 at 230 k, 6390 / 6045.
-constexpr uint32_t WALK_MAX = 5u << 16, WALK_MAX_SHORT_ROUNDS = 10u << 16;
+// the slowest ray of each cost more.  Walked paths are best as many as there are
+// lanes for, 262,144 (131,072 with normal maps, whose lanes then take two each):
+// beyond, waves begin again with full-length paths.  Walked / queued us, at 229 k,
+// 262 k, 328 k paths: 100 k triangle room (depth 16) 2240 / 2425, 2260 / 2410, 3180 /
+// 2840; Cornell box (depth 8) 530 / 587, 537 / 594, 794 / 692; material zoo 861 / 863,
+// 875 / 865, 1180 / 982; 0.5 M triangle canyon under a sky 1450 / 1494, 1529 / 1529,
+// 1930 / 1702; with normal-mapped materials room 3257 / 3273, 3330 / 3340, 4350 /
+// 3440, Cornell box 766 / 803, 774 / 811, 990 / 886.
+// In an open scene (scene_open) most paths leave early, and later ones fill
+// their lanes.  Walked / queued at 328 k, 461 k, 655 k: 0.5 M triangle field 562 /
+// 922, 776 / 993, 970 / 1118, with depth 20 442 / 777, 550 / 821, 660 / 916; object in
+// a lat-long sky 444 / 598, 454 / 617, 533 / 676; normal-mapped plane 785 / 993 at
+// 328 k, 1060 / 1150 at 459 k, 1176 / 1248 at 524 k, 1468 / 1354 at 590 k.
+// Without a depth cap the last paths go on for many rounds: at 328 k, 459 k,
+// 590 k, 655 k Cornell box 1332 / 1350, 1545 / 1573, 1734 / 1752, 1821 / 1884; zoo
+// 2168 / 2235, 2405 / 2544, 2651 / 2810, 2788 / 2916; room 4960 / 5277, 5970 / 6002,
+// 6670 / 6650, 7015 / 6975 (8800 / 8106 at 922 k); with normal-mapped materials Cornell
+// box 1556 / 1582, 1917 / 1744, room 6270 / 6010, 7605 / 6910.
+constexpr uint32_t WALK_MAX = 4u << 16;
+constexpr uint32_t WALK_MAX_OPEN = 10u << 16, WALK_MAX_OPEN_NMAP = 8u << 16;
+constexpr uint32_t WALK_MAX_UNCAPPED = 10u << 16, WALK_MAX_UNCAPPED_NMAP = 5u << 16;
 // Paths of a queue that are walked to their ends instead of queued on: the
 // last rounds of a large batch (material zoo at 460 k paths, us: 1782 from
 // 32 Ki, 1646 from 128 Ki, 1577 from 256 Ki, 1519 from 384 Ki; 100 k triangle

@@ -812,7 +812,8 @@ __global__ __launch_bounds__(shade_block(GUIDE, NMAP), NMAP || (GUIDE && SORT) ?
 // normal-mapped plane's).  1080p field, 132 M paths, 57.5 -> 55.3 ms a frame, its
 // second round 6.1 -> 4.3 ms, now some 3.3 TB/s; plane at 6.2 M paths 8.0 -> 6.8.
 // A first round, whose camera rays miss together, is faster in queue order
-// (plane 6.72 against 6.87 ms).
+// (plane 6.72 against 6.87 ms).  Where nearly every ray hits it costs nothing
+// that shows: 100 k triangle room at 655 k paths 3.70 ms under a sky and without.
 // list: 2 * BLOCK entries, wave_hits: one count per wave.
 template <int BLOCK, class Miss, class Hit>
 __device__ __forceinline__ void shade_open(uint32_t n, const float4* __restrict__ hits, const PathQueue& qout,

@@ -182,6 +182,7 @@ struct xt_scene {
     size_t qout_cap = 0;
     unsigned long long* d_qvisits = nullptr;   // node, tri fetches of the last counted ray query
     uint32_t* d_qdyn = nullptr;                // chunk cursor of the ray-query traversal
+    bool open = false;                // scene_open
     float bounds_lo[3] = {0, 0, 0}, bounds_hi[3] = {0, 0, 0};
     GuideState guide;
 };
@@ -307,6 +308,25 @@ xt_status xt_scene_destroy(xt_scene* s) {
     if (s->stream) hipStreamDestroy(s->stream);
     delete s;
     return XT_OK;
+}
+
+// Whether most rays that leave a surface of the scene leave it for the sky: a
+// random line that crosses the bounds meets, on average, 2 A / A_bounds surfaces
+// (Cauchy-Crofton; A the triangles' area, A_bounds the box's).  A ground has some
+// 0.9 (its paths 1.8 vertices), one as high as wide 1.4 (2.9), a closed room more
+// than 2 (11, to depth 16).  walk_max has what it decides, at 0.95 and at 1.3 by as
+// much either way; at 1.1 neither side gains up to 460 k paths.
+static bool scene_open(const std::vector<BuildTri>& bt, bool has_sky, const float lo[3], const float hi[3]) {
+    if (!has_sky || bt.empty()) return false;
+    double area2 = 0.0;
+    for (const BuildTri& t : bt) {
+        const float ux = t.p[1][0] - t.p[0][0], uy = t.p[1][1] - t.p[0][1], uz = t.p[1][2] - t.p[0][2];
+        const float vx = t.p[2][0] - t.p[0][0], vy = t.p[2][1] - t.p[0][1], vz = t.p[2][2] - t.p[0][2];
+        const float cx = uy * vz - uz * vy, cy = uz * vx - ux * vz, cz = ux * vy - uy * vx;
+        area2 += std::sqrt(cx * cx + cy * cy + cz * cz);
+    }
+    const double x = hi[0] - lo[0], y = hi[1] - lo[1], z = hi[2] - lo[2];
+    return area2 < 1.05 * 2.0 * (x * y + y * z + z * x);
 }
 
 // Lat-long importance distribution of an image sky: texel weight = the
@@ -719,6 +739,7 @@ xt_status xt_scene_create(xt_device* dev, const xt_scene_desc* desc, xt_scene** 
                 s->bounds_lo[a] = std::min(s->bounds_lo[a], t.p[k][a]);
                 s->bounds_hi[a] = std::max(s->bounds_hi[a], t.p[k][a]);
             }
+    s->open = scene_open(bt, e.has_sky != 0, s->bounds_lo, s->bounds_hi);
     {
         hipError_t r = dalloc(&s->d_ds, 1);
         if (r == hipSuccess) r = hipMemcpy(s->d_ds, &ds, sizeof(DevScene), hipMemcpyHostToDevice);
@@ -756,10 +777,12 @@ static uint32_t shade_blocks_for(uint64_t n, uint32_t grid, uint32_t block) {
 }
 
 // Most paths that k_walk follows from their camera rays.
-static uint32_t walk_max(const xt_scene* s, int max_depth) {
-    return s->ds.env.has_sky || max_depth <= 0 ? WALK_MAX_SHORT_ROUNDS : WALK_MAX;
+static uint32_t walk_max(bool open, bool nmap, int max_depth) {
+    const uint32_t in_open = nmap ? WALK_MAX_OPEN_NMAP : WALK_MAX_OPEN;
+    const uint32_t uncapped = nmap ? WALK_MAX_UNCAPPED_NMAP : WALK_MAX_UNCAPPED;
+    return open ? in_open : max_depth <= 0 ? uncapped : WALK_MAX;
 }
-
+static uint32_t walk_max(const xt_scene* s, int max_depth) { return walk_max(s->open, s->nmap, max_depth); }
 
 // Paths a wave of k_walk follows at a time, of n in all.
 static uint32_t walk_lanes(uint64_t n) {
@@ -2007,8 +2030,8 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
     std::vector<DevScene>& ds = run.ds;
     uint64_t total = 0;
     int max_depth = 1;
-    bool nmap = false, open = false;   // some scene has normal maps, a sky
-    uint32_t wmax = WALK_MAX_SHORT_ROUNDS;   // paths up to which the window is walked
+    bool nmap = false, sky = false;    // some scene has normal maps, a sky
+    bool open = true;                  // every scene is open
     uint32_t ovf_depth = 0;
     for (uint32_t i : which) {
         const xt_batch_item& it = items[i];
@@ -2020,8 +2043,8 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
             sc_list.push_back(s);
             ds.push_back(s->ds);
             nmap |= s->nmap;
-            open |= s->ds.env.has_sky != 0;
-            wmax = std::min(wmax, walk_max(s, it.params.max_depth));
+            sky |= s->ds.env.has_sky != 0;
+            open &= s->open;
             ovf_depth = std::max(ovf_depth, s->ovf_depth);
         }
         MultiItem e{};
@@ -2060,7 +2083,7 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
         m.capacity = window;
     }
     xt_scene* s0 = sc_list[0];
-    const bool whole = window <= wmax;   // each path in one launch
+    const bool whole = window <= walk_max(open, nmap, max_depth);   // each path in one launch
     const uint32_t lanes = walk_lanes(window);
     const uint32_t tblocks = whole ? walk_blocks(s0, window, lanes, nmap, s0->trace_grid_max) : trace_blocks(s0, window);
     const uint32_t jblocks = trace_blocks(s0, 2 * (size_t)window);   // launches of two queues
@@ -2135,7 +2158,7 @@ static xt_status render_unified(xt_batch_item* items, const std::vector<uint32_t
             hipLaunchKernelGGL((dyn ? k_trace_shadow<true, true> : k_trace_shadow<true, false>), dim3(jblocks), dim3(TRACE_BLOCK),
                                0, m.stream, s0->ds, m.q[cur].o, m.q[cur].d, m.hits, m.sq, m.counts, cur, m.radiance, m.pending,
                                m.ovf, m.dyn, nullptr, m.item_of, m.items);
-        auto shade = open && it > 0 ? (nmap ? k_shade_multi_open<true> : k_shade_multi_open<false>)
+        auto shade = sky && it > 0 ? (nmap ? k_shade_multi_open<true> : k_shade_multi_open<false>)
                                     : (nmap ? k_shade_multi<true> : k_shade_multi<false>);
         hipLaunchKernelGGL(shade, dim3(sblocks), dim3(sblock), 0, m.stream, mb, m.q[cur], path_count(m.counts, cur), m.hits,
                            m.q[1 - cur], pair_count(m.counts, 1 - cur), m.sq, m.radiance, m.pending);
