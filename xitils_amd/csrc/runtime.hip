@@ -1572,7 +1572,7 @@ xt_status xt_render(xt_scene* s, const xt_camera* cam, const xt_render_params* p
                 if (launch && can_walk && bound <= WALK_TAIL && result == XT_OK) {
                     // few paths are left: the queue of the next round, whose
                     // length is at most `bound`, in one launch
-                    if (joint) shadow_round(round - 1, cur);
+                    shadow_round(round - 1, cur);
                     walk(cur, bound);
                     while (verified < round)
                         if (!read_round()) break;
