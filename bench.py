@@ -136,8 +136,7 @@ def kernel_roofline(kernel, algo_bytes_per_launch, avg_launch_ms, pmc, extra=Non
     cross HBM (rocprof PMC) and the VALU issue rate (SQ_INSTS_VALU) are
     reported beside it, and `bound` names what limits the kernel: "hbm" or
     "valu-issue" when that measured rate is at 70% of its peak or more, else
-    "latency" (neither unit saturated: the kernel waits on its dependent
-    loads and tests)."""
+    "latency" (neither unit saturated over the launches taken together)."""
     sec = avg_launch_ms * 1e-3
     achieved = algo_bytes_per_launch / sec / 1e9
     r = {
@@ -165,7 +164,7 @@ def kernel_roofline(kernel, algo_bytes_per_launch, avg_launch_ms, pmc, extra=Non
             r["bound"] = "latency"
         r["note"] = ("frac counts the kernel's algorithmic bytes at full size; most of them hit in L2/MALL, so the "
                      "bytes crossing HBM (hbm_measured_frac) are fewer; with VALU issue (valu_issue_frac) below "
-                     "its peak too, the kernel is bound by the latency of its dependent fetches and tests"
+                     "its peak too, no unit is saturated over the launches taken together"
                      if r["bound"] == "latency" else
                      "frac counts the kernel's algorithmic bytes at full size; the measured rates name the bound")
     if extra:
@@ -941,7 +940,9 @@ def main():
     roofline = kernel_roofline(
         "k_trace + k_trace_shadow (extension and shadow rays)", bytes_trav / launches,
         (agg["ms_extend"] + agg["ms_shadow"]) / agg["extend_launches"], pmc,
-        {"per_ray": {"node_fetches": round((cst["ext_node_fetches"] + cst["shadow_node_fetches"]) / n_rays, 3),
+        {"launches": "camera rays at the rate of independent FMAs, bounced and shadow rays at 5.8 TB/s on the memory "
+                     "side (profiles/traverse_heightfield1080p_pmc.txt)",
+         "per_ray": {"node_fetches": round((cst["ext_node_fetches"] + cst["shadow_node_fetches"]) / n_rays, 3),
                      "tri_fetches": round((cst["ext_tri_fetches"] + cst["shadow_tri_fetches"]) / n_rays, 3),
                      "bytes": round(bytes_trav / n_rays, 1)}})
     out = {

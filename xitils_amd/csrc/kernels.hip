@@ -1,13 +1,15 @@
 // gfx950 kernels: ray queries and the wavefront path tracer.
 //
 // Wavefront pipeline per batch of paths (one path = one pixel sample):
-//   generate -> [extend -> shade -> shadow]* -> accumulate
+//   extend (camera rays) -> shade -> [extend + shadow -> shade]* -> accumulate
+// (guided and counting renders begin with generate; a batch of few paths, or
+// a large one's last, is one launch: k_walk)
 // extend  : closest hit for every queued ray         (Scene::intersect, Scene.h:30)
 // shade   : one StandardPathTracer / NaivePathTracer loop step
 //           (PathTracer.h:147-246 / 65-101): emission at the new vertex,
 //           roulette, BSDF sample -> next queue, light sample -> shadow queue
 // shadow  : any hit for every shadow ray             (Scene::intersectAny, Scene.h:34)
-// Queues are compacted with one atomic per 512-thread block for both (wave
+// Queues are compacted with one atomic per block for both (wave
 // ballots + an LDS prefix); per-wave atomics on the two queue counters were
 // the shade kernel's bottleneck.
 // Radiance is kept per path id and summed in the reference's order (BSDF-hit

@@ -400,7 +400,11 @@ __global__ __launch_bounds__(64 * W) void k_vmf_fit_block(const float* __restric
 // waves, and fewer sets than a wave each would fill the chip with.  6 lobes,
 // a wave against a block per set: 1024 sets of 256 samples 4.6 / 2.1 ms, 400
 // of 256 3.3 / 1.4 ms, 1024 of 3000 19.2 / 6.1 ms, 1 of 3000 1.7 / 0.46 ms;
-// 1 lobe, 96 of 3000 (2 steps) 0.26 / 0.25 ms.
+// 1 lobe, 96 of 3000 (2 steps) 0.26 / 0.25 ms.  The line lies on the safe side of
+// where the forms cross, not there: with 6 and 12 lobes the block is still the
+// faster one at 2048 sets of 256 (8.5 / 5.8, 43 / 14 ms) and of 64 (5.1 / 3.2, 5.2 /
+// 4.5), the wave at 8192 sets of 64 (8.3 / 9.8, 13.4 / 14.7); with one lobe they
+// differ by 10% from 64 sets on, the wave ahead.
 constexpr int FIT_BLOCK_WAVES = 16;
 bool fit_in_blocks(uint32_t nfits, uint32_t num_samples) {
     return nfits <= 1024 && num_samples / nfits >= 256;
