@@ -314,8 +314,11 @@ xt_status xt_scene_destroy(xt_scene* s) {
 // random line that crosses the bounds meets, on average, 2 A / A_bounds surfaces
 // (Cauchy-Crofton; A the triangles' area, A_bounds the box's).  A ground has some
 // 0.9 (its paths 1.8 vertices), one as high as wide 1.4 (2.9), a closed room more
-// than 2 (11, to depth 16).  walk_max has what it decides, at 0.95 and at 1.3 by as
-// much either way; at 1.1 neither side gains up to 460 k paths.
+// than 2 (11, to depth 16).  walk_max has what it decides: fields of 0.95 are up to
+// 33% faster walked, of 1.3 up to 20% queued, and at 1.1 neither gains up to 460 k
+// paths.  It cannot see which side of a surface the camera is on: a lone box seen
+// from outside (1.3) is taken for closed (328 k to 655 k paths 136-201 us walked,
+// 214-251 queued), an empty room askew in its bounds for open.
 static bool scene_open(const std::vector<BuildTri>& bt, bool has_sky, const float lo[3], const float hi[3]) {
     if (!has_sky || bt.empty()) return false;
     double area2 = 0.0;
