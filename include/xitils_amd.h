@@ -287,9 +287,10 @@ xt_status xt_render_batch(xt_batch_item* items, uint32_t n);
  * hipMalloc): xt_render into a device film (film_device) with every buffer --
  * the paths' radiance, the cursors, the traversal spill stack -- carved from one
  * static device array of XT_STATIC_SCRATCH_BYTES per GPU, which the GPU holds
- * until the process ends.  Calls no hipMalloc, hipFree or allocating library routine.  Renders
- * in batches of as many paths as the array holds (3 to 4 million), so any
- * image size works; unguided only, with a bounce cap (1 <= max_depth <= 1024).
+ * until the process ends.  Calls no hipMalloc, hipFree or allocating library
+ * routine.  Renders in batches of as many paths as the array holds (3 to 4
+ * million), so any image size works; unguided only, with a bounce cap
+ * (1 <= max_depth <= 1024).
  * Gives xt_render's film bit for bit.  XT_ERR_TOO_LARGE if the scene's
  * traversal stack does not fit the array's spill part (16 MiB).  Every call
  * on one GPU uses that GPU's one array: calls that overlap on one GPU race. */
